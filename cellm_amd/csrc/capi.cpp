@@ -221,6 +221,40 @@ int32_t get_workspace(cellm_hip_ctx* ctx, hipStream_t st, size_t need, float** o
     return get_stream_buffer(ctx, ctx->workspaces, st, need, out);
 }
 
+// A stream under graph capture.  Calls whose scratch is only a matter of speed take the form without it
+// there: a workspace cannot grow during a capture, and one that grows later would leave the graph with
+// the address of the freed one.
+bool capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
+// The multi-row GEMM over f32 x (qgemm_exact.hip) where it applies: *done tells whether it was enqueued.
+// It needs scratch for x's parts, which the one-wave-per-row kernels do without, so a call that cannot
+// have it (captures, no memory) is left to them.
+int32_t try_qgemm_exact(cellm_hip_ctx* ctx, int fmt, const XgSeg* segs, int nseg, int32_t sdt, const void* x,
+                        int64_t m, int64_t k, hipStream_t st, bool* done)
+{
+    *done = false;
+    if (!qgemm_exact_supported(fmt, segs, nseg, (int)m, (int)k, x) || capturing(st)) return CELLM_HIP_OK;
+    float* ws = nullptr;
+    const int32_t rc = get_workspace(ctx, st, qgemm_exact_workspace_bytes(segs, nseg, (int)m, (int)k), &ws);
+    if (rc == CELLM_HIP_ERR_OUT_OF_MEMORY) {
+        (void)hipGetLastError();
+        return CELLM_HIP_OK;
+    }
+    if (rc) return rc;
+    HIP_TRY(launch_qgemm_exact(fmt, segs, nseg, sdt, static_cast<const float*>(x), (int)m, (int)k, ws, st),
+            "qgemm_exact launch");
+    *done = true;
+    return CELLM_HIP_OK;
+}
+
 int32_t qgemv_i8_impl(cellm_hip_ctx* ctx, const int8_t* w, const void* scales, int32_t sdt, int64_t n_scales,
                       const void* x, int32_t xdt, const float* bias, float* y, int64_t m, int64_t n, int64_t k,
                       hipStream_t st, bool force_gemm)
@@ -263,6 +297,12 @@ int32_t qgemv_i8_impl(cellm_hip_ctx* ctx, const int8_t* w, const void* scales, i
                                           (int)n, (int)k, st),
                 "qgemv_i8_f32x_mfma launch");
         return CELLM_HIP_OK;
+    }
+    if (xdt == DT_F32) {
+        const XgSeg seg{w, scales, bias, y, (int)n, per_channel};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, XG_I8, &seg, 1, sdt, x, m, k, st, &done)) return rc;
+        if (done) return CELLM_HIP_OK;
     }
     HIP_TRY(launch_qgemv_i8(w, scales, sdt, per_channel, x, xdt, bias, y, (int)m, (int)n, (int)k, st, k == 0),
             "qgemv_i8 launch");

@@ -85,6 +85,22 @@ hipError_t launch_qgemm_q4_affine_ws(const uint32_t* wq, const void* S, const vo
 hipError_t launch_qgemm_i8_ws(const int8_t* w, const void* S, int sdt, int per_channel, const _Float16* x,
                               const float* bias, float* y, int M, int N, int K, float* workspace, hipStream_t st);
 
+// Multi-row GEMM over f32 x, weights exact in f16 (qgemm_exact.hip): M >= 5 (and rows enough to pay
+// for its launches), K % 16 == 0, 16-byte aligned W and x.  Up to three matrices share x.  `ws` holds x's f16 parts and the split sums.
+enum { XG_I8 = 0 };
+struct XgSeg {
+    const void* w;
+    const void* s;
+    const float* bias;
+    float* y;
+    int n;
+    int per_channel;
+};
+bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int M, int K, const void* x);
+size_t qgemm_exact_workspace_bytes(const XgSeg* segs, int nseg, int M, int K);
+hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, const float* x, int M, int K, void* ws,
+                              hipStream_t st);
+
 // Batched decode on MFMA (2 <= M <= 64, f16 x): int8 needs K % 64 == 0 and
 // K >= 128, q4 K % 128 == 0, K >= 256 and group >= 32; 16-byte aligned W and x;
 // ceil16(M) * N * 4 < 2^31.

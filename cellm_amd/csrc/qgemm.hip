@@ -28,6 +28,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "lds_dma.hpp"
 
 namespace cellm {
 
@@ -264,46 +265,15 @@ __global__ void add_bias_kernel(float* __restrict__ y, const float* __restrict__
 // Direct-to-LDS helpers for the q4 qGEMM below (K % 128 == 0): LDS tiles hold
 // rows of 16 chunks of 8 halves, chunk position XOR-swizzled by (row & 15) so
 // that the 16 rows a fragment read touches fall in 16 distinct 4-bank groups.
-// The DMA loads are issued from inline asm with the LDS base in M0 and are
-// waited for with explicit s_waitcnt counts: the compiler treats LDS DMA as
-// aliasing every LDS read and would otherwise wait for all of them (including
-// the stage just issued) before each fragment read.
 // ---------------------------------------------------------------------------
 namespace dma {
 
+using namespace ldsdma;
+
 constexpr int BK = 128;
 constexpr int kStageHalves = BM * BK;       // one f16 X or W tile
-constexpr size_t kMaxLds = 160 * 1024;
 
 __device__ __forceinline__ int slot(int r, int c) { return r * 16 + (c ^ (r & 15)); }
-
-__device__ __forceinline__ uint32_t lds_addr(const void* p)
-{
-    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
-}
-
-// 16 bytes per lane, global -> LDS; lane i lands at lds + 16 i (checked on gfx950)
-__device__ __forceinline__ void dma16(const void* g, uint32_t lds)
-{
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(__builtin_amdgcn_readfirstlane(lds))
-                 : "memory", "m0");
-}
-
-// Same with a uniform 64-bit base in SGPRs and a per-lane 32-bit byte offset: a loop that only changes
-// the base never rewrites the VGPR operand (the compiler's wait pass treats an asm's VGPR operands as
-// pending after it, and rewriting them cost a vmcnt(0) drain per iteration).
-__device__ __forceinline__ void dma16_s(uint32_t voff, const void* sbase, uint32_t lds)
-{
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase),
-                 "s"(__builtin_amdgcn_readfirstlane(lds))
-                 : "memory", "m0");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt()
-{
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 // ---------------------------------------------------------------------------
 // q4 affine qGEMM, dequant at the MFMA (K % 128 == 0).

@@ -1,0 +1,520 @@
+// Multi-row GEMM on f16 MFMA whose weights are exact in f16 (gfx950):
+//
+//   Y[m,n] = (sum_k w[n,k] x[m,k]) * scale[n] (+ bias[n]),   w exact in f16
+//
+// for M >= 5 rows of f32 activations over int8 weights
+// (cpu_kernels::matmul_i8_f32, crates/cellm-kernels/src/cpu_kernels.rs:66-133,
+// run once per prompt token by the reference, crates/cellm-model/src/llama.rs:214-233).
+//
+// f32 activations keep their 24 bits: a first kernel scales each row by the
+// power of two that puts its largest |x| in [2^13, 2^14) and splits it into
+// hi = RNE_f16(x') and lo = RNE_f16(x' - hi); x' - hi - lo is below 2^-23 |x'|
+// (and 2^-25 absolute, 2^-38 of the row's largest).  Both parts are rows of the
+// GEMM's A operand over one weight tile, so every weight is fetched and unpacked
+// once for the two.  Products of f16 values are exact in f32.  The MFMA chain
+// rounds its f32 accumulator once per 8 or 16 products, so a chain over the whole
+// K carries more rounding error than the tree sums of the one-wave-per-row
+// kernels: accumulators run over one K step (64 k), low parts before high ones,
+// and are then added to a second set.  Error against 64 bits at 512 rows, K = 960
+// / 2560 / 4096: 8.6e-8 / 1.0e-7 / 1.3e-7 with a sum per step, 9.7e-8 / 1.1e-7 /
+// 1.2e-7 per two steps, 1.3e-7 / 1.4e-7 / 1.4e-7 per four, 9.7e-8 / 1.3e-7 /
+// 1.7e-7 in the one-wave-per-row kernels; a sum per step costs 1-4 % in time.
+// Results that are not finite (an infinity or NaN in x or w, or an overflow: the
+// split turns inf into inf * lo) are recomputed by a plain f32 sum.
+//
+// Measured, int8 at 512 rows (us, one-wave-per-row kernel -> this one with its
+// split of x): 960 -> 960 1963 -> 20, 2560 -> 960 5098 -> 25, 4096 -> 4096
+// 8034 -> 60; 16 rows of 1152 -> 1536 35 -> 15; 2048 rows of 2048 -> 8192 164,
+// 839 TFLOP/s of MFMA work.  The small ones are bound by three dependent launches
+// and the latency of a few K steps, the wide ones by the MFMAs.
+//
+// Tile: WM x WN waves of (32 TA) x (32 TB); X parts and raw weights go
+// global -> LDS by DMA through a ring of NST stages of 64 k, one barrier per
+// step.  Weights stay raw in LDS and are unpacked right before their MFMAs by
+// the lane that multiplies them.  A lane (r32 = lane % 32, h32 = lane / 32)
+// supplies k = 32 h32 + 8 ks + 0..7 of the step to substep ks = 0..3: the MFMA's
+// k order is free as long as X and W agree, and this one makes a lane's weights
+// of a step contiguous.  LDS rows are XOR-swizzled in 16-byte chunks so that the
+// eight rows of a read phase fall in different banks.
+#include <algorithm>
+
+#include "common.hpp"
+#include "kernels.hpp"
+#include "launch_util.hpp"
+#include "lds_dma.hpp"
+
+namespace cellm {
+
+namespace {
+
+using namespace ldsdma;
+
+constexpr int kBK = 64;
+
+struct XgArgs {
+    XgSeg seg[3];
+    int tile0[3];  // first column tile of each segment
+    int nseg;
+    const _Float16* xp;   // [M][P][Kp] activation parts
+    const int32_t* xe;    // [M] row exponents e (x' = x 2^e); P == 2
+    const void* x;        // the caller's activations [M][K], for the recomputed sums
+    float* part;          // [splits][M][vcols] raw sums, or nullptr (unsplit)
+    int M, K, Kp;
+    int steps_per_split;
+    int vcols;            // column tiles * BN
+    int sdt;
+};
+
+template <int FMT>
+struct Fmt;
+template <>
+struct Fmt<XG_I8> {
+    static constexpr int kStepBytes = 64;  // of a weight row per K step
+};
+
+template <int FMT>
+__device__ __forceinline__ size_t row_bytes(int K)
+{
+    return (size_t)K * Fmt<FMT>::kStepBytes / kBK;
+}
+
+// eight consecutive int8 weights as f16, in order: bytes biased to u8 land under 0x64 (1024 + u8), minus 1152
+__device__ __forceinline__ h8_t i8x8(uint32_t w0, uint32_t w1)
+{
+    const uint32_t b0 = w0 ^ 0x80808080u, b1 = w1 ^ 0x80808080u, hi = 0x64646464u;
+    const h2_t off = {(_Float16)1152.0f, (_Float16)1152.0f};
+    const h2_t a0 = as_h2(__builtin_amdgcn_perm(hi, b0, 0x04010400u)) - off;
+    const h2_t a1 = as_h2(__builtin_amdgcn_perm(hi, b0, 0x04030402u)) - off;
+    const h2_t a2 = as_h2(__builtin_amdgcn_perm(hi, b1, 0x04010400u)) - off;
+    const h2_t a3 = as_h2(__builtin_amdgcn_perm(hi, b1, 0x04030402u)) - off;
+    return h8_t{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+}
+
+// LDS position of 16-byte chunk c of row r: rows of RB bytes, the eight rows of a read phase in
+// different banks
+template <int RB>
+__device__ __forceinline__ int swz(int r, int c)
+{
+    if constexpr (RB == 128) return c ^ (r & 7);
+    else if constexpr (RB == 64) return c ^ ((r >> 2) & 3);
+    else return c;
+}
+
+__device__ __forceinline__ float scale_at(const void* s, int sdt, size_t i)
+{
+    return sdt == DT_F32 ? load_f32<DT_F32>(s, i) : sdt == DT_F16 ? load_f32<DT_F16>(s, i) : load_f32<DT_BF16>(s, i);
+}
+
+// sum_k w[n,k] x[m,k] by a plain f32 loop: the results that MFMA left non-finite
+template <int FMT, int P>
+__device__ __forceinline__ float plain_dot(const XgSeg& g, const void* x, int m, int n, int K)
+{
+    float acc = 0.0f;
+    for (int k = 0; k < K; ++k) {
+        float xv;
+        if constexpr (P == 2) xv = static_cast<const float*>(x)[(size_t)m * K + k];
+        else xv = (float)static_cast<const _Float16*>(x)[(size_t)m * K + k];
+        if constexpr (FMT == XG_I8) acc += (float)static_cast<const int8_t*>(g.w)[(size_t)n * K + k] * xv;
+    }
+    return acc;
+}
+
+__device__ __forceinline__ bool finite_f32(float v) { return (__builtin_bit_cast(uint32_t, v) & 0x7F800000u) != 0x7F800000u; }
+
+__device__ __forceinline__ float column_scale(const XgSeg& g, int sdt, int n)
+{
+    return scale_at(g.s, sdt, g.per_channel ? (size_t)n : 0);
+}
+
+template <int FMT, int P, int TA, int TB, int WM, int WN, int NST>
+__global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgArgs a)
+{
+    constexpr int NW = WM * WN, BM = 32 * TA * WM, BN = 32 * TB * WN, RB = Fmt<FMT>::kStepBytes;
+    constexpr int kXBytes = BM * P * 128, kWBytes = BN * RB, kStage = kXBytes + kWBytes;
+    constexpr int XD = kXBytes / 1024 / NW, WD = kWBytes / 1024 / NW;  // DMA loads per wave and step
+    constexpr int NDMA = XD + WD, LA = NST - 1;
+    static_assert(XD * NW * 1024 == kXBytes && WD * NW * 1024 == kWBytes, "whole DMA loads per wave");
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave / WN, wn = wave % WN, r32 = lane & 31, h32 = lane >> 5;
+    const int vt = blockIdx.x, m0 = blockIdx.y * BM;
+    const int step0 = blockIdx.z * a.steps_per_split, total = a.Kp / kBK;
+    const int nsteps = min(a.steps_per_split, total - step0);
+    if (nsteps <= 0) return;  // the launcher makes no empty split
+    const int si = (a.nseg > 1 && vt >= a.tile0[1]) + (a.nseg > 2 && vt >= a.tile0[2]);
+    const XgSeg g = a.seg[si];
+    const int n0 = (vt - a.tile0[si]) * BN;
+    const size_t rbytes = row_bytes<FMT>(a.K);
+
+    // X DMA: load j of a wave covers 8 part rows (128 bytes each); part row p BM + i is part p of row
+    // m0 + i, rows past M re-read the last one (computed, never stored)
+    uint32_t xoff[XD];
+#pragma unroll
+    for (int j = 0; j < XD; ++j) {
+        const int pr = (wave * XD + j) * 8 + (lane >> 3);
+        const int p = pr / BM, i = min(pr % BM, a.M - 1 - m0);
+        xoff[j] = (uint32_t)(i * P + p) * (uint32_t)(a.Kp * 2) + 16 * ((lane & 7) ^ (pr & 7));
+    }
+    // W DMA: load j covers 1024 / RB rows.  In the last step of a K that is no multiple of 64, chunks
+    // past the row's end re-read its last one (they meet the zeros that pad X)
+    constexpr int RPD = 1024 / RB, CPR = RB / 16;
+    uint32_t woff[WD], woff_tail[WD];
+    const int tail_chunks = (int)(rbytes - (size_t)(total - 1) * RB) / 16;
+#pragma unroll
+    for (int j = 0; j < WD; ++j) {
+        const int r = (wave * WD + j) * RPD + lane / CPR;
+        const int c = swz<RB>(r, lane % CPR);
+        const uint32_t row = (uint32_t)min(r, g.n - 1 - n0) * (uint32_t)rbytes;
+        woff[j] = row + 16 * c;
+        woff_tail[j] = row + 16 * min(c, tail_chunks - 1);
+    }
+    const unsigned char* xbase = reinterpret_cast<const unsigned char*>(a.xp) + (size_t)m0 * P * a.Kp * 2;
+    const unsigned char* wbase = static_cast<const unsigned char*>(g.w) + (size_t)n0 * rbytes;
+    const uint32_t lds0 = lds_addr(smem);
+    const bool ragged = tail_chunks < CPR;
+    auto issue = [&](int s, int slot) {
+        const int t = step0 + min(s, nsteps - 1);
+        const uint32_t base = lds0 + slot * kStage;
+        const unsigned char* xs = xbase + (size_t)t * 128;
+        const unsigned char* ws = wbase + (size_t)t * RB;
+#pragma unroll
+        for (int j = 0; j < XD; ++j) dma16_s(xoff[j], xs, base + (wave * XD + j) * 1024);
+        if (ragged && t == total - 1) {
+#pragma unroll
+            for (int j = 0; j < WD; ++j) dma16_s(woff_tail[j], ws, base + kXBytes + (wave * WD + j) * 1024);
+        } else {
+#pragma unroll
+            for (int j = 0; j < WD; ++j) dma16_s(woff[j], ws, base + kXBytes + (wave * WD + j) * 1024);
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < LA; ++j) issue(j, j);
+
+    f16v_t acc[TA][TB], sum[TA][TB];
+#pragma unroll
+    for (int i = 0; i < TA; ++i)
+#pragma unroll
+        for (int j = 0; j < TB; ++j) sum[i][j] = f16v_t{};
+
+    int slot = 0;
+    auto step = [&](int s) {
+        // stage s landed in this wave's share of the slot; only the LA - 1 stages after it may be in
+        // flight.  A bare s_barrier: __syncthreads()'s release fence waits for every DMA in flight.
+        wait_vmcnt<(LA - 1) * NDMA>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();  // stage s complete everywhere; stage s - 1 no longer read
+        issue(s + LA, slot == 0 ? NST - 1 : slot - 1);  // into the slot of stage s - 1
+        const unsigned char* xs = smem + slot * kStage;
+        const unsigned char* ws = xs + kXBytes;
+        slot = slot + 1 == NST ? 0 : slot + 1;
+        h8_t b[TB][4];
+#pragma unroll
+        for (int j = 0; j < TB; ++j) {
+            const int r = (wn * TB + j) * 32 + r32;
+            if constexpr (FMT == XG_I8) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const u4_t w = *reinterpret_cast<const u4_t*>(ws + r * RB + 16 * swz<RB>(r, 2 * h32 + c));
+                    b[j][2 * c] = i8x8(w[0], w[1]);
+                    b[j][2 * c + 1] = i8x8(w[2], w[3]);
+                }
+            }
+        }
+#pragma unroll
+        for (int p = P - 1; p >= 0; --p)  // low parts first
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                h8_t x[TA];
+#pragma unroll
+                for (int i = 0; i < TA; ++i) {
+                    const int r = p * BM + (wm * TA + i) * 32 + r32;
+                    x[i] = *reinterpret_cast<const h8_t*>(xs + r * 128 + 16 * swz<128>(r, 4 * h32 + ks));
+                }
+#pragma unroll
+                for (int i = 0; i < TA; ++i)
+#pragma unroll
+                    for (int j = 0; j < TB; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i], b[j][ks], acc[i][j], 0, 0, 0);
+            }
+    };
+    for (int s = 0; s < nsteps; ++s) {
+#pragma unroll
+        for (int i = 0; i < TA; ++i)
+#pragma unroll
+            for (int j = 0; j < TB; ++j) acc[i][j] = f16v_t{};
+        step(s);
+#pragma unroll
+        for (int i = 0; i < TA; ++i)
+#pragma unroll
+            for (int j = 0; j < TB; ++j) sum[i][j] += acc[i][j];
+    }
+    wait_vmcnt<0>();  // the trailing (re-read) DMA, before the block's LDS is given back
+
+    // register r of a 32x32 tile: row (r / 4) * 8 + h32 * 4 + r % 4, column r32
+    if (a.part) {
+#pragma unroll
+        for (int i = 0; i < TA; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3);
+                float* row = a.part + ((size_t)blockIdx.z * a.M + m) * a.vcols + (size_t)vt * BN + wn * TB * 32 + r32;
+                if (m < a.M)
+#pragma unroll
+                    for (int j = 0; j < TB; ++j) row[j * 32] = sum[i][j][r];
+            }
+        return;
+    }
+    int e[TA][16];
+    if constexpr (P == 2) {
+#pragma unroll
+        for (int i = 0; i < TA; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                e[i][r] = -a.xe[min(m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3), a.M - 1)];
+    }
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < TB; ++j) {
+        const int n = n0 + (wn * TB + j) * 32 + r32;
+        if (n >= g.n) continue;
+        const float sc = column_scale(g, a.sdt, n), bi = g.bias ? g.bias[n] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < TA; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3);
+                float v = sum[i][j][r];
+                if constexpr (P == 2) v = ldexpf(v, e[i][r]);
+                v = v * sc + bi;
+                if (m < a.M) {
+                    g.y[(size_t)m * g.n + n] = v;
+                    bad |= !finite_f32(v);
+                }
+            }
+    }
+    if (!bad) return;
+    // rolled and rare: this lane's non-finite results again
+    for (int t = 0; t < TA * TB * 16; ++t) {
+        const int i = t / (16 * TB), j = (t / 16) % TB, r = t & 15;
+        const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3), n = n0 + (wn * TB + j) * 32 + r32;
+        if (m >= a.M || n >= g.n || finite_f32(g.y[(size_t)m * g.n + n])) continue;
+        g.y[(size_t)m * g.n + n] =
+            plain_dot<FMT, P>(g, a.x, m, n, a.K) * column_scale(g, a.sdt, n) + (g.bias ? g.bias[n] : 0.0f);
+    }
+}
+
+// y of a split GEMM: the splits' sums added in split order, then the epilogue above.  A thread owns four
+// neighbouring columns of one row.
+template <int FMT, int P>
+__global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a, int splits, int bn)
+{
+    const int quads = a.vcols / 4;
+    const size_t stride = (size_t)a.M * quads;
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < stride; t += (size_t)gridDim.x * 256) {
+        const int m = (int)(t / quads), vc = (int)(t - (size_t)m * quads) * 4, vt = vc / bn;
+        const int si = (a.nseg > 1 && vt >= a.tile0[1]) + (a.nseg > 2 && vt >= a.tile0[2]);
+        const XgSeg g = a.seg[si];
+        const int n = vc - a.tile0[si] * bn;
+        if (n >= g.n) continue;
+        const f4_t v = sum_splits_f4(reinterpret_cast<const f4_t*>(a.part) + t, stride, splits);
+        const int e = P == 2 ? -a.xe[m] : 0;
+        float* y = g.y + (size_t)m * g.n + n;
+        f4_t o;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int nc = min(n + c, g.n - 1);
+            const float sc = column_scale(g, a.sdt, nc), bi = g.bias ? g.bias[nc] : 0.0f;
+            o[c] = (P == 2 ? ldexpf(v[c], e) : v[c]) * sc + bi;
+            if (!finite_f32(o[c])) o[c] = plain_dot<FMT, P>(g, a.x, m, nc, a.K) * sc + bi;
+        }
+        if ((g.n & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
+            *reinterpret_cast<f4_t*>(y) = o;
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (n + c < g.n) y[c] = o[c];
+        }
+    }
+}
+
+// One block per row of x: its parts, zero-padded to Kp, and its exponent.  Eight elements per thread
+// and round; rows of up to 8192 stay in registers between the maximum and the split.
+constexpr int kSplitUnits = 4;
+__global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ x, int K, int Kp,
+                                                      _Float16* __restrict__ xp, int32_t* __restrict__ xe)
+{
+    __shared__ float wmax[4];
+    const int m = blockIdx.x, tid = threadIdx.x, units = Kp / 8;
+    const float* row = x + (size_t)m * K;
+    f4_t v[kSplitUnits][2];
+    auto load = [&](int u, f4_t (&d)[2]) {
+        const bool in = u * 8 < K;  // K % 8 == 0
+        const f4_t* p = reinterpret_cast<const f4_t*>(row + (in ? u * 8 : 0));
+        d[0] = p[0];
+        d[1] = p[1];
+        if (!in) d[0] = d[1] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    auto largest = [](const f4_t (&d)[2], float mx) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float q = fabsf(d[i >> 2][i & 3]);
+            mx = finite_f32(q) ? fmaxf(mx, q) : mx;
+        }
+        return mx;
+    };
+    const bool held = units <= kSplitUnits * 256;
+    float mx = 0.0f;
+    if (held) {
+#pragma unroll
+        for (int j = 0; j < kSplitUnits; ++j) load(min(tid + j * 256, units - 1), v[j]);
+#pragma unroll
+        for (int j = 0; j < kSplitUnits; ++j) mx = largest(v[j], mx);
+    } else {
+        for (int u = tid; u < units; u += 256) {
+            load(u, v[0]);
+            mx = largest(v[0], mx);
+        }
+    }
+    mx = group_max<64>(mx);
+    if ((tid & 63) == 0) wmax[tid >> 6] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    const int top = (int)(__builtin_bit_cast(uint32_t, mx) >> 23);  // biased exponent; 0: zero or subnormal
+    const int e = mx > 0.0f ? 13 - (max(top, 1) - 127) : 0;
+    if (tid == 0) xe[m] = e;
+    _Float16* out = xp + (size_t)m * 2 * Kp;
+    auto store = [&](int u, const f4_t (&d)[2]) {
+        h8_t hi, lo;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float s = ldexpf(d[i >> 2][i & 3], e);
+            hi[i] = (_Float16)s;
+            lo[i] = finite_f32(s) ? (_Float16)(s - (float)hi[i]) : (_Float16)0.0f;
+        }
+        *reinterpret_cast<h8_t*>(out + u * 8) = hi;
+        *reinterpret_cast<h8_t*>(out + Kp + u * 8) = lo;
+    };
+    if (held) {
+#pragma unroll
+        for (int j = 0; j < kSplitUnits; ++j)
+            if (tid + j * 256 < units) store(tid + j * 256, v[j]);
+    } else {
+        for (int u = tid; u < units; u += 256) {
+            load(u, v[0]);
+            store(u, v[0]);
+        }
+    }
+}
+
+// The tile forms: 0 = 32 rows x 128 columns (2 waves), 1 = 64 x 128 (4 waves), 2 = 128 x 256 (8 waves).
+struct XgPlan {
+    int form, bm, bn, vtiles, steps_per_split, splits;
+    size_t part_off, bytes;  // workspace: exponents, parts, then the split sums
+};
+
+XgPlan xg_plan(const int* n, int nseg, int M, int K)
+{
+    XgPlan p{};
+    const int steps = (K + kBK - 1) / kBK;
+    auto tiles = [&](int bm, int bn) {
+        int t = 0;
+        for (int i = 0; i < nseg; ++i) t += (n[i] + bn - 1) / bn;
+        p.bm = bm, p.bn = bn, p.vtiles = t;
+        return (int64_t)t * ((M + bm - 1) / bm);
+    };
+    int64_t blocks = tiles(128, 256);
+    p.form = 2;
+    if (blocks < 192) {
+        p.form = M > 32 ? 1 : 0;
+        blocks = p.form ? tiles(64, 128) : tiles(32, 128);
+    }
+    int splits = 1;
+    const int64_t want = p.form == 2 ? 256 : 512;
+    while (blocks * splits * 2 <= want && steps / (splits * 2) >= 4) splits *= 2;
+    p.steps_per_split = (steps + splits - 1) / splits;
+    p.splits = (steps + p.steps_per_split - 1) / p.steps_per_split;
+    const size_t xe = ((size_t)M * 4 + 255) & ~(size_t)255;
+    p.part_off = xe + (((size_t)M * 2 * steps * kBK * 2 + 255) & ~(size_t)255);
+    p.bytes = p.part_off + (p.splits > 1 ? (size_t)p.splits * M * p.vtiles * p.bn * 4 : 0);
+    return p;
+}
+
+template <int FMT, int P, int TA, int TB, int WM, int WN, int NST>
+hipError_t launch_form(const XgArgs& a, const XgPlan& p, hipStream_t st)
+{
+    constexpr int lds = NST * (32 * TA * WM * P * 128 + 32 * TB * WN * Fmt<FMT>::kStepBytes);
+    auto kern = qgemm_exact_kernel<FMT, P, TA, TB, WM, WN, NST>;
+    if constexpr (lds > 64 * 1024) {
+        const hipError_t e = allow_big_lds(kern, lds);
+        if (e != hipSuccess) return e;
+    }
+    const dim3 grid(p.vtiles, (a.M + p.bm - 1) / p.bm, p.splits);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * WM * WN), lds, st, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int M, int K, const void* x)
+{
+    if (fmt != XG_I8 || M < 5 || K <= 0 || K % 16 != 0) return false;
+    // the one-wave-per-row kernels walk the rows one after the other, about 2 ns per row and element of
+    // k; the three launches here take 14-16 us (5 rows of 960 -> 960: 10.7 against 16.2 us, of 1536 ->
+    // 576: 15.2 against 14.4).  Long outputs cost them more (5 rows of 960 -> 32768: 68 against 18.5)
+    if ((int64_t)M * K < 7000 && segs[0].n < 8192) return false;
+    if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (M + 31) / 32 > 65535) return false;
+    int64_t n = 0;
+    for (int i = 0; i < nseg; ++i) {
+        if (segs[i].n <= 0 || (reinterpret_cast<uintptr_t>(segs[i].w) & 15) != 0) return false;
+        n += segs[i].n;
+    }
+    // a tile's byte offsets are 32-bit
+    return (uint64_t)K * 1024 < (1ull << 31) && n < (1 << 30);
+}
+
+size_t qgemm_exact_workspace_bytes(const XgSeg* segs, int nseg, int M, int K)
+{
+    const int n[3] = {segs[0].n, nseg > 1 ? segs[1].n : 0, nseg > 2 ? segs[2].n : 0};
+    return xg_plan(n, nseg, M, K).bytes;
+}
+
+hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, const float* x, int M, int K, void* ws,
+                              hipStream_t st)
+{
+    if (fmt != XG_I8) return hipErrorInvalidValue;
+    const int n[3] = {segs[0].n, nseg > 1 ? segs[1].n : 0, nseg > 2 ? segs[2].n : 0};
+    const XgPlan p = xg_plan(n, nseg, M, K);
+    XgArgs a{};
+    a.nseg = nseg;
+    for (int i = 0, t = 0; i < nseg; ++i) {
+        a.seg[i] = segs[i];
+        a.tile0[i] = t;
+        t += (n[i] + p.bn - 1) / p.bn;
+    }
+    unsigned char* base = static_cast<unsigned char*>(ws);
+    int32_t* xe = reinterpret_cast<int32_t*>(base);
+    _Float16* xp = reinterpret_cast<_Float16*>(base + (((size_t)M * 4 + 255) & ~(size_t)255));
+    a.xe = xe;
+    a.xp = xp;
+    a.x = x;
+    a.part = p.splits > 1 ? reinterpret_cast<float*>(base + p.part_off) : nullptr;
+    a.M = M;
+    a.K = K;
+    a.Kp = (K + kBK - 1) / kBK * kBK;
+    a.steps_per_split = p.steps_per_split;
+    a.vcols = p.vtiles * p.bn;
+    a.sdt = sdt;
+    hipLaunchKernelGGL(split_x_kernel, dim3(M), dim3(256), 0, st, x, K, a.Kp, xp, xe);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    e = p.form == 2   ? launch_form<XG_I8, 2, 2, 2, 2, 4, 3>(a, p, st)
+        : p.form == 1 ? launch_form<XG_I8, 2, 1, 2, 2, 2, 3>(a, p, st)
+                      : launch_form<XG_I8, 2, 1, 2, 1, 2, 3>(a, p, st);
+    if (e != hipSuccess || p.splits == 1) return e;
+    const size_t quads = (size_t)M * a.vcols / 4;
+    const unsigned blocks = (unsigned)std::min<size_t>((quads + 255) / 256, 4096);
+    hipLaunchKernelGGL((qgemm_exact_reduce_kernel<XG_I8, 2>), dim3(blocks), dim3(256), 0, st, a, p.splits, p.bn);
+    return hipGetLastError();
+}
+
+}  // namespace cellm

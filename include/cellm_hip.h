@@ -122,7 +122,12 @@ int32_t cellm_hip_weight_cache_stats(cellm_hip_ctx_t* ctx, size_t* out_entries, 
  * int8 MFMA: each x row becomes x' = rint(x * 2^e) with |x'| <= 2^20 for the
  * row's power of two, split into three signed 8-bit digits; the integer sums
  * over k are exact and the row scale follows them, so x keeps 2^-20 of its
- * row's largest |x| (within 3e-5 normwise of the f32 reference order). */
+ * row's largest |x| (within 3e-5 normwise of the f32 reference order).  f32 x
+ * at 5 rows and more (k % 16 == 0, 16-byte aligned w and x, m * k >= 7000 or
+ * n >= 8192) runs on f16 MFMA over two f16 parts of each x, 2^-23 of every
+ * element, with the parts and split sums in the context's per-stream workspace;
+ * under graph capture, or without memory for it, such calls take the kernels
+ * that need none. */
 int32_t cellm_hip_qgemv_i8(cellm_hip_ctx_t* ctx, const int8_t* w, const void* scales, int32_t scale_dtype,
                            int64_t n_scales, const void* x, int32_t x_dtype, const float* bias, float* y, int64_t m,
                            int64_t n, int64_t k, void* stream);

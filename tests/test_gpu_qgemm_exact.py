@@ -1,0 +1,121 @@
+"""The multi-row GEMM over f32 activations (qgemm_exact.hip) against 64-bit results.
+
+The bar: x is carried to 2^-23 of each element and every sum is f32 over chains
+of at most 16 MFMA roundings plus one add per 64 k, so the 2-norm error stays
+within a few 2^-24 (6e-8) times the square root of the number of roundings: 1e-6
+holds up to K = 8192 with a wide margin (the one-wave-per-row kernels show 1e-7
+to 2e-7 at these sizes)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-6
+
+
+def _x(m, k, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(m, k, generator=g)
+    return x * torch.where(torch.rand(k, generator=g) < 0.02, 30.0, 1.0)  # a few large channels
+
+
+def _i8(n, k, seed):
+    g = torch.Generator().manual_seed(seed)
+    w = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8)
+    return w, (torch.rand(n, generator=g) * 0.01 + 1e-3)
+
+
+def _rel(got, ref):
+    got, ref = got.double(), ref.double()
+    return float((got - ref).norm() / ref.norm())
+
+
+# edges of the 32 / 64 / 128-row and 128 / 256-column tiles, K not a multiple of 64 and of one step,
+# split and unsplit K, the forms of xg_plan (small, middle, wide)
+SIZES = [(440, 16, 16), (110, 1, 64), (5, 8200, 48), (5, 33, 1408), (31, 127, 80), (32, 128, 128), (33, 129, 960), (64, 257, 2560), (65, 384, 1056),
+         (77, 40, 4864), (200, 1000, 1024), (512, 960, 960), (513, 4100, 208), (1030, 6000, 320)]
+
+
+@pytest.mark.parametrize("m,n,k", SIZES)
+@pytest.mark.parametrize("sdt", [torch.float32, torch.float16])
+def test_i8_f32_rows(ops, m, n, k, sdt):
+    x = _x(m, k, m * 7 + k)
+    w, s = _i8(n, k, n * 3 + k)
+    s = s.to(sdt)
+    bias = torch.randn(n, generator=torch.Generator().manual_seed(n))
+    ref = x.double() @ w.double().t() * s.double() + bias.double()
+    y = torch.full((m, n), float("nan"), device="cuda")
+    ops.encode_qgemv_i8(w.cuda(), s.cuda(), x.cuda(), y, bias=bias.cuda())
+    torch.cuda.synchronize()
+    assert _rel(y.cpu(), ref) <= TOL
+
+
+def test_i8_per_tensor_scale_and_row_spread(ops):
+    """Rows whose magnitudes lie 2^80 apart (zero and subnormal rows among them) keep their own precision."""
+    m, n, k = 40, 130, 192
+    x = _x(m, k, 5)
+    x *= torch.pow(2.0, torch.linspace(-60, 20, m))[:, None].float()
+    x[3] = 0.0
+    x[4] = x[4] * 0.0 + 1e-41  # subnormal
+    w, _ = _i8(n, k, 6)
+    s = torch.tensor([0.0625])
+    y = torch.empty(m, n, device="cuda")
+    ops.encode_qgemv_i8(w.cuda(), s.cuda(), x.cuda(), y)
+    torch.cuda.synchronize()
+    ref = x.double() @ w.double().t() * 0.0625
+    got = y.cpu().double()
+    assert torch.equal(got[3], torch.zeros(n, dtype=torch.float64))
+    for r in range(m):
+        if r not in (3, 4):
+            assert _rel(got[r], ref[r]) <= TOL, r
+    assert _rel(got[4], ref[4]) <= 1e-3  # a subnormal has few bits of its own
+
+
+@pytest.mark.parametrize("k", [832, 2560])  # unsplit and split over k
+def test_i8_non_finite_activations(ops, k):
+    """inf and NaN reach exactly the outputs they reach in a plain f32 sum, and overflow is an infinity."""
+    m, n = 9, 70
+    x = _x(m, k, 8)
+    x[1, 5], x[2, 7], x[3, 0], x[3, 1] = float("inf"), float("nan"), float("inf"), float("-inf")
+    x[4] = 3e38
+    w, s = _i8(n, k, 9)
+    w[::3, 5] = 0  # inf * 0 = nan
+    y = torch.empty(m, n, device="cuda")
+    ops.encode_qgemv_i8(w.cuda(), s.cuda(), x.cuda(), y)
+    torch.cuda.synchronize()
+    ref = (x[:4] @ w.float().t()) * s
+    got = y.cpu()
+    assert np.array_equal(torch.isnan(got[:4]).numpy(), torch.isnan(ref).numpy())
+    assert np.array_equal(torch.isposinf(got[:4]).numpy(), torch.isposinf(ref).numpy())
+    assert np.array_equal(torch.isneginf(got[:4]).numpy(), torch.isneginf(ref).numpy())
+    big = torch.full((k,), 3e38).double() @ w.double().t()
+    far = (big.abs() > 2.0**129)  # overflows f32 in any order of the sum
+    assert torch.equal(torch.isfinite(got[4])[far], torch.zeros(int(far.sum()), dtype=torch.bool))
+    assert _rel(got[5:], x[5:].double() @ w.double().t() * s.double()) <= TOL
+
+
+def test_captured_calls_use_no_scratch(ops):
+    """Under capture the call takes the kernels without scratch: a replay stays right after later eager calls
+    with larger shapes have regrown the workspace."""
+    m, n, k = 32, 96, 256
+    x, (w, s) = _x(m, k, 1).cuda(), _i8(n, k, 2)
+    w, s = w.cuda(), s.cuda()
+    y = torch.zeros(m, n, device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        ops.encode_qgemv_i8(w, s, x, y, stream=torch.cuda.current_stream())
+    big = torch.empty(600, 4096, device="cuda")
+    bx, (bw, bs) = _x(600, 512, 3).cuda(), _i8(4096, 512, 4)
+    ref = x.cpu().double() @ w.cpu().double().t() * s.cpu().double()
+    for _ in range(3):
+        y.zero_()
+        ops.encode_qgemv_i8(bw.cuda(), bs.cuda(), bx, big, stream=side)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _rel(y.cpu(), ref) <= TOL
