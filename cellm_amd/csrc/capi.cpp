@@ -310,7 +310,7 @@ int32_t qgemv_i8_impl(cellm_hip_ctx* ctx, const int8_t* w, const void* scales, i
 }
 
 // f16 / i2 / q1_0_g128 row GEMVs (lowbit.hip)
-int32_t qgemv_lowbit_impl(int fmt, const void* w, const uint16_t* scales_f16, int32_t scale_mode, const void* x,
+int32_t qgemv_lowbit_impl(cellm_hip_ctx* ctx, int fmt, const void* w, const uint16_t* scales_f16, int32_t scale_mode, const void* x,
                           int32_t xdt, float* y, int64_t m, int64_t n, int64_t k, hipStream_t st)
 {
     if (int32_t rc = check_dims(m, n, k)) return rc;
@@ -327,6 +327,12 @@ int32_t qgemv_lowbit_impl(int fmt, const void* w, const uint16_t* scales_f16, in
     if (k == 0) {
         HIP_TRY(launch_fill_f32(y, 0.0f, (size_t)m * n, st), "zero fill of y");
         return CELLM_HIP_OK;
+    }
+    if (fmt == LB_F16 && xdt == DT_F32) {
+        const XgSeg seg{w, nullptr, nullptr, y, (int)n, 0};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, XG_F16, &seg, 1, DT_F32, x, m, k, st, &done)) return rc;
+        if (done) return CELLM_HIP_OK;
     }
     HIP_TRY(launch_qgemv_lowbit(fmt, w, scales_f16, scale_mode, x, xdt, y, (int)m, (int)n, (int)k, st),
             "qgemv lowbit launch");
@@ -730,7 +736,7 @@ int32_t cellm_hip_qgemv_q4_affine(cellm_hip_ctx_t* ctx, const uint32_t* wq, cons
     CELLM_API_END(report_exception)
 }
 
-static int32_t qgemv_i4_impl(const uint8_t* w, const uint16_t* scales_f16, int64_t n_scales, int64_t gs,
+static int32_t qgemv_i4_impl(cellm_hip_ctx* ctx, const uint8_t* w, const uint16_t* scales_f16, int64_t n_scales, int64_t gs,
                              const void* x, int32_t x_dtype, float* y, int64_t m, int64_t n, int64_t k, hipStream_t st);
 
 int32_t cellm_hip_qgemv_batch(cellm_hip_ctx_t* ctx, const cellm_hip_qgemv_op_t* ops, int64_t n_ops, void* stream)
@@ -751,14 +757,14 @@ int32_t cellm_hip_qgemv_batch(cellm_hip_ctx_t* ctx, const cellm_hip_qgemv_op_t* 
             rc = qgemv_q4_impl(ctx, static_cast<const uint32_t*>(o.w), o.scales, o.biases, o.sb_dtype, o.group, o.x,
                                o.x_dtype, o.y, o.m, o.n, o.k, st, false);
         else if (o.kind == CELLM_HIP_OP_QGEMV_F16)
-            rc = qgemv_lowbit_impl(LB_F16, o.w, nullptr, 0, o.x, o.x_dtype, o.y, o.m, o.n, o.k, st);
+            rc = qgemv_lowbit_impl(ctx, LB_F16, o.w, nullptr, 0, o.x, o.x_dtype, o.y, o.m, o.n, o.k, st);
         else if (o.kind == CELLM_HIP_OP_QGEMV_I2)
-            rc = qgemv_lowbit_impl(LB_I2, o.w, static_cast<const uint16_t*>(o.scales), o.group, o.x, o.x_dtype, o.y,
+            rc = qgemv_lowbit_impl(ctx, LB_I2, o.w, static_cast<const uint16_t*>(o.scales), o.group, o.x, o.x_dtype, o.y,
                                    o.m, o.n, o.k, st);
         else if (o.kind == CELLM_HIP_OP_QGEMV_Q1_0_G128)
-            rc = qgemv_lowbit_impl(LB_Q1, o.w, nullptr, 0, o.x, o.x_dtype, o.y, o.m, o.n, o.k, st);
+            rc = qgemv_lowbit_impl(ctx, LB_Q1, o.w, nullptr, 0, o.x, o.x_dtype, o.y, o.m, o.n, o.k, st);
         else if (o.kind == CELLM_HIP_OP_QGEMV_I4_SYM)
-            rc = qgemv_i4_impl(static_cast<const uint8_t*>(o.w), static_cast<const uint16_t*>(o.scales), o.n_scales,
+            rc = qgemv_i4_impl(ctx, static_cast<const uint8_t*>(o.w), static_cast<const uint16_t*>(o.scales), o.n_scales,
                                o.group, o.x, o.x_dtype, o.y, o.m, o.n, o.k, st);
         else
             rc = set_error(CELLM_HIP_ERR_INVALID_ARG, "op %lld: unknown kind %d", (long long)i, (int)o.kind);
@@ -889,7 +895,7 @@ int32_t cellm_hip_qgemv_q4_affine_gate_up_gelu(cellm_hip_ctx_t* ctx, const uint3
     CELLM_API_END(report_exception)
 }
 
-static int32_t qgemv_i4_impl(const uint8_t* w, const uint16_t* scales_f16, int64_t n_scales, int64_t gs,
+static int32_t qgemv_i4_impl(cellm_hip_ctx* ctx, const uint8_t* w, const uint16_t* scales_f16, int64_t n_scales, int64_t gs,
                              const void* x, int32_t x_dtype, float* y, int64_t m, int64_t n, int64_t k, hipStream_t st)
 {
     if (int32_t rc = check_dims(m, n, k)) return rc;
@@ -902,6 +908,12 @@ static int32_t qgemv_i4_impl(const uint8_t* w, const uint16_t* scales_f16, int64
         return set_error(CELLM_HIP_ERR_INVALID_ARG, "scale index (k-1)/gs=%lld out of range spr=%lld",
                          (long long)((k - 1) / gs), (long long)spr);
     if ((k > 0 && (!w || !scales_f16 || !x)) || !y) return set_error(CELLM_HIP_ERR_INVALID_ARG, "null pointer");
+    if (x_dtype == DT_F32 && k > 0 && (k - 1) / gs == 0 && spr <= INT32_MAX) {  // one scale per row
+        const XgSeg seg{w, scales_f16, nullptr, y, (int)n, (int)spr};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, XG_I4, &seg, 1, DT_F16, x, m, k, st, &done)) return rc;
+        if (done) return CELLM_HIP_OK;
+    }
     HIP_TRY(launch_qgemv_i4_sym(w, scales_f16, (int)spr, (int)gs, x, x_dtype, y, (int)m, (int)n, (int)k, st),
             "qgemv_i4_sym launch");
     return CELLM_HIP_OK;
@@ -924,8 +936,8 @@ int32_t cellm_hip_qgemv_i4_gate_up_gelu(cellm_hip_ctx_t* ctx, const uint8_t* wg,
     hipStream_t st = pick_stream(ctx, stream);
     float* up = nullptr;
     if (int32_t rc = get_stream_buffer(ctx, ctx->aux, st, (size_t)m * n * sizeof(float), &up)) return rc;
-    if (int32_t rc = qgemv_i4_impl(wg, sg, n_sg, gs, x, x_dtype, h, m, n, k, st)) return rc;
-    if (int32_t rc = qgemv_i4_impl(wu, su, n_su, gs, x, x_dtype, up, m, n, k, st)) return rc;
+    if (int32_t rc = qgemv_i4_impl(ctx, wg, sg, n_sg, gs, x, x_dtype, h, m, n, k, st)) return rc;
+    if (int32_t rc = qgemv_i4_impl(ctx, wu, su, n_su, gs, x, x_dtype, up, m, n, k, st)) return rc;
     HIP_TRY(launch_act_mul(ACT_GELU_TANH, h, up, (size_t)m * n, st), "gelu_tanh_mul launch");
     return CELLM_HIP_OK;
     CELLM_API_END(report_exception)
@@ -938,7 +950,8 @@ int32_t cellm_hip_qgemv_i4_sym(cellm_hip_ctx_t* ctx, const uint8_t* w, const uin
     CELLM_API_BEGIN
     if (int32_t rc = check_ctx(ctx)) return rc;
     DeviceGuard g(ctx->device);
-    return qgemv_i4_impl(w, scales_f16, n_scales, gs, x, x_dtype, y, m, n, k, pick_stream(ctx, stream));
+    const std::lock_guard<std::recursive_mutex> lk(ctx->mu);  // held until the scratch users are enqueued
+    return qgemv_i4_impl(ctx, w, scales_f16, n_scales, gs, x, x_dtype, y, m, n, k, pick_stream(ctx, stream));
     CELLM_API_END(report_exception)
 }
 
@@ -948,7 +961,8 @@ int32_t cellm_hip_qgemv_f16(cellm_hip_ctx_t* ctx, const uint16_t* w_f16, const v
     CELLM_API_BEGIN
     if (int32_t rc = check_ctx(ctx)) return rc;
     DeviceGuard g(ctx->device);
-    return qgemv_lowbit_impl(LB_F16, w_f16, nullptr, 0, x, x_dtype, y, m, n, k, pick_stream(ctx, stream));
+    const std::lock_guard<std::recursive_mutex> lk(ctx->mu);  // held until the scratch users are enqueued
+    return qgemv_lowbit_impl(ctx, LB_F16, w_f16, nullptr, 0, x, x_dtype, y, m, n, k, pick_stream(ctx, stream));
     CELLM_API_END(report_exception)
 }
 
@@ -958,7 +972,8 @@ int32_t cellm_hip_qgemv_i2(cellm_hip_ctx_t* ctx, const uint8_t* w, const uint16_
     CELLM_API_BEGIN
     if (int32_t rc = check_ctx(ctx)) return rc;
     DeviceGuard g(ctx->device);
-    return qgemv_lowbit_impl(LB_I2, w, scales_f16, scale_mode, x, x_dtype, y, m, n, k, pick_stream(ctx, stream));
+    const std::lock_guard<std::recursive_mutex> lk(ctx->mu);  // held until the scratch users are enqueued
+    return qgemv_lowbit_impl(ctx, LB_I2, w, scales_f16, scale_mode, x, x_dtype, y, m, n, k, pick_stream(ctx, stream));
     CELLM_API_END(report_exception)
 }
 
@@ -968,7 +983,8 @@ int32_t cellm_hip_qgemv_q1_0_g128(cellm_hip_ctx_t* ctx, const uint8_t* w, const 
     CELLM_API_BEGIN
     if (int32_t rc = check_ctx(ctx)) return rc;
     DeviceGuard g(ctx->device);
-    return qgemv_lowbit_impl(LB_Q1, w, nullptr, 0, x, x_dtype, y, m, n, k, pick_stream(ctx, stream));
+    const std::lock_guard<std::recursive_mutex> lk(ctx->mu);  // held until the scratch users are enqueued
+    return qgemv_lowbit_impl(ctx, LB_Q1, w, nullptr, 0, x, x_dtype, y, m, n, k, pick_stream(ctx, stream));
     CELLM_API_END(report_exception)
 }
 

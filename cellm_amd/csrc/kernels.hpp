@@ -86,15 +86,16 @@ hipError_t launch_qgemm_i8_ws(const int8_t* w, const void* S, int sdt, int per_c
                               const float* bias, float* y, int M, int N, int K, float* workspace, hipStream_t st);
 
 // Multi-row GEMM over f32 x, weights exact in f16 (qgemm_exact.hip): M >= 5 (and rows enough to pay
-// for its launches), K % 16 == 0, 16-byte aligned W and x.  Up to three matrices share x.  `ws` holds x's f16 parts and the split sums.
-enum { XG_I8 = 0 };
+// for its launches), 16-byte aligned W, x and weight rows.  Up to three matrices share x.  `ws` holds
+// x's f16 parts and the split sums.
+enum { XG_I8 = 0, XG_I4 = 1, XG_F16 = 2 };
 struct XgSeg {
     const void* w;
-    const void* s;
-    const float* bias;
+    const void* s;     // row scales of dtype sdt at s[n * s_stride], or nullptr
+    const float* bias;  // [n], or nullptr
     float* y;
     int n;
-    int per_channel;
+    int s_stride;      // 0: one scale per tensor
 };
 bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int M, int K, const void* x);
 size_t qgemm_exact_workspace_bytes(const XgSeg* segs, int nseg, int M, int K);

@@ -2,9 +2,10 @@
 //
 //   Y[m,n] = (sum_k w[n,k] x[m,k]) * scale[n] (+ bias[n]),   w exact in f16
 //
-// for M >= 5 rows of f32 activations over int8 weights
-// (cpu_kernels::matmul_i8_f32, crates/cellm-kernels/src/cpu_kernels.rs:66-133,
-// run once per prompt token by the reference, crates/cellm-model/src/llama.rs:214-233).
+// for M >= 5 rows of f32 activations over int8, symmetric 4-bit (one scale per
+// row) and f16 weights (cpu_kernels::matmul_i8_f32, matmul_i4_f32, matmul_f16_f32,
+// crates/cellm-kernels/src/cpu_kernels.rs:66-243, run once per prompt token by the
+// reference, crates/cellm-model/src/llama.rs:214-233).
 //
 // f32 activations keep their 24 bits: a first kernel scales each row by the
 // power of two that puts its largest |x| in [2^13, 2^14) and splits it into
@@ -25,7 +26,7 @@
 // Measured, int8 at 512 rows (us, one-wave-per-row kernel -> this one with its
 // split of x): 960 -> 960 1963 -> 20, 2560 -> 960 5098 -> 25, 4096 -> 4096
 // 8034 -> 60; 16 rows of 1152 -> 1536 35 -> 15; 2048 rows of 2048 -> 8192 164,
-// 839 TFLOP/s of MFMA work.  The small ones are bound by three dependent launches
+// 839 TFLOP/s of MFMA work; 16 rows of 2560 -> 960, i4 109 -> 14, f16 63 -> 14.  The small ones are bound by three dependent launches
 // and the latency of a few K steps, the wide ones by the MFMAs.
 //
 // Tile: WM x WN waves of (32 TA) x (32 TB); X parts and raw weights go
@@ -70,6 +71,17 @@ struct Fmt;
 template <>
 struct Fmt<XG_I8> {
     static constexpr int kStepBytes = 64;  // of a weight row per K step
+    static constexpr bool kPairs = false;  // x in k order
+};
+template <>
+struct Fmt<XG_I4> {
+    static constexpr int kStepBytes = 32;
+    static constexpr bool kPairs = true;  // each 8 x as 0,4,1,5,2,6,3,7: the order nib8 unpacks a word in
+};
+template <>
+struct Fmt<XG_F16> {
+    static constexpr int kStepBytes = 128;
+    static constexpr bool kPairs = false;
 };
 
 template <int FMT>
@@ -87,6 +99,21 @@ __device__ __forceinline__ h8_t i8x8(uint32_t w0, uint32_t w1)
     const h2_t a1 = as_h2(__builtin_amdgcn_perm(hi, b0, 0x04030402u)) - off;
     const h2_t a2 = as_h2(__builtin_amdgcn_perm(hi, b1, 0x04010400u)) - off;
     const h2_t a3 = as_h2(__builtin_amdgcn_perm(hi, b1, 0x04030402u)) - off;
+    return h8_t{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+}
+
+// the eight nibbles of a word minus 8 as f16, in the order 0,4,1,5,2,6,3,7: the low nibble of a byte
+// lands as 1024 + q, the high one as 1024 + 16 q, which one fma takes to q - 8
+__device__ __forceinline__ h8_t nib8(uint32_t w)
+{
+    const uint32_t mlo = 0x000F000Fu, mhi = 0x00F000F0u, magic = 0x64006400u;
+    const h2_t off = {(_Float16)1032.0f, (_Float16)1032.0f}, off16 = {(_Float16)-72.0f, (_Float16)-72.0f},
+               inv = {(_Float16)0.0625f, (_Float16)0.0625f};
+    const uint32_t v = w >> 8;
+    const h2_t a0 = as_h2(and_or(w, mlo, magic)) - off;
+    const h2_t a1 = __builtin_elementwise_fma(as_h2(and_or(w, mhi, magic)), inv, off16);
+    const h2_t a2 = as_h2(and_or(v, mlo, magic)) - off;
+    const h2_t a3 = __builtin_elementwise_fma(as_h2(and_or(v, mhi, magic)), inv, off16);
     return h8_t{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
 }
 
@@ -114,7 +141,11 @@ __device__ __forceinline__ float plain_dot(const XgSeg& g, const void* x, int m,
         float xv;
         if constexpr (P == 2) xv = static_cast<const float*>(x)[(size_t)m * K + k];
         else xv = (float)static_cast<const _Float16*>(x)[(size_t)m * K + k];
-        if constexpr (FMT == XG_I8) acc += (float)static_cast<const int8_t*>(g.w)[(size_t)n * K + k] * xv;
+        float w;
+        if constexpr (FMT == XG_I8) w = (float)static_cast<const int8_t*>(g.w)[(size_t)n * K + k];
+        else if constexpr (FMT == XG_F16) w = (float)static_cast<const _Float16*>(g.w)[(size_t)n * K + k];
+        else w = (float)((static_cast<const uint8_t*>(g.w)[((size_t)n * K + k) >> 1] >> (4 * (k & 1))) & 15) - 8.0f;
+        acc += w * xv;
     }
     return acc;
 }
@@ -123,7 +154,7 @@ __device__ __forceinline__ bool finite_f32(float v) { return (__builtin_bit_cast
 
 __device__ __forceinline__ float column_scale(const XgSeg& g, int sdt, int n)
 {
-    return scale_at(g.s, sdt, g.per_channel ? (size_t)n : 0);
+    return g.s ? scale_at(g.s, sdt, (size_t)n * g.s_stride) : 1.0f;
 }
 
 template <int FMT, int P, int TA, int TB, int WM, int WN, int NST>
@@ -218,6 +249,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
                     b[j][2 * c] = i8x8(w[0], w[1]);
                     b[j][2 * c + 1] = i8x8(w[2], w[3]);
                 }
+            } else if constexpr (FMT == XG_F16) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    b[j][c] = *reinterpret_cast<const h8_t*>(ws + r * RB + 16 * swz<RB>(r, 4 * h32 + c));
+            } else {
+                const u4_t w = *reinterpret_cast<const u4_t*>(ws + r * RB + 16 * h32);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) b[j][c] = nib8(w[c]);
             }
         }
 #pragma unroll
@@ -340,6 +379,7 @@ __global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a,
 // One block per row of x: its parts, zero-padded to Kp, and its exponent.  Eight elements per thread
 // and round; rows of up to 8192 stay in registers between the maximum and the split.
 constexpr int kSplitUnits = 4;
+template <bool PAIRS>
 __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ x, int K, int Kp,
                                                       _Float16* __restrict__ xp, int32_t* __restrict__ xe)
 {
@@ -387,7 +427,8 @@ __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ 
         h8_t hi, lo;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float s = ldexpf(d[i >> 2][i & 3], e);
+            const int k = PAIRS ? (i >> 1) + 4 * (i & 1) : i;
+            const float s = ldexpf(d[k >> 2][k & 3], e);
             hi[i] = (_Float16)s;
             lo[i] = finite_f32(s) ? (_Float16)(s - (float)hi[i]) : (_Float16)0.0f;
         }
@@ -457,11 +498,16 @@ hipError_t launch_form(const XgArgs& a, const XgPlan& p, hipStream_t st)
 
 bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int M, int K, const void* x)
 {
-    if (fmt != XG_I8 || M < 5 || K <= 0 || K % 16 != 0) return false;
-    // the one-wave-per-row kernels walk the rows one after the other, about 2 ns per row and element of
-    // k; the three launches here take 14-16 us (5 rows of 960 -> 960: 10.7 against 16.2 us, of 1536 ->
-    // 576: 15.2 against 14.4).  Long outputs cost them more (5 rows of 960 -> 32768: 68 against 18.5)
-    if ((int64_t)M * K < 7000 && segs[0].n < 8192) return false;
+    // weight rows start on 16-byte boundaries
+    if (M < 5 || K <= 0 || K % (fmt == XG_I4 ? 32 : fmt == XG_I8 ? 16 : 8) != 0) return false;
+    // the kernels of single rows walk the rows one after the other, 1.2 (f16) to 3.2 ns (i4) per row and
+    // element of k, the f16 ones four rows at a time; the three launches here take 14-16 us.  int8: 5 rows
+    // of 960 -> 960 10.7 against 16.2 us, of 1536 -> 576 15.2 against 14.4; i4: 5 of 960 -> 960 16.0
+    // against 16.0, 8 24.4 against 15.3; f16: 8 of 960 -> 960 11.3 against 14.9, 5 of 1536 -> 960 12.1
+    // against 12.4, 12 of 960 -> 2560 21.2 against 14.9.  Long outputs cost the row kernels more (int8, 5
+    // rows of 960 -> 32768: 68 against 18.5)
+    const int64_t pays = fmt == XG_F16 ? 10000 : fmt == XG_I4 ? 5000 : 7000;
+    if ((int64_t)M * K < pays && segs[0].n < 8192) return false;
     if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (M + 31) / 32 > 65535) return false;
     int64_t n = 0;
     for (int i = 0; i < nseg; ++i) {
@@ -478,10 +524,27 @@ size_t qgemm_exact_workspace_bytes(const XgSeg* segs, int nseg, int M, int K)
     return xg_plan(n, nseg, M, K).bytes;
 }
 
+template <int FMT>
+static hipError_t launch_fmt(XgArgs& a, const XgPlan& p, const float* x, int32_t* xe, _Float16* xp, hipStream_t st)
+{
+    hipLaunchKernelGGL((split_x_kernel<Fmt<FMT>::kPairs>), dim3(a.M), dim3(256), 0, st, x, a.K, a.Kp, xp, xe);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    // f16 rows are twice the bytes: two stages keep two blocks (form 1) or one (form 2) on a CU
+    constexpr int NST = FMT == XG_F16 ? 2 : 3;
+    e = p.form == 2   ? launch_form<FMT, 2, 2, 2, 2, 4, NST>(a, p, st)
+        : p.form == 1 ? launch_form<FMT, 2, 1, 2, 2, 2, NST>(a, p, st)
+                      : launch_form<FMT, 2, 1, 2, 1, 2, 3>(a, p, st);
+    if (e != hipSuccess || p.splits == 1) return e;
+    const size_t quads = (size_t)a.M * a.vcols / 4;
+    const unsigned blocks = (unsigned)std::min<size_t>((quads + 255) / 256, 4096);
+    hipLaunchKernelGGL((qgemm_exact_reduce_kernel<FMT, 2>), dim3(blocks), dim3(256), 0, st, a, p.splits, p.bn);
+    return hipGetLastError();
+}
+
 hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, const float* x, int M, int K, void* ws,
                               hipStream_t st)
 {
-    if (fmt != XG_I8) return hipErrorInvalidValue;
     const int n[3] = {segs[0].n, nseg > 1 ? segs[1].n : 0, nseg > 2 ? segs[2].n : 0};
     const XgPlan p = xg_plan(n, nseg, M, K);
     XgArgs a{};
@@ -504,17 +567,12 @@ hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, con
     a.steps_per_split = p.steps_per_split;
     a.vcols = p.vtiles * p.bn;
     a.sdt = sdt;
-    hipLaunchKernelGGL(split_x_kernel, dim3(M), dim3(256), 0, st, x, K, a.Kp, xp, xe);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    e = p.form == 2   ? launch_form<XG_I8, 2, 2, 2, 2, 4, 3>(a, p, st)
-        : p.form == 1 ? launch_form<XG_I8, 2, 1, 2, 2, 2, 3>(a, p, st)
-                      : launch_form<XG_I8, 2, 1, 2, 1, 2, 3>(a, p, st);
-    if (e != hipSuccess || p.splits == 1) return e;
-    const size_t quads = (size_t)M * a.vcols / 4;
-    const unsigned blocks = (unsigned)std::min<size_t>((quads + 255) / 256, 4096);
-    hipLaunchKernelGGL((qgemm_exact_reduce_kernel<XG_I8, 2>), dim3(blocks), dim3(256), 0, st, a, p.splits, p.bn);
-    return hipGetLastError();
+    switch (fmt) {
+        case XG_I8: return launch_fmt<XG_I8>(a, p, x, xe, xp, st);
+        case XG_I4: return launch_fmt<XG_I4>(a, p, x, xe, xp, st);
+        case XG_F16: return launch_fmt<XG_F16>(a, p, x, xe, xp, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace cellm

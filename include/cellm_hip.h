@@ -272,14 +272,18 @@ typedef struct {
 int32_t cellm_hip_qgemv_batch(cellm_hip_ctx_t* ctx, const cellm_hip_qgemv_op_t* ops, int64_t n_ops, void* stream);
 
 /* Symmetric i4 GEMV: y[i, r] = sum_j ((nib - 8) * scale[r*spr + j/gs]) * x[i, j],
- * spr = n_scales / n.  Replaces cpu_kernels::matmul_i4_f32 (cpu_kernels.rs:219-243)
+ * spr = n_scales / n.  f32 x at 5 rows and more with one scale per row (gs >= k)
+ * runs on MFMA as in cellm_hip_qgemv_i8 (k % 32 == 0, 16-byte aligned w and x,
+ * m * k >= 5000 or n >= 8192).  Replaces cpu_kernels::matmul_i4_f32 (cpu_kernels.rs:219-243)
  * and MetalOps::encode_mv_i4 (metal.rs:1167-1176). */
 int32_t cellm_hip_qgemv_i4_sym(cellm_hip_ctx_t* ctx, const uint8_t* w, const uint16_t* scales_f16, int64_t n_scales,
                                int64_t gs, const void* x, int32_t x_dtype, float* y, int64_t m, int64_t n, int64_t k,
                                void* stream);
 
 /* f16-weight GEMV: y[i, r] = sum_j f32(W[r, j]) * x[i, j], W [n][k] f16
- * (2-byte aligned).  Replaces cpu_kernels::matmul_f16_f32
+ * (2-byte aligned).  f32 x at 5 rows and more runs on MFMA as in
+ * cellm_hip_qgemv_i8 (k % 8 == 0, 16-byte aligned w and x, m * k >= 10000 or
+ * n >= 8192).  Replaces cpu_kernels::matmul_f16_f32
  * (cpu_kernels.rs:135-214) in the runners' "f16" linear arms (qwen.rs:1073,
  * llama.rs:898) and MetalOps::encode_mv_f16 / mv_f16 (metal.rs:347-363,
  * 1089). */

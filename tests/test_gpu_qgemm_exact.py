@@ -53,6 +53,52 @@ def test_i8_f32_rows(ops, m, n, k, sdt):
     assert _rel(y.cpu(), ref) <= TOL
 
 
+@pytest.mark.parametrize("m,n,k", [s for s in SIZES if s[2] % 32 == 0])
+@pytest.mark.parametrize("spr", [1, 3])  # scales per row; the first one holds for the whole row
+def test_i4_f32_rows(ops, m, n, k, spr):
+    g = torch.Generator().manual_seed(m + n + k)
+    w = torch.randint(0, 256, (n, k // 2), generator=g, dtype=torch.uint8)
+    s = (torch.rand(n, spr, generator=g) * 0.01 + 1e-3).half()
+    q = torch.stack([w & 15, w >> 4], 2).reshape(n, k).double() - 8
+    x = _x(m, k, m + k)
+    y = torch.full((m, n), float("nan"), device="cuda")
+    ops.encode_qgemv_i4_sym(w.cuda(), s.cuda(), k, x.cuda(), y, k)
+    torch.cuda.synchronize()
+    assert _rel(y.cpu(), x.double() @ q.t() * s[:, 0].double()) <= TOL
+
+
+@pytest.mark.parametrize("m,n,k", SIZES + [(300, 70, 8), (64, 130, 904)])
+def test_f16_weights_f32_rows(ops, m, n, k):
+    g = torch.Generator().manual_seed(m + n + k)
+    w = (torch.randn(n, k, generator=g) * 0.02).half()
+    w[0, 0] = 6e-8  # a subnormal weight
+    x = _x(m, k, m + k)
+    y = torch.full((m, n), float("nan"), device="cuda")
+    ops.encode_qgemv_f16(w.cuda(), x.cuda(), y)
+    torch.cuda.synchronize()
+    assert _rel(y.cpu(), x.double() @ w.double().t()) <= TOL
+
+
+@pytest.mark.parametrize("k", [840, 2560])  # a ragged last step; split over k
+def test_f16_non_finite_weights(ops, k):
+    """An infinite weight gives the infinities (and 0 * inf its NaN) of a plain f32 sum, in its own column only."""
+    m, n = 10, 70
+    x = _x(m, k, 2)
+    w = (torch.randn(n, k, generator=torch.Generator().manual_seed(3)) * 0.02).half()
+    w[3, k - 1], w[4, 0], w[5, 1], w[5, 2] = float("inf"), float("nan"), float("inf"), float("-inf")
+    x[2, k - 1] = 0.0
+    x[1, 1], x[1, 2] = 1.0, 1.0
+    y = torch.empty(m, n, device="cuda")
+    ops.encode_qgemv_f16(w.cuda(), x.cuda(), y)
+    torch.cuda.synchronize()
+    got, ref = y.cpu(), x @ w.float().t()
+    assert np.array_equal(torch.isnan(got).numpy(), torch.isnan(ref).numpy())
+    assert np.array_equal(torch.isinf(got).numpy(), torch.isinf(ref).numpy())
+    assert torch.equal(torch.sign(got[:, 3]).nan_to_num(), torch.sign(ref[:, 3]).nan_to_num())
+    fine = [c for c in range(n) if c not in (3, 4, 5)]
+    assert _rel(got[:, fine], x.double() @ w[fine].double().t()) <= TOL
+
+
 def test_i8_per_tensor_scale_and_row_spread(ops):
     """Rows whose magnitudes lie 2^80 apart (zero and subnormal rows among them) keep their own precision."""
     m, n, k = 40, 130, 192
