@@ -237,19 +237,20 @@ bool capturing(hipStream_t st)
 // The multi-row GEMM over f32 x (qgemm_exact.hip) where it applies: *done tells whether it was enqueued.
 // It needs scratch for x's parts, which the one-wave-per-row kernels do without, so a call that cannot
 // have it (captures, no memory) is left to them.
-int32_t try_qgemm_exact(cellm_hip_ctx* ctx, int fmt, const XgSeg* segs, int nseg, int32_t sdt, const void* x,
-                        int64_t m, int64_t k, hipStream_t st, bool* done)
+int32_t try_qgemm_exact(cellm_hip_ctx* ctx, int fmt, const XgSeg* segs, int nseg, int32_t sdt, int64_t group,
+                        int64_t gpr, const void* x, int64_t m, int64_t k, hipStream_t st, bool* done)
 {
     *done = false;
-    if (!qgemm_exact_supported(fmt, segs, nseg, (int)m, (int)k, x) || capturing(st)) return CELLM_HIP_OK;
+    if (!qgemm_exact_supported(fmt, segs, nseg, (int)group, (int)m, (int)k, x) || capturing(st)) return CELLM_HIP_OK;
     float* ws = nullptr;
-    const int32_t rc = get_workspace(ctx, st, qgemm_exact_workspace_bytes(segs, nseg, (int)m, (int)k), &ws);
+    const int32_t rc = get_workspace(ctx, st, qgemm_exact_workspace_bytes(fmt, segs, nseg, (int)m, (int)k), &ws);
     if (rc == CELLM_HIP_ERR_OUT_OF_MEMORY) {
         (void)hipGetLastError();
         return CELLM_HIP_OK;
     }
     if (rc) return rc;
-    HIP_TRY(launch_qgemm_exact(fmt, segs, nseg, sdt, static_cast<const float*>(x), (int)m, (int)k, ws, st),
+    HIP_TRY(launch_qgemm_exact(fmt, segs, nseg, sdt, (int)group, (int)gpr, static_cast<const float*>(x), (int)m,
+                               (int)k, ws, st),
             "qgemm_exact launch");
     *done = true;
     return CELLM_HIP_OK;
@@ -299,9 +300,9 @@ int32_t qgemv_i8_impl(cellm_hip_ctx* ctx, const int8_t* w, const void* scales, i
         return CELLM_HIP_OK;
     }
     if (xdt == DT_F32) {
-        const XgSeg seg{w, scales, bias, y, (int)n, per_channel};
+        const XgSeg seg{w, scales, bias, y, (int)n, per_channel, nullptr, nullptr};
         bool done = false;
-        if (int32_t rc = try_qgemm_exact(ctx, XG_I8, &seg, 1, sdt, x, m, k, st, &done)) return rc;
+        if (int32_t rc = try_qgemm_exact(ctx, XG_I8, &seg, 1, sdt, 0, 0, x, m, k, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;
     }
     HIP_TRY(launch_qgemv_i8(w, scales, sdt, per_channel, x, xdt, bias, y, (int)m, (int)n, (int)k, st, k == 0),
@@ -329,9 +330,9 @@ int32_t qgemv_lowbit_impl(cellm_hip_ctx* ctx, int fmt, const void* w, const uint
         return CELLM_HIP_OK;
     }
     if (fmt == LB_F16 && xdt == DT_F32) {
-        const XgSeg seg{w, nullptr, nullptr, y, (int)n, 0};
+        const XgSeg seg{w, nullptr, nullptr, y, (int)n, 0, nullptr, nullptr};
         bool done = false;
-        if (int32_t rc = try_qgemm_exact(ctx, XG_F16, &seg, 1, DT_F32, x, m, k, st, &done)) return rc;
+        if (int32_t rc = try_qgemm_exact(ctx, XG_F16, &seg, 1, DT_F32, 0, 0, x, m, k, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;
     }
     HIP_TRY(launch_qgemv_lowbit(fmt, w, scales_f16, scale_mode, x, xdt, y, (int)m, (int)n, (int)k, st),
@@ -400,6 +401,13 @@ int32_t qgemv_q4_impl(cellm_hip_ctx* ctx, const uint32_t* wq, const void* scales
     }
     if (force_gemm)
         return set_error(CELLM_HIP_ERR_UNSUPPORTED, "qgemm_q4_affine needs f16 x, k %% 64 == 0, group >= 32, alignment");
+    if (xdt == DT_F32) {
+        const XgSeg seg{wq, nullptr, nullptr, y, (int)n, 0, scales, biases};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, XG_Q4, &seg, 1, sbt, group, (k + group - 1) / group, x, m, k, st, &done))
+            return rc;
+        if (done) return CELLM_HIP_OK;
+    }
     HIP_TRY(launch_qgemv_q4_affine(wq, scales, biases, sbt, (int)group, x, xdt, y, (int)m, (int)n, (int)k, st, k == 0),
             "qgemv_q4_affine launch");
     return CELLM_HIP_OK;
@@ -908,10 +916,13 @@ static int32_t qgemv_i4_impl(cellm_hip_ctx* ctx, const uint8_t* w, const uint16_
         return set_error(CELLM_HIP_ERR_INVALID_ARG, "scale index (k-1)/gs=%lld out of range spr=%lld",
                          (long long)((k - 1) / gs), (long long)spr);
     if ((k > 0 && (!w || !scales_f16 || !x)) || !y) return set_error(CELLM_HIP_ERR_INVALID_ARG, "null pointer");
-    if (x_dtype == DT_F32 && k > 0 && (k - 1) / gs == 0 && spr <= INT32_MAX) {  // one scale per row
-        const XgSeg seg{w, scales_f16, nullptr, y, (int)n, (int)spr};
+    if (x_dtype == DT_F32 && k > 0 && spr <= INT32_MAX && gs <= INT32_MAX) {
+        const bool per_row = (k - 1) / gs == 0;  // the row's last element still uses its first scale
+        const XgSeg seg{w,      per_row ? scales_f16 : nullptr, nullptr, y, (int)n, (int)spr,
+                        per_row ? nullptr : scales_f16, nullptr};
         bool done = false;
-        if (int32_t rc = try_qgemm_exact(ctx, XG_I4, &seg, 1, DT_F16, x, m, k, st, &done)) return rc;
+        if (int32_t rc = try_qgemm_exact(ctx, per_row ? XG_I4 : XG_Q4, &seg, 1, DT_F16, gs, spr, x, m, k, st, &done))
+            return rc;
         if (done) return CELLM_HIP_OK;
     }
     HIP_TRY(launch_qgemv_i4_sym(w, scales_f16, (int)spr, (int)gs, x, x_dtype, y, (int)m, (int)n, (int)k, st),

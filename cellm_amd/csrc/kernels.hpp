@@ -88,7 +88,7 @@ hipError_t launch_qgemm_i8_ws(const int8_t* w, const void* S, int sdt, int per_c
 // Multi-row GEMM over f32 x, weights exact in f16 (qgemm_exact.hip): M >= 5 (and rows enough to pay
 // for its launches), 16-byte aligned W, x and weight rows.  Up to three matrices share x.  `ws` holds
 // x's f16 parts and the split sums.
-enum { XG_I8 = 0, XG_I4 = 1, XG_F16 = 2 };
+enum { XG_I8 = 0, XG_I4 = 1, XG_F16 = 2, XG_Q4 = 3 };
 struct XgSeg {
     const void* w;
     const void* s;     // row scales of dtype sdt at s[n * s_stride], or nullptr
@@ -96,11 +96,14 @@ struct XgSeg {
     float* y;
     int n;
     int s_stride;      // 0: one scale per tensor
+    const void* gs;    // XG_Q4: group scales of dtype sdt [n][gpr], and group biases: w = q gs + gb, or
+    const void* gb;    // nullptr: w = (q - 8) gs
 };
-bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int M, int K, const void* x);
-size_t qgemm_exact_workspace_bytes(const XgSeg* segs, int nseg, int M, int K);
-hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, const float* x, int M, int K, void* ws,
-                              hipStream_t st);
+// group, gpr: XG_Q4's elements per scale (a multiple of 64) and scales per row.
+bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int group, int M, int K, const void* x);
+size_t qgemm_exact_workspace_bytes(int fmt, const XgSeg* segs, int nseg, int M, int K);
+hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, int group, int gpr, const float* x, int M,
+                              int K, void* ws, hipStream_t st);
 
 // Batched decode on MFMA (2 <= M <= 64, f16 x): int8 needs K % 64 == 0 and
 // K >= 128, q4 K % 128 == 0, K >= 256 and group >= 32; 16-byte aligned W and x;

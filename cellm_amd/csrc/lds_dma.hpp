@@ -37,6 +37,14 @@ __device__ __forceinline__ void dma4_s(uint32_t voff, const void* sbase, uint32_
                  : "memory", "m0");
 }
 
+// 2 bytes per lane, zero-extended; lane i lands at lds + 4 i
+__device__ __forceinline__ void dma2_s(uint32_t voff, const void* sbase, uint32_t lds)
+{
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_ushort %0, %1" ::"v"(voff), "s"(sbase),
+                 "s"(__builtin_amdgcn_readfirstlane(lds))
+                 : "memory", "m0");
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt()
 {

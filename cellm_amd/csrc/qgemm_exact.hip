@@ -1,11 +1,18 @@
 // Multi-row GEMM on f16 MFMA whose weights are exact in f16 (gfx950):
 //
-//   Y[m,n] = (sum_k w[n,k] x[m,k]) * scale[n] (+ bias[n]),   w exact in f16
+//   Y[m,n] = (sum_k w[n,k] x[m,k]) * scale[n] (+ bias[n]),   w (or q - 8) exact in f16
 //
-// for M >= 5 rows of f32 activations over int8, symmetric 4-bit (one scale per
-// row) and f16 weights (cpu_kernels::matmul_i8_f32, matmul_i4_f32, matmul_f16_f32,
+// for M >= 5 rows of f32 activations over int8, symmetric 4-bit and f16 weights
+// (cpu_kernels::matmul_i8_f32, matmul_i4_f32, matmul_f16_f32,
 // crates/cellm-kernels/src/cpu_kernels.rs:66-243, run once per prompt token by the
-// reference, crates/cellm-model/src/llama.rs:214-233).
+// reference, crates/cellm-model/src/llama.rs:214-233) and MLX 4-bit affine ones
+// (crates/cellm-model/src/lfm.rs:985-1066).
+//
+// Group-scaled nibbles (w = q s + b or (q - 8) s, one scale per 64 k or a multiple)
+// multiply as the exact q - 8: every K step's sum is folded as
+// sum += s acc + (b + 8 s) sum(x'), the sums of x' coming from the split kernel and
+// the step's scales and biases with the weights through the DMA ring.  With q - 8
+// in place of q the step's two terms do not cancel (b is near -7.5 s).
 //
 // f32 activations keep their 24 bits: a first kernel scales each row by the
 // power of two that puts its largest |x| in [2^13, 2^14) and splits it into
@@ -26,7 +33,8 @@
 // Measured, int8 at 512 rows (us, one-wave-per-row kernel -> this one with its
 // split of x): 960 -> 960 1963 -> 20, 2560 -> 960 5098 -> 25, 4096 -> 4096
 // 8034 -> 60; 16 rows of 1152 -> 1536 35 -> 15; 2048 rows of 2048 -> 8192 164,
-// 839 TFLOP/s of MFMA work; 16 rows of 2560 -> 960, i4 109 -> 14, f16 63 -> 14.  The small ones are bound by three dependent launches
+// 839 TFLOP/s of MFMA work; 16 rows of 2560 -> 960, i4 109 -> 14, f16 63 -> 14; MLX
+// q4 with f32 scales, 512 rows of 4096 -> 4096, 1480 -> 66 (error 1.6e-7, as before).  The small ones are bound by three dependent launches
 // and the latency of a few K steps, the wide ones by the MFMAs.
 //
 // Tile: WM x WN waves of (32 TA) x (32 TB); X parts and raw weights go
@@ -59,11 +67,13 @@ struct XgArgs {
     const _Float16* xp;   // [M][P][Kp] activation parts
     const int32_t* xe;    // [M] row exponents e (x' = x 2^e); P == 2
     const void* x;        // the caller's activations [M][K], for the recomputed sums
+    const float* xsum;    // XG_Q4: sum of x' over the 64 k of each step, [steps][M]
     float* part;          // [splits][M][vcols] raw sums, or nullptr (unsplit)
     int M, K, Kp;
     int steps_per_split;
     int vcols;            // column tiles * BN
     int sdt;
+    int group, gpr;       // XG_Q4: elements per scale, scales per row
 };
 
 template <int FMT>
@@ -79,10 +89,17 @@ struct Fmt<XG_I4> {
     static constexpr bool kPairs = true;  // each 8 x as 0,4,1,5,2,6,3,7: the order nib8 unpacks a word in
 };
 template <>
+struct Fmt<XG_Q4> : Fmt<XG_I4> {};
+template <>
 struct Fmt<XG_F16> {
     static constexpr int kStepBytes = 128;
     static constexpr bool kPairs = false;
 };
+
+constexpr int stage_bytes(int fmt, int P, int bm, int bn, int step_bytes)
+{
+    return bm * P * 128 + bn * step_bytes + (fmt == XG_Q4 ? 8 * bn + 4 * (bm > 64 ? bm : 64) : 0);
+}
 
 template <int FMT>
 __device__ __forceinline__ size_t row_bytes(int K)
@@ -134,8 +151,11 @@ __device__ __forceinline__ float scale_at(const void* s, int sdt, size_t i)
 
 // sum_k w[n,k] x[m,k] by a plain f32 loop: the results that MFMA left non-finite
 template <int FMT, int P>
-__device__ __forceinline__ float plain_dot(const XgSeg& g, const void* x, int m, int n, int K)
+__device__ __forceinline__ float plain_dot(const XgArgs& a, const XgSeg& g, int m, int n)
 {
+#pragma clang fp contract(off)
+    const int K = a.K;
+    const void* x = a.x;
     float acc = 0.0f;
     for (int k = 0; k < K; ++k) {
         float xv;
@@ -144,7 +164,14 @@ __device__ __forceinline__ float plain_dot(const XgSeg& g, const void* x, int m,
         float w;
         if constexpr (FMT == XG_I8) w = (float)static_cast<const int8_t*>(g.w)[(size_t)n * K + k];
         else if constexpr (FMT == XG_F16) w = (float)static_cast<const _Float16*>(g.w)[(size_t)n * K + k];
-        else w = (float)((static_cast<const uint8_t*>(g.w)[((size_t)n * K + k) >> 1] >> (4 * (k & 1))) & 15) - 8.0f;
+        else w = (float)((static_cast<const uint8_t*>(g.w)[((size_t)n * K + k) >> 1] >> (4 * (k & 1))) & 15);
+        if constexpr (FMT == XG_Q4) {
+            const size_t i = (size_t)n * a.gpr + k / a.group;
+            const float s = scale_at(g.gs, a.sdt, i);
+            w = g.gb ? w * s + scale_at(g.gb, a.sdt, i) : (w - 8.0f) * s;
+        } else if constexpr (FMT == XG_I4) {
+            w -= 8.0f;
+        }
         acc += w * xv;
     }
     return acc;
@@ -157,13 +184,19 @@ __device__ __forceinline__ float column_scale(const XgSeg& g, int sdt, int n)
     return g.s ? scale_at(g.s, sdt, (size_t)n * g.s_stride) : 1.0f;
 }
 
-template <int FMT, int P, int TA, int TB, int WM, int WN, int NST>
+// S16: XG_Q4's scales are 16 bits wide
+template <int FMT, bool S16, int P, int TA, int TB, int WM, int WN, int NST>
 __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgArgs a)
 {
     constexpr int NW = WM * WN, BM = 32 * TA * WM, BN = 32 * TB * WN, RB = Fmt<FMT>::kStepBytes;
-    constexpr int kXBytes = BM * P * 128, kWBytes = BN * RB, kStage = kXBytes + kWBytes;
+    constexpr bool GROUPED = FMT == XG_Q4;
+    // a stage: X parts, raw weights, and the step's group scales, group biases and sums of x'
+    constexpr int kXBytes = BM * P * 128, kWBytes = BN * RB, kGroupAt = kXBytes + kWBytes, kSumAt = kGroupAt + 8 * BN;
+    constexpr int kStage = stage_bytes(FMT, P, BM, BN, RB);
     constexpr int XD = kXBytes / 1024 / NW, WD = kWBytes / 1024 / NW;  // DMA loads per wave and step
-    constexpr int NDMA = XD + WD, LA = NST - 1;
+    constexpr int GD = GROUPED ? 2 * BN / 64 / NW : 0;                 // of 64 scales or biases
+    constexpr int NDMA = XD + WD + GD + (GROUPED ? 1 : 0), LA = NST - 1;
+    static_assert(!GROUPED || GD * NW * 64 == 2 * BN, "whole DMA loads per wave");
     static_assert(XD * NW * 1024 == kXBytes && WD * NW * 1024 == kWBytes, "whole DMA loads per wave");
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -201,6 +234,21 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
     }
     const unsigned char* xbase = reinterpret_cast<const unsigned char*>(a.xp) + (size_t)m0 * P * a.Kp * 2;
     const unsigned char* wbase = static_cast<const unsigned char*>(g.w) + (size_t)n0 * rbytes;
+    // scale and bias DMA: load j of a wave covers 64 columns of either (symmetric weights fetch their scales
+    // twice); x' sums: 64 rows per load, waves past the tile's rows repeat one
+    uint32_t goff[GROUPED ? GD : 1], soff = 0;
+    const unsigned char* gbase[GROUPED ? GD : 1];
+    constexpr int SB = S16 ? 2 : 4;
+    const int sum_at = (wave % (BM > 64 ? BM / 64 : 1)) * 64;
+    if constexpr (GROUPED) {
+#pragma unroll
+        for (int j = 0; j < GD; ++j) {
+            const int q = wave * GD + j, c = (q % (BN / 64)) * 64 + lane;
+            goff[j] = (uint32_t)min(c, g.n - 1 - n0) * (uint32_t)(a.gpr * SB);
+            gbase[j] = static_cast<const unsigned char*>(q < BN / 64 || !g.gb ? g.gs : g.gb) + (size_t)n0 * a.gpr * SB;
+        }
+        soff = (uint32_t)min(sum_at + lane, a.M - 1 - m0) * 4u;
+    }
     const uint32_t lds0 = lds_addr(smem);
     const bool ragged = tail_chunks < CPR;
     auto issue = [&](int s, int slot) {
@@ -216,6 +264,16 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
         } else {
 #pragma unroll
             for (int j = 0; j < WD; ++j) dma16_s(woff[j], ws, base + kXBytes + (wave * WD + j) * 1024);
+        }
+        if constexpr (GROUPED) {
+            const size_t gi = (size_t)(t * kBK / a.group) * SB;
+#pragma unroll
+            for (int j = 0; j < GD; ++j) {
+                const uint32_t to = base + kGroupAt + (wave * GD + j) * 256;
+                if constexpr (S16) dma2_s(goff[j], gbase[j] + gi, to);
+                else dma4_s(goff[j], gbase[j] + gi, to);
+            }
+            dma4_s(soff, a.xsum + (size_t)t * a.M + m0, base + kSumAt + sum_at * 4);
         }
     };
 #pragma unroll
@@ -275,6 +333,43 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
                     for (int j = 0; j < TB; ++j)
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i], b[j][ks], acc[i][j], 0, 0, 0);
             }
+        if constexpr (GROUPED) {
+            // w = q s + b = (q - 8) s + (b + 8 s): the step's sum of (q - 8) x' times s, plus (b + 8 s) times
+            // its sum of x'
+            const uint32_t* gs = reinterpret_cast<const uint32_t*>(xs + kGroupAt);
+            const f4_t* sums = reinterpret_cast<const f4_t*>(xs + kSumAt);
+            float sc[TB], bi[TB];
+#pragma unroll
+            for (int j = 0; j < TB; ++j) {
+                const int c = (wn * TB + j) * 32 + r32;
+                const uint32_t s = gs[c], b = gs[BN + c];
+                if constexpr (S16) {
+                    sc[j] = a.sdt == DT_F16 ? raw_to_f32<DT_F16>(s) : raw_to_f32<DT_BF16>(s);
+                    bi[j] = a.sdt == DT_F16 ? raw_to_f32<DT_F16>(b) : raw_to_f32<DT_BF16>(b);
+                } else {
+                    sc[j] = raw_to_f32<DT_F32>(s);
+                    bi[j] = raw_to_f32<DT_F32>(b);
+                }
+                bi[j] = g.gb ? __builtin_fmaf(8.0f, sc[j], bi[j]) : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < TA; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const f4_t xv = sums[(wm * TA + i) * 8 + q * 2 + h32];
+#pragma unroll
+                    for (int j = 0; j < TB; ++j)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c)
+                            sum[i][j][4 * q + c] = __builtin_fmaf(
+                                sc[j], acc[i][j][4 * q + c], __builtin_fmaf(bi[j], xv[c], sum[i][j][4 * q + c]));
+                }
+        } else {
+#pragma unroll
+            for (int i = 0; i < TA; ++i)
+#pragma unroll
+                for (int j = 0; j < TB; ++j) sum[i][j] += acc[i][j];
+        }
     };
     for (int s = 0; s < nsteps; ++s) {
 #pragma unroll
@@ -282,10 +377,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
 #pragma unroll
             for (int j = 0; j < TB; ++j) acc[i][j] = f16v_t{};
         step(s);
-#pragma unroll
-        for (int i = 0; i < TA; ++i)
-#pragma unroll
-            for (int j = 0; j < TB; ++j) sum[i][j] += acc[i][j];
     }
     wait_vmcnt<0>();  // the trailing (re-read) DMA, before the block's LDS is given back
 
@@ -338,7 +429,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
         const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3), n = n0 + (wn * TB + j) * 32 + r32;
         if (m >= a.M || n >= g.n || finite_f32(g.y[(size_t)m * g.n + n])) continue;
         g.y[(size_t)m * g.n + n] =
-            plain_dot<FMT, P>(g, a.x, m, n, a.K) * column_scale(g, a.sdt, n) + (g.bias ? g.bias[n] : 0.0f);
+            plain_dot<FMT, P>(a, g, m, n) * column_scale(g, a.sdt, n) + (g.bias ? g.bias[n] : 0.0f);
     }
 }
 
@@ -364,7 +455,7 @@ __global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a,
             const int nc = min(n + c, g.n - 1);
             const float sc = column_scale(g, a.sdt, nc), bi = g.bias ? g.bias[nc] : 0.0f;
             o[c] = (P == 2 ? ldexpf(v[c], e) : v[c]) * sc + bi;
-            if (!finite_f32(o[c])) o[c] = plain_dot<FMT, P>(g, a.x, m, nc, a.K) * sc + bi;
+            if (!finite_f32(o[c])) o[c] = plain_dot<FMT, P>(a, g, m, nc) * sc + bi;
         }
         if ((g.n & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
             *reinterpret_cast<f4_t*>(y) = o;
@@ -379,9 +470,10 @@ __global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a,
 // One block per row of x: its parts, zero-padded to Kp, and its exponent.  Eight elements per thread
 // and round; rows of up to 8192 stay in registers between the maximum and the split.
 constexpr int kSplitUnits = 4;
-template <bool PAIRS>
+template <bool PAIRS, bool SUMS>
 __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ x, int K, int Kp,
-                                                      _Float16* __restrict__ xp, int32_t* __restrict__ xe)
+                                                      _Float16* __restrict__ xp, int32_t* __restrict__ xe,
+                                                      float* __restrict__ xsum)
 {
     __shared__ float wmax[4];
     const int m = blockIdx.x, tid = threadIdx.x, units = Kp / 8;
@@ -425,6 +517,11 @@ __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ 
     _Float16* out = xp + (size_t)m * 2 * Kp;
     auto store = [&](int u, const f4_t (&d)[2]) {
         h8_t hi, lo;
+        if constexpr (SUMS) {  // eight threads hold a step's 64 (Kp / 8 is a multiple of 8, so all or none are here)
+            const f4_t q = d[0] + d[1];
+            const float sum = oct_sum(ldexpf((q[0] + q[1]) + (q[2] + q[3]), e));
+            if ((u & 7) == 0) xsum[(size_t)(u >> 3) * gridDim.x + m] = sum;
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int k = PAIRS ? (i >> 1) + 4 * (i & 1) : i;
@@ -450,16 +547,16 @@ __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ 
 // The tile forms: 0 = 32 rows x 128 columns (2 waves), 1 = 64 x 128 (4 waves), 2 = 128 x 256 (8 waves).
 struct XgPlan {
     int form, bm, bn, vtiles, steps_per_split, splits;
-    size_t part_off, bytes;  // workspace: exponents, parts, then the split sums
+    size_t xp_off, sum_off, part_off, bytes;  // workspace: exponents, parts, sums of x', split sums
 };
 
-XgPlan xg_plan(const int* n, int nseg, int M, int K)
+XgPlan xg_plan(int fmt, const XgSeg* segs, int nseg, int M, int K)
 {
     XgPlan p{};
     const int steps = (K + kBK - 1) / kBK;
     auto tiles = [&](int bm, int bn) {
         int t = 0;
-        for (int i = 0; i < nseg; ++i) t += (n[i] + bn - 1) / bn;
+        for (int i = 0; i < nseg; ++i) t += (segs[i].n + bn - 1) / bn;
         p.bm = bm, p.bn = bn, p.vtiles = t;
         return (int64_t)t * ((M + bm - 1) / bm);
     };
@@ -474,17 +571,19 @@ XgPlan xg_plan(const int* n, int nseg, int M, int K)
     while (blocks * splits * 2 <= want && steps / (splits * 2) >= 4) splits *= 2;
     p.steps_per_split = (steps + splits - 1) / splits;
     p.splits = (steps + p.steps_per_split - 1) / p.steps_per_split;
-    const size_t xe = ((size_t)M * 4 + 255) & ~(size_t)255;
-    p.part_off = xe + (((size_t)M * 2 * steps * kBK * 2 + 255) & ~(size_t)255);
+    const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    p.xp_off = up((size_t)M * 4);
+    p.sum_off = p.xp_off + up((size_t)M * 2 * steps * kBK * 2);
+    p.part_off = p.sum_off + (fmt == XG_Q4 ? up((size_t)M * steps * 4) : 0);
     p.bytes = p.part_off + (p.splits > 1 ? (size_t)p.splits * M * p.vtiles * p.bn * 4 : 0);
     return p;
 }
 
-template <int FMT, int P, int TA, int TB, int WM, int WN, int NST>
+template <int FMT, bool S16, int P, int TA, int TB, int WM, int WN, int NST>
 hipError_t launch_form(const XgArgs& a, const XgPlan& p, hipStream_t st)
 {
-    constexpr int lds = NST * (32 * TA * WM * P * 128 + 32 * TB * WN * Fmt<FMT>::kStepBytes);
-    auto kern = qgemm_exact_kernel<FMT, P, TA, TB, WM, WN, NST>;
+    constexpr int lds = NST * stage_bytes(FMT, P, 32 * TA * WM, 32 * TB * WN, Fmt<FMT>::kStepBytes);
+    auto kern = qgemm_exact_kernel<FMT, S16, P, TA, TB, WM, WN, NST>;
     if constexpr (lds > 64 * 1024) {
         const hipError_t e = allow_big_lds(kern, lds);
         if (e != hipSuccess) return e;
@@ -496,45 +595,52 @@ hipError_t launch_form(const XgArgs& a, const XgPlan& p, hipStream_t st)
 
 }  // namespace
 
-bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int M, int K, const void* x)
+bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int group, int M, int K, const void* x)
 {
-    // weight rows start on 16-byte boundaries
-    if (M < 5 || K <= 0 || K % (fmt == XG_I4 ? 32 : fmt == XG_I8 ? 16 : 8) != 0) return false;
-    // the kernels of single rows walk the rows one after the other, 1.2 (f16) to 3.2 ns (i4) per row and
-    // element of k, the f16 ones four rows at a time; the three launches here take 14-16 us.  int8: 5 rows
-    // of 960 -> 960 10.7 against 16.2 us, of 1536 -> 576 15.2 against 14.4; i4: 5 of 960 -> 960 16.0
-    // against 16.0, 8 24.4 against 15.3; f16: 8 of 960 -> 960 11.3 against 14.9, 5 of 1536 -> 960 12.1
-    // against 12.4, 12 of 960 -> 2560 21.2 against 14.9.  Long outputs cost the row kernels more (int8, 5
-    // rows of 960 -> 32768: 68 against 18.5)
-    const int64_t pays = fmt == XG_F16 ? 10000 : fmt == XG_I4 ? 5000 : 7000;
-    if ((int64_t)M * K < pays && segs[0].n < 8192) return false;
+    const bool nibbles = fmt == XG_I4 || fmt == XG_Q4;
+    // weight rows start on 16-byte boundaries; a K step has one scale
+    if (M < 5 || K <= 0 || K % (nibbles ? 32 : fmt == XG_I8 ? 16 : 8) != 0) return false;
+    if (fmt == XG_Q4 && (group <= 0 || group % kBK != 0)) return false;
+    // The kernels of single rows walk the rows one after the other (f16: four at a time), so they take
+    // longer with M K (a wave's walk) and with M K N (the whole work); the three launches here take 14-17
+    // us at small sizes.  Measured, row kernels against these (us, rows x outputs x k):
+    //   int8  5 x 960 x 960 10.7 / 16.2, 5 x 576 x 1536 15.2 / 14.4, 5 x 8192 x 960 22.8 / 17.4
+    //   i4    5 x 960 x 960 16.0 / 16.0, 8 x 960 x 960 24.4 / 15.3
+    //   f16   8 x 960 x 960 11.3 / 14.9, 12 x 2560 x 960 21.2 / 14.9, 5 x 8192 x 960 19.5 / 14.9
+    //   q4    16 x 2560 x 960 13.3 / 17.7, 24 x 1024 x 1024 14.6 / 13.3, 5 x 16384 x 960 17.5 / 17.4
+    const bool affine = fmt == XG_Q4 && segs[0].gb;
+    const int64_t walk = affine ? 24000 : fmt == XG_F16 ? 10000 : nibbles ? 5000 : 7000;
+    const double work = affine ? 78e6 : 35e6;
+    if ((int64_t)M * K < walk && (double)M * K * segs[0].n < work) return false;
     if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (M + 31) / 32 > 65535) return false;
     int64_t n = 0;
     for (int i = 0; i < nseg; ++i) {
         if (segs[i].n <= 0 || (reinterpret_cast<uintptr_t>(segs[i].w) & 15) != 0) return false;
+        // group scales and biases are fetched as whole elements
+        if (((reinterpret_cast<uintptr_t>(segs[i].gs) | reinterpret_cast<uintptr_t>(segs[i].gb)) & 3) != 0) return false;
         n += segs[i].n;
     }
     // a tile's byte offsets are 32-bit
     return (uint64_t)K * 1024 < (1ull << 31) && n < (1 << 30);
 }
 
-size_t qgemm_exact_workspace_bytes(const XgSeg* segs, int nseg, int M, int K)
+size_t qgemm_exact_workspace_bytes(int fmt, const XgSeg* segs, int nseg, int M, int K)
 {
-    const int n[3] = {segs[0].n, nseg > 1 ? segs[1].n : 0, nseg > 2 ? segs[2].n : 0};
-    return xg_plan(n, nseg, M, K).bytes;
+    return xg_plan(fmt, segs, nseg, M, K).bytes;
 }
 
-template <int FMT>
-static hipError_t launch_fmt(XgArgs& a, const XgPlan& p, const float* x, int32_t* xe, _Float16* xp, hipStream_t st)
+template <int FMT, bool S16>
+static hipError_t launch_fmt(const XgArgs& a, const XgPlan& p, int32_t* xe, _Float16* xp, float* xsum, hipStream_t st)
 {
-    hipLaunchKernelGGL((split_x_kernel<Fmt<FMT>::kPairs>), dim3(a.M), dim3(256), 0, st, x, a.K, a.Kp, xp, xe);
+    hipLaunchKernelGGL((split_x_kernel<Fmt<FMT>::kPairs, FMT == XG_Q4>), dim3(a.M), dim3(256), 0, st,
+                       static_cast<const float*>(a.x), a.K, a.Kp, xp, xe, xsum);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // f16 rows are twice the bytes: two stages keep two blocks (form 1) or one (form 2) on a CU
     constexpr int NST = FMT == XG_F16 ? 2 : 3;
-    e = p.form == 2   ? launch_form<FMT, 2, 2, 2, 2, 4, NST>(a, p, st)
-        : p.form == 1 ? launch_form<FMT, 2, 1, 2, 2, 2, NST>(a, p, st)
-                      : launch_form<FMT, 2, 1, 2, 1, 2, 3>(a, p, st);
+    e = p.form == 2   ? launch_form<FMT, S16, 2, 2, 2, 2, 4, NST>(a, p, st)
+        : p.form == 1 ? launch_form<FMT, S16, 2, 1, 2, 2, 2, NST>(a, p, st)
+                      : launch_form<FMT, S16, 2, 1, 2, 1, 2, 3>(a, p, st);
     if (e != hipSuccess || p.splits == 1) return e;
     const size_t quads = (size_t)a.M * a.vcols / 4;
     const unsigned blocks = (unsigned)std::min<size_t>((quads + 255) / 256, 4096);
@@ -542,23 +648,24 @@ static hipError_t launch_fmt(XgArgs& a, const XgPlan& p, const float* x, int32_t
     return hipGetLastError();
 }
 
-hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, const float* x, int M, int K, void* ws,
-                              hipStream_t st)
+hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, int group, int gpr, const float* x, int M,
+                              int K, void* ws, hipStream_t st)
 {
-    const int n[3] = {segs[0].n, nseg > 1 ? segs[1].n : 0, nseg > 2 ? segs[2].n : 0};
-    const XgPlan p = xg_plan(n, nseg, M, K);
+    const XgPlan p = xg_plan(fmt, segs, nseg, M, K);
     XgArgs a{};
     a.nseg = nseg;
     for (int i = 0, t = 0; i < nseg; ++i) {
         a.seg[i] = segs[i];
         a.tile0[i] = t;
-        t += (n[i] + p.bn - 1) / p.bn;
+        t += (segs[i].n + p.bn - 1) / p.bn;
     }
     unsigned char* base = static_cast<unsigned char*>(ws);
     int32_t* xe = reinterpret_cast<int32_t*>(base);
-    _Float16* xp = reinterpret_cast<_Float16*>(base + (((size_t)M * 4 + 255) & ~(size_t)255));
+    _Float16* xp = reinterpret_cast<_Float16*>(base + p.xp_off);
+    float* xsum = reinterpret_cast<float*>(base + p.sum_off);
     a.xe = xe;
     a.xp = xp;
+    a.xsum = xsum;
     a.x = x;
     a.part = p.splits > 1 ? reinterpret_cast<float*>(base + p.part_off) : nullptr;
     a.M = M;
@@ -567,10 +674,15 @@ hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, con
     a.steps_per_split = p.steps_per_split;
     a.vcols = p.vtiles * p.bn;
     a.sdt = sdt;
+    a.group = group;
+    a.gpr = gpr;
     switch (fmt) {
-        case XG_I8: return launch_fmt<XG_I8>(a, p, x, xe, xp, st);
-        case XG_I4: return launch_fmt<XG_I4>(a, p, x, xe, xp, st);
-        case XG_F16: return launch_fmt<XG_F16>(a, p, x, xe, xp, st);
+        case XG_I8: return launch_fmt<XG_I8, false>(a, p, xe, xp, xsum, st);
+        case XG_I4: return launch_fmt<XG_I4, false>(a, p, xe, xp, xsum, st);
+        case XG_F16: return launch_fmt<XG_F16, false>(a, p, xe, xp, xsum, st);
+        case XG_Q4:
+            return sdt == DT_F32 ? launch_fmt<XG_Q4, false>(a, p, xe, xp, xsum, st)
+                                 : launch_fmt<XG_Q4, true>(a, p, xe, xp, xsum, st);
         default: return hipErrorInvalidValue;
     }
 }

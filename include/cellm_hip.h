@@ -124,7 +124,7 @@ int32_t cellm_hip_weight_cache_stats(cellm_hip_ctx_t* ctx, size_t* out_entries, 
  * over k are exact and the row scale follows them, so x keeps 2^-20 of its
  * row's largest |x| (within 3e-5 normwise of the f32 reference order).  f32 x
  * at 5 rows and more (k % 16 == 0, 16-byte aligned w and x, m * k >= 7000 or
- * n >= 8192) runs on f16 MFMA over two f16 parts of each x, 2^-23 of every
+ * m * n * k >= 35e6) runs on f16 MFMA over two f16 parts of each x, 2^-23 of every
  * element, with the parts and split sums in the context's per-stream workspace;
  * under graph capture, or without memory for it, such calls take the kernels
  * that need none. */
@@ -150,7 +150,10 @@ int32_t cellm_hip_qgemv_i8(cellm_hip_ctx_t* ctx, const int8_t* w, const void* sc
  * aligned wq and x: the affine lm_head) run on int8 MFMA instead: each row
  * is rounded to integers x' = rint(x * 2^e) with |x'| <= 2^20 for the row's
  * largest |x|, split into three signed 8-bit digits, and summed exactly per
- * group; x keeps 2^-20 of its row's largest value, scaled back exactly. */
+ * group; x keeps 2^-20 of its row's largest value, scaled back exactly.  f32 x
+ * at 5 rows and more (k % 32 == 0, group >= 64, 16-byte aligned wq and x,
+ * m * k >= 24000 or m * n * k >= 78e6) runs on MFMA as in cellm_hip_qgemv_i8:
+ * exact nibbles over two f16 parts of x, scale and bias folded per 64 k in f32. */
 int32_t cellm_hip_qgemv_q4_affine(cellm_hip_ctx_t* ctx, const uint32_t* wq, const void* scales, const void* biases,
                                   int32_t sb_dtype, int64_t group, const void* x, int32_t x_dtype, float* y,
                                   int64_t m, int64_t n, int64_t k, void* stream);
@@ -273,8 +276,8 @@ int32_t cellm_hip_qgemv_batch(cellm_hip_ctx_t* ctx, const cellm_hip_qgemv_op_t* 
 
 /* Symmetric i4 GEMV: y[i, r] = sum_j ((nib - 8) * scale[r*spr + j/gs]) * x[i, j],
  * spr = n_scales / n.  f32 x at 5 rows and more with one scale per row (gs >= k)
- * runs on MFMA as in cellm_hip_qgemv_i8 (k % 32 == 0, 16-byte aligned w and x,
- * m * k >= 5000 or n >= 8192).  Replaces cpu_kernels::matmul_i4_f32 (cpu_kernels.rs:219-243)
+ * or gs a multiple of 64 runs on MFMA as in cellm_hip_qgemv_i8 (k % 32 == 0,
+ * 16-byte aligned w and x, m * k >= 5000 or m * n * k >= 35e6).  Replaces cpu_kernels::matmul_i4_f32 (cpu_kernels.rs:219-243)
  * and MetalOps::encode_mv_i4 (metal.rs:1167-1176). */
 int32_t cellm_hip_qgemv_i4_sym(cellm_hip_ctx_t* ctx, const uint8_t* w, const uint16_t* scales_f16, int64_t n_scales,
                                int64_t gs, const void* x, int32_t x_dtype, float* y, int64_t m, int64_t n, int64_t k,
@@ -283,7 +286,7 @@ int32_t cellm_hip_qgemv_i4_sym(cellm_hip_ctx_t* ctx, const uint8_t* w, const uin
 /* f16-weight GEMV: y[i, r] = sum_j f32(W[r, j]) * x[i, j], W [n][k] f16
  * (2-byte aligned).  f32 x at 5 rows and more runs on MFMA as in
  * cellm_hip_qgemv_i8 (k % 8 == 0, 16-byte aligned w and x, m * k >= 10000 or
- * n >= 8192).  Replaces cpu_kernels::matmul_f16_f32
+ * m * n * k >= 35e6).  Replaces cpu_kernels::matmul_f16_f32
  * (cpu_kernels.rs:135-214) in the runners' "f16" linear arms (qwen.rs:1073,
  * llama.rs:898) and MetalOps::encode_mv_f16 / mv_f16 (metal.rs:347-363,
  * 1089). */

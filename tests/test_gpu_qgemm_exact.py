@@ -35,7 +35,7 @@ def _rel(got, ref):
 
 # edges of the 32 / 64 / 128-row and 128 / 256-column tiles, K not a multiple of 64 and of one step,
 # split and unsplit K, the forms of xg_plan (small, middle, wide)
-SIZES = [(440, 16, 16), (110, 1, 64), (5, 8200, 48), (5, 33, 1408), (31, 127, 80), (32, 128, 128), (33, 129, 960), (64, 257, 2560), (65, 384, 1056),
+SIZES = [(440, 16, 16), (110, 1, 64), (5, 150000, 48), (5, 33, 1408), (6, 70, 4096), (31, 127, 80), (32, 128, 128), (33, 129, 960), (64, 257, 2560), (65, 384, 1056),
          (77, 40, 4864), (200, 1000, 1024), (512, 960, 960), (513, 4100, 208), (1030, 6000, 320)]
 
 
@@ -65,6 +65,58 @@ def test_i4_f32_rows(ops, m, n, k, spr):
     ops.encode_qgemv_i4_sym(w.cuda(), s.cuda(), k, x.cuda(), y, k)
     torch.cuda.synchronize()
     assert _rel(y.cpu(), x.double() @ q.t() * s[:, 0].double()) <= TOL
+
+
+@pytest.mark.parametrize("m,n,k", [s for s in SIZES if s[2] % 32 == 0])
+@pytest.mark.parametrize("sdt,group", [(torch.float32, 64), (torch.float16, 64), (torch.bfloat16, 64),
+                                       (torch.float32, 128), (torch.float16, 256)])
+def test_q4_affine_f32_rows(ops, m, n, k, sdt, group):
+    """Group scales and biases in each dtype, groups of one and of several K steps, a last group cut short."""
+    g = torch.Generator().manual_seed(m + n + k)
+    w = torch.randint(-2**31, 2**31, (n, k // 8), generator=g, dtype=torch.int64).to(torch.int32)
+    s = (torch.rand(n, -(-k // group), generator=g) * 0.01 + 1e-3).to(sdt)
+    b = (s.float() * (-7.5 + torch.randn(s.shape, generator=g))).to(sdt)
+    q = ((w[:, :, None] >> torch.arange(0, 32, 4)) & 15).reshape(n, k).double()
+    wide = lambda t: t.double().repeat_interleave(group, 1)[:, :k]
+    x = _x(m, k, m + k)
+    y = torch.full((m, n), float("nan"), device="cuda")
+    ops.encode_qgemv_q4_affine(w.cuda(), s.cuda(), b.cuda(), x.cuda(), y, group=group)
+    torch.cuda.synchronize()
+    assert _rel(y.cpu(), x.double() @ (q * wide(s) + wide(b)).t()) <= TOL
+
+
+@pytest.mark.parametrize("m,n,k,gs", [(40, 130, 192, 64), (65, 257, 1056, 192), (300, 384, 2560, 640)])
+def test_i4_grouped_f32_rows(ops, m, n, k, gs):
+    g = torch.Generator().manual_seed(m + n + k)
+    w = torch.randint(0, 256, (n, k // 2), generator=g, dtype=torch.uint8)
+    s = (torch.rand(n, -(-k // gs), generator=g) * 0.01 + 1e-3).half()
+    q = torch.stack([w & 15, w >> 4], 2).reshape(n, k).double() - 8
+    x = _x(m, k, m + k)
+    y = torch.full((m, n), float("nan"), device="cuda")
+    ops.encode_qgemv_i4_sym(w.cuda(), s.cuda(), gs, x.cuda(), y, k)
+    torch.cuda.synchronize()
+    assert _rel(y.cpu(), x.double() @ (q * s.double().repeat_interleave(gs, 1)[:, :k]).t()) <= TOL
+
+
+def test_q4_affine_non_finite(ops):
+    """inf and NaN in x, in a group's scale and in its bias reach the outputs of a plain f32 sum."""
+    m, n, k = 100, 96, 256
+    g = torch.Generator().manual_seed(1)
+    w = torch.randint(-2**31, 2**31, (n, k // 8), generator=g, dtype=torch.int64).to(torch.int32)
+    s, b = torch.rand(n, 4, generator=g) * 0.01 + 1e-3, torch.randn(n, 4, generator=g) * 0.01
+    s[5, 1], b[6, 2], b[7, 0] = float("inf"), float("-inf"), float("nan")
+    x = _x(m, k, 2)
+    x[3, 77], x[4, 200] = float("inf"), float("nan")
+    q = ((w[:, :, None] >> torch.arange(0, 32, 4)) & 15).reshape(n, k).float()
+    ref = x @ (q * s.repeat_interleave(64, 1) + b.repeat_interleave(64, 1)).t()
+    y = torch.empty(m, n, device="cuda")
+    ops.encode_qgemv_q4_affine(w.cuda(), s.cuda(), b.cuda(), x.cuda(), y)
+    torch.cuda.synchronize()
+    got = y.cpu()
+    assert np.array_equal(torch.isnan(got).numpy(), torch.isnan(ref).numpy())
+    assert np.array_equal(torch.isposinf(got).numpy(), torch.isposinf(ref).numpy())
+    fine = torch.isfinite(ref)
+    assert _rel(got[fine], ref[fine]) <= TOL
 
 
 @pytest.mark.parametrize("m,n,k", SIZES + [(300, 70, 8), (64, 130, 904)])
