@@ -234,24 +234,23 @@ bool capturing(hipStream_t st)
     return status != hipStreamCaptureStatusNone;
 }
 
-// The multi-row GEMM over f32 x (qgemm_exact.hip) where it applies: *done tells whether it was enqueued.
-// It needs scratch for x's parts, which the one-wave-per-row kernels do without, so a call that cannot
-// have it (captures, no memory) is left to them.
-int32_t try_qgemm_exact(cellm_hip_ctx* ctx, int fmt, const XgSeg* segs, int nseg, int32_t sdt, int64_t group,
-                        int64_t gpr, const void* x, int64_t m, int64_t k, hipStream_t st, bool* done)
+// The multi-row GEMM (qgemm_exact.hip) where it applies: *done tells whether it was enqueued.  It needs
+// scratch for x's parts, which the one-wave-per-row kernels do without, so a call that cannot have it
+// (captures, no memory) is left to them.
+int32_t try_qgemm_exact(cellm_hip_ctx* ctx, const XgCall& c, int64_t m, int64_t k, hipStream_t st, bool* done)
 {
     *done = false;
-    if (!qgemm_exact_supported(fmt, segs, nseg, (int)group, (int)m, (int)k, x) || capturing(st)) return CELLM_HIP_OK;
+    if (!qgemm_exact_supported(c, (int)m, (int)k)) return CELLM_HIP_OK;
+    const size_t need = qgemm_exact_workspace_bytes(c, (int)m, (int)k);
+    if (need && capturing(st)) return CELLM_HIP_OK;
     float* ws = nullptr;
-    const int32_t rc = get_workspace(ctx, st, qgemm_exact_workspace_bytes(fmt, segs, nseg, (int)m, (int)k), &ws);
+    const int32_t rc = get_workspace(ctx, st, need, &ws);
     if (rc == CELLM_HIP_ERR_OUT_OF_MEMORY) {
         (void)hipGetLastError();
         return CELLM_HIP_OK;
     }
     if (rc) return rc;
-    HIP_TRY(launch_qgemm_exact(fmt, segs, nseg, sdt, (int)group, (int)gpr, static_cast<const float*>(x), (int)m,
-                               (int)k, ws, st),
-            "qgemm_exact launch");
+    HIP_TRY(launch_qgemm_exact(c, (int)m, (int)k, ws, st), "qgemm_exact launch");
     *done = true;
     return CELLM_HIP_OK;
 }
@@ -302,7 +301,8 @@ int32_t qgemv_i8_impl(cellm_hip_ctx* ctx, const int8_t* w, const void* scales, i
     if (xdt == DT_F32) {
         const XgSeg seg{w, scales, bias, y, (int)n, per_channel, nullptr, nullptr};
         bool done = false;
-        if (int32_t rc = try_qgemm_exact(ctx, XG_I8, &seg, 1, sdt, 0, 0, x, m, k, st, &done)) return rc;
+        const XgCall call{XG_I8, &seg, 1, sdt, x, false, -1, 0, 0};
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;
     }
     HIP_TRY(launch_qgemv_i8(w, scales, sdt, per_channel, x, xdt, bias, y, (int)m, (int)n, (int)k, st, k == 0),
@@ -332,7 +332,8 @@ int32_t qgemv_lowbit_impl(cellm_hip_ctx* ctx, int fmt, const void* w, const uint
     if (fmt == LB_F16 && xdt == DT_F32) {
         const XgSeg seg{w, nullptr, nullptr, y, (int)n, 0, nullptr, nullptr};
         bool done = false;
-        if (int32_t rc = try_qgemm_exact(ctx, XG_F16, &seg, 1, DT_F32, 0, 0, x, m, k, st, &done)) return rc;
+        const XgCall call{XG_F16, &seg, 1, DT_F32, x, false, -1, 0, 0};
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;
     }
     HIP_TRY(launch_qgemv_lowbit(fmt, w, scales_f16, scale_mode, x, xdt, y, (int)m, (int)n, (int)k, st),
@@ -404,8 +405,8 @@ int32_t qgemv_q4_impl(cellm_hip_ctx* ctx, const uint32_t* wq, const void* scales
     if (xdt == DT_F32) {
         const XgSeg seg{wq, nullptr, nullptr, y, (int)n, 0, scales, biases};
         bool done = false;
-        if (int32_t rc = try_qgemm_exact(ctx, XG_Q4, &seg, 1, sbt, group, (k + group - 1) / group, x, m, k, st, &done))
-            return rc;
+        const XgCall call{XG_Q4, &seg, 1, sbt, x, false, -1, (int)group, (int)((k + group - 1) / group)};
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;
     }
     HIP_TRY(launch_qgemv_q4_affine(wq, scales, biases, sbt, (int)group, x, xdt, y, (int)m, (int)n, (int)k, st, k == 0),
@@ -436,6 +437,16 @@ int32_t qkv_i8_impl(cellm_hip_ctx* ctx, const int8_t* const w[3], const void* co
         HIP_TRY(launch_qgemv_i8_fused(segs, 3, false, ACT_SILU, sdt, x, xdt, (int)m, (int)k, st), "qgemv_i8_qkv launch");
         return CELLM_HIP_OK;
     }
+    // many f32 rows: x split once for the three
+    if (xdt == DT_F32) {
+        XgSeg xs[3];
+        for (int i = 0; i < 3; ++i)
+            xs[i] = XgSeg{w[i], s[i], b[i], y[i], (int)rows[i], n_s[i] >= rows[i] ? 1 : 0, nullptr, nullptr};
+        const XgCall call{XG_I8, xs, 3, sdt, x, false, -1, 0, 0};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
+        if (done) return CELLM_HIP_OK;
+    }
     for (int i = 0; i < 3; ++i)
         if (rows[i] > 0)
             if (int32_t rc = qgemv_i8_impl(ctx, w[i], s[i], sdt, n_s[i], x, xdt, b[i], y[i], m, rows[i], k, st, false))
@@ -458,6 +469,14 @@ int32_t gate_up_i8_impl(cellm_hip_ctx* ctx, const int8_t* wg, const void* sg, in
     if (k > 0 && qgemv_i8_fused_supported(xdt, (int)m, (int)k, x, segs, 2)) {
         HIP_TRY(launch_qgemv_i8_fused(segs, 2, true, act, sdt, x, xdt, (int)m, (int)k, st), "qgemv_i8 gate/up launch");
         return CELLM_HIP_OK;
+    }
+    if (xdt == DT_F32) {
+        const XgSeg xs[2] = {XgSeg{wg, sg, bg, h, (int)n, n_sg >= n ? 1 : 0, nullptr, nullptr},
+                             XgSeg{wu, su, bu, nullptr, (int)n, n_su >= n ? 1 : 0, nullptr, nullptr}};
+        const XgCall call{XG_I8, xs, 2, sdt, x, false, act, 0, 0};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
+        if (done) return CELLM_HIP_OK;
     }
     float* up = nullptr;
     if (int32_t rc = get_stream_buffer(ctx, ctx->aux, st, (size_t)m * n * sizeof(float), &up)) return rc;
@@ -483,6 +502,14 @@ int32_t gate_up_q4_impl(cellm_hip_ctx* ctx, const uint32_t* wg, const void* sg, 
                                              act, st),
                 "qgemv_q4 gate/up launch");
         return CELLM_HIP_OK;
+    }
+    if (xdt == DT_F32) {
+        const XgSeg xs[2] = {XgSeg{wg, nullptr, nullptr, h, (int)n, 0, sg, bg},
+                             XgSeg{wu, nullptr, nullptr, nullptr, (int)n, 0, su, bu}};
+        const XgCall call{XG_Q4, xs, 2, sbt, x, false, act, (int)group, (int)((k + group - 1) / group)};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
+        if (done) return CELLM_HIP_OK;
     }
     float* up = nullptr;
     if (int32_t rc = get_stream_buffer(ctx, ctx->aux, st, (size_t)m * n * sizeof(float), &up)) return rc;
@@ -835,6 +862,14 @@ int32_t cellm_hip_qgemv_q4_affine_qkv(cellm_hip_ctx_t* ctx, const uint32_t* wq, 
                 "qgemv_q4_qkv launch");
         return CELLM_HIP_OK;
     }
+    if (x_dtype == DT_F32) {
+        XgSeg xs[3];
+        for (int i = 0; i < 3; ++i) xs[i] = XgSeg{w[i], nullptr, pb[i], y[i], (int)rows[i], 0, s[i], b[i]};
+        const XgCall call{XG_Q4, xs, 3, sb_dtype, x, false, -1, (int)group, (int)((cols + group - 1) / group)};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, cols, st, &done)) return rc;
+        if (done) return CELLM_HIP_OK;
+    }
     // other shapes: one GEMV per projection, then its bias
     for (int i = 0; i < 3; ++i) {
         if (rows[i] == 0) continue;
@@ -903,6 +938,13 @@ int32_t cellm_hip_qgemv_q4_affine_gate_up_gelu(cellm_hip_ctx_t* ctx, const uint3
     CELLM_API_END(report_exception)
 }
 
+// One symmetric i4 matrix for the multi-row GEMM: a scale per row (the row's last element still uses its
+// first scale) follows the sum, group scales go with the K steps.
+static XgSeg i4_seg(const uint8_t* w, const uint16_t* scales_f16, int64_t spr, bool per_row, float* y, int64_t n)
+{
+    return XgSeg{w, per_row ? scales_f16 : nullptr, nullptr, y, (int)n, (int)spr, per_row ? nullptr : scales_f16, nullptr};
+}
+
 static int32_t qgemv_i4_impl(cellm_hip_ctx* ctx, const uint8_t* w, const uint16_t* scales_f16, int64_t n_scales, int64_t gs,
                              const void* x, int32_t x_dtype, float* y, int64_t m, int64_t n, int64_t k, hipStream_t st)
 {
@@ -917,12 +959,11 @@ static int32_t qgemv_i4_impl(cellm_hip_ctx* ctx, const uint8_t* w, const uint16_
                          (long long)((k - 1) / gs), (long long)spr);
     if ((k > 0 && (!w || !scales_f16 || !x)) || !y) return set_error(CELLM_HIP_ERR_INVALID_ARG, "null pointer");
     if (x_dtype == DT_F32 && k > 0 && spr <= INT32_MAX && gs <= INT32_MAX) {
-        const bool per_row = (k - 1) / gs == 0;  // the row's last element still uses its first scale
-        const XgSeg seg{w,      per_row ? scales_f16 : nullptr, nullptr, y, (int)n, (int)spr,
-                        per_row ? nullptr : scales_f16, nullptr};
+        const bool per_row = (k - 1) / gs == 0;
+        const XgSeg seg = i4_seg(w, scales_f16, spr, per_row, y, n);
+        const XgCall call{per_row ? XG_I4 : XG_Q4, &seg, 1, DT_F16, x, false, -1, (int)gs, (int)spr};
         bool done = false;
-        if (int32_t rc = try_qgemm_exact(ctx, per_row ? XG_I4 : XG_Q4, &seg, 1, DT_F16, gs, spr, x, m, k, st, &done))
-            return rc;
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;
     }
     HIP_TRY(launch_qgemv_i4_sym(w, scales_f16, (int)spr, (int)gs, x, x_dtype, y, (int)m, (int)n, (int)k, st),
@@ -945,6 +986,16 @@ int32_t cellm_hip_qgemv_i4_gate_up_gelu(cellm_hip_ctx_t* ctx, const uint8_t* wg,
     DeviceGuard g(ctx->device);
     const std::lock_guard<std::recursive_mutex> lk(ctx->mu);  // held until the scratch users are enqueued
     hipStream_t st = pick_stream(ctx, stream);
+    const int64_t spr = n_sg / n;
+    if (x_dtype == DT_F32 && k > 0 && gs >= 1 && spr >= 1 && n_su / n == spr && (k - 1) / gs < spr && wg && sg && wu && su &&
+        x && spr <= INT32_MAX && gs <= INT32_MAX) {
+        const bool per_row = (k - 1) / gs == 0;
+        const XgSeg xs[2] = {i4_seg(wg, sg, spr, per_row, h, n), i4_seg(wu, su, spr, per_row, nullptr, n)};
+        const XgCall call{per_row ? XG_I4 : XG_Q4, xs, 2, DT_F16, x, false, ACT_GELU_TANH, (int)gs, (int)spr};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
+        if (done) return CELLM_HIP_OK;
+    }
     float* up = nullptr;
     if (int32_t rc = get_stream_buffer(ctx, ctx->aux, st, (size_t)m * n * sizeof(float), &up)) return rc;
     if (int32_t rc = qgemv_i4_impl(ctx, wg, sg, n_sg, gs, x, x_dtype, h, m, n, k, st)) return rc;

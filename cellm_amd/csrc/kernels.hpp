@@ -99,11 +99,19 @@ struct XgSeg {
     const void* gs;    // XG_Q4: group scales of dtype sdt [n][gpr], and group biases: w = q gs + gb, or
     const void* gb;    // nullptr: w = (q - 8) gs
 };
-// group, gpr: XG_Q4's elements per scale (a multiple of 64) and scales per row.
-bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int group, int M, int K, const void* x);
-size_t qgemm_exact_workspace_bytes(int fmt, const XgSeg* segs, int nseg, int M, int K);
-hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, int group, int gpr, const float* x, int M,
-                              int K, void* ws, hipStream_t st);
+struct XgCall {
+    int fmt;
+    const XgSeg* segs;
+    int nseg;
+    int sdt;
+    const void* x;      // [M][K] f32, or f16 (int8 weights only)
+    bool x_f16;
+    int act;            // -1, or ACT_*: y of seg 0 = act(seg 0) * seg 1
+    int group, gpr;     // XG_Q4: elements per scale (a multiple of 64) and scales per row
+};
+bool qgemm_exact_supported(const XgCall& c, int M, int K);
+size_t qgemm_exact_workspace_bytes(const XgCall& c, int M, int K);
+hipError_t launch_qgemm_exact(const XgCall& c, int M, int K, void* ws, hipStream_t st);
 
 // Batched decode on MFMA (2 <= M <= 64, f16 x): int8 needs K % 64 == 0 and
 // K >= 128, q4 K % 128 == 0, K >= 256 and group >= 32; 16-byte aligned W and x;

@@ -10,7 +10,7 @@
 //
 // Group-scaled nibbles (w = q s + b or (q - 8) s, one scale per 64 k or a multiple)
 // multiply as the exact q - 8: every K step's sum is folded as
-// sum += s acc + (b + 8 s) sum(x'), the sums of x' coming from the split kernel and
+// s acc + (b + 8 s) sum(x'), the sums of x' coming from the split kernel and
 // the step's scales and biases with the weights through the DMA ring.  With q - 8
 // in place of q the step's two terms do not cancel (b is near -7.5 s).
 //
@@ -23,10 +23,12 @@
 // rounds its f32 accumulator once per 8 or 16 products, so a chain over the whole
 // K carries more rounding error than the tree sums of the one-wave-per-row
 // kernels: accumulators run over one K step (64 k), low parts before high ones,
-// and are then added to a second set.  Error against 64 bits at 512 rows, K = 960
-// / 2560 / 4096: 8.6e-8 / 1.0e-7 / 1.3e-7 with a sum per step, 9.7e-8 / 1.1e-7 /
-// 1.2e-7 per two steps, 1.3e-7 / 1.4e-7 / 1.4e-7 per four, 9.7e-8 / 1.3e-7 /
-// 1.7e-7 in the one-wave-per-row kernels; a sum per step costs 1-4 % in time.
+// the sums of two steps are added and then join the total.  Error against 64 bits,
+// int8 at 512 rows, K = 960 / 2560 / 4096 / 8192: 8.4e-8 / 1.0e-7 / 1.1e-7 / 1.2e-7
+// (each step added to the total by itself 8.6e-8 / 1.0e-7 / 1.3e-7 / 1.3e-7, chains
+// over two steps 9.7e-8 / 1.1e-7 / 1.2e-7, over four 1.3e-7 / 1.4e-7 / 1.4e-7, the
+// one-wave-per-row kernels 9.7e-8 / 1.3e-7 / 1.7e-7 / 2.1e-7); against chains over
+// four steps this costs 4-5 % of the wide shapes' time.
 // Results that are not finite (an infinity or NaN in x or w, or an overflow: the
 // split turns inf into inf * lo) are recomputed by a plain f32 sum.
 //
@@ -34,7 +36,7 @@
 // split of x): 960 -> 960 1963 -> 20, 2560 -> 960 5098 -> 25, 4096 -> 4096
 // 8034 -> 60; 16 rows of 1152 -> 1536 35 -> 15; 2048 rows of 2048 -> 8192 164,
 // 839 TFLOP/s of MFMA work; 16 rows of 2560 -> 960, i4 109 -> 14, f16 63 -> 14; MLX
-// q4 with f32 scales, 512 rows of 4096 -> 4096, 1480 -> 66 (error 1.6e-7, as before).  The small ones are bound by three dependent launches
+// q4 with f32 scales, 512 rows of 4096 -> 4096, 1480 -> 67 (error 1.6e-7 -> 1.1e-7).  The small ones are bound by three dependent launches
 // and the latency of a few K steps, the wide ones by the MFMAs.
 //
 // Tile: WM x WN waves of (32 TA) x (32 TB); X parts and raw weights go
@@ -74,6 +76,7 @@ struct XgArgs {
     int vcols;            // column tiles * BN
     int sdt;
     int group, gpr;       // XG_Q4: elements per scale, scales per row
+    int act;              // ACT: h = act(seg 0) * seg 1, written to seg 0's y
 };
 
 template <int FMT>
@@ -184,12 +187,22 @@ __device__ __forceinline__ float column_scale(const XgSeg& g, int sdt, int n)
     return g.s ? scale_at(g.s, sdt, (size_t)n * g.s_stride) : 1.0f;
 }
 
-// S16: XG_Q4's scales are 16 bits wide
-template <int FMT, bool S16, int P, int TA, int TB, int WM, int WN, int NST>
+template <int FMT, int P, bool ACT>
+__device__ __forceinline__ float plain_output(const XgArgs& a, const XgSeg& g, const XgSeg& gu, int m, int n)
+{
+    const float v = plain_dot<FMT, P>(a, g, m, n) * column_scale(g, a.sdt, n) + (g.bias ? g.bias[n] : 0.0f);
+    if constexpr (!ACT) return v;
+    return act_mul(a.act, v, plain_dot<FMT, P>(a, gu, m, n) * column_scale(gu, a.sdt, n) + (gu.bias ? gu.bias[n] : 0.0f));
+}
+
+// S16: XG_Q4's scales are 16 bits wide.  ACT: segments 0 and 1 are gate and up; each wave's 64 columns are 32
+// gate columns and the same 32 up columns, so both sums of an output end in one lane.
+template <int FMT, bool S16, int P, int TA, int TB, int WM, int WN, int NST, bool ACT>
 __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgArgs a)
 {
     constexpr int NW = WM * WN, BM = 32 * TA * WM, BN = 32 * TB * WN, RB = Fmt<FMT>::kStepBytes;
-    constexpr bool GROUPED = FMT == XG_Q4;
+    constexpr bool GROUPED = FMT == XG_Q4, FOLD = P == 2 || GROUPED;
+    static_assert(!ACT || TB == 2, "a gate and an up tile per wave");
     // a stage: X parts, raw weights, and the step's group scales, group biases and sums of x'
     constexpr int kXBytes = BM * P * 128, kWBytes = BN * RB, kGroupAt = kXBytes + kWBytes, kSumAt = kGroupAt + 8 * BN;
     constexpr int kStage = stage_bytes(FMT, P, BM, BN, RB);
@@ -205,9 +218,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
     const int step0 = blockIdx.z * a.steps_per_split, total = a.Kp / kBK;
     const int nsteps = min(a.steps_per_split, total - step0);
     if (nsteps <= 0) return;  // the launcher makes no empty split
-    const int si = (a.nseg > 1 && vt >= a.tile0[1]) + (a.nseg > 2 && vt >= a.tile0[2]);
+    const int si = ACT ? 0 : (a.nseg > 1 && vt >= a.tile0[1]) + (a.nseg > 2 && vt >= a.tile0[2]);
     const XgSeg g = a.seg[si];
-    const int n0 = (vt - a.tile0[si]) * BN;
+    const XgSeg gu = ACT ? a.seg[1] : g;
+    const int n0 = (vt - a.tile0[si]) * (ACT ? BN / 2 : BN);
     const size_t rbytes = row_bytes<FMT>(a.K);
 
     // X DMA: load j of a wave covers 8 part rows (128 bytes each); part row p BM + i is part p of row
@@ -223,17 +237,20 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
     // past the row's end re-read its last one (they meet the zeros that pad X)
     constexpr int RPD = 1024 / RB, CPR = RB / 16;
     uint32_t woff[WD], woff_tail[WD];
+    const unsigned char* wbase[WD];
     const int tail_chunks = (int)(rbytes - (size_t)(total - 1) * RB) / 16;
 #pragma unroll
     for (int j = 0; j < WD; ++j) {
         const int r = (wave * WD + j) * RPD + lane / CPR;
         const int c = swz<RB>(r, lane % CPR);
-        const uint32_t row = (uint32_t)min(r, g.n - 1 - n0) * (uint32_t)rbytes;
+        // a load's rows lie in one 32-row slice: for ACT, slices alternate between gate and up
+        const int slice = (wave * WD + j) * RPD / 32, col = ACT ? (slice >> 1) * 32 + (r & 31) : r;
+        wbase[j] = static_cast<const unsigned char*>(ACT && (slice & 1) ? gu.w : g.w) + (size_t)n0 * rbytes;
+        const uint32_t row = (uint32_t)min(col, g.n - 1 - n0) * (uint32_t)rbytes;
         woff[j] = row + 16 * c;
         woff_tail[j] = row + 16 * min(c, tail_chunks - 1);
     }
     const unsigned char* xbase = reinterpret_cast<const unsigned char*>(a.xp) + (size_t)m0 * P * a.Kp * 2;
-    const unsigned char* wbase = static_cast<const unsigned char*>(g.w) + (size_t)n0 * rbytes;
     // scale and bias DMA: load j of a wave covers 64 columns of either (symmetric weights fetch their scales
     // twice); x' sums: 64 rows per load, waves past the tile's rows repeat one
     uint32_t goff[GROUPED ? GD : 1], soff = 0;
@@ -243,9 +260,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
     if constexpr (GROUPED) {
 #pragma unroll
         for (int j = 0; j < GD; ++j) {
-            const int q = wave * GD + j, c = (q % (BN / 64)) * 64 + lane;
+            // ACT: the gate columns' scales, then the up columns', the same for the biases
+            constexpr int PER = ACT ? BN / 128 : BN / 64;
+            const int q = wave * GD + j, c = (q % PER) * 64 + lane;
+            const XgSeg& h = ACT && (q / PER & 1) ? gu : g;
             goff[j] = (uint32_t)min(c, g.n - 1 - n0) * (uint32_t)(a.gpr * SB);
-            gbase[j] = static_cast<const unsigned char*>(q < BN / 64 || !g.gb ? g.gs : g.gb) + (size_t)n0 * a.gpr * SB;
+            gbase[j] = static_cast<const unsigned char*>(q < BN / 64 || !h.gb ? h.gs : h.gb) + (size_t)n0 * a.gpr * SB;
         }
         soff = (uint32_t)min(sum_at + lane, a.M - 1 - m0) * 4u;
     }
@@ -255,15 +275,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
         const int t = step0 + min(s, nsteps - 1);
         const uint32_t base = lds0 + slot * kStage;
         const unsigned char* xs = xbase + (size_t)t * 128;
-        const unsigned char* ws = wbase + (size_t)t * RB;
+        const size_t wt = (size_t)t * RB;
 #pragma unroll
         for (int j = 0; j < XD; ++j) dma16_s(xoff[j], xs, base + (wave * XD + j) * 1024);
         if (ragged && t == total - 1) {
 #pragma unroll
-            for (int j = 0; j < WD; ++j) dma16_s(woff_tail[j], ws, base + kXBytes + (wave * WD + j) * 1024);
+            for (int j = 0; j < WD; ++j) dma16_s(woff_tail[j], wbase[j] + wt, base + kXBytes + (wave * WD + j) * 1024);
         } else {
 #pragma unroll
-            for (int j = 0; j < WD; ++j) dma16_s(woff[j], ws, base + kXBytes + (wave * WD + j) * 1024);
+            for (int j = 0; j < WD; ++j) dma16_s(woff[j], wbase[j] + wt, base + kXBytes + (wave * WD + j) * 1024);
         }
         if constexpr (GROUPED) {
             const size_t gi = (size_t)(t * kBK / a.group) * SB;
@@ -279,14 +299,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
 #pragma unroll
     for (int j = 0; j < LA; ++j) issue(j, j);
 
-    f16v_t acc[TA][TB], sum[TA][TB];
+    f16v_t sum[TA][TB];
 #pragma unroll
     for (int i = 0; i < TA; ++i)
 #pragma unroll
         for (int j = 0; j < TB; ++j) sum[i][j] = f16v_t{};
 
     int slot = 0;
-    auto step = [&](int s) {
+    // K step s into acc: onto it, or (grouped) the step's scaled sum added to pair
+    auto step = [&](int s, f16v_t(&acc)[TA][TB], f16v_t(&pair)[TA][TB]) {
         // stage s landed in this wave's share of the slot; only the LA - 1 stages after it may be in
         // flight.  A bare s_barrier: __syncthreads()'s release fence waits for every DMA in flight.
         wait_vmcnt<(LA - 1) * NDMA>();
@@ -341,7 +362,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
             float sc[TB], bi[TB];
 #pragma unroll
             for (int j = 0; j < TB; ++j) {
-                const int c = (wn * TB + j) * 32 + r32;
+                const int c = ACT ? j * (BN / 2) + wn * 32 + r32 : (wn * TB + j) * 32 + r32;
                 const uint32_t s = gs[c], b = gs[BN + c];
                 if constexpr (S16) {
                     sc[j] = a.sdt == DT_F16 ? raw_to_f32<DT_F16>(s) : raw_to_f32<DT_BF16>(s);
@@ -361,22 +382,35 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
                     for (int j = 0; j < TB; ++j)
 #pragma unroll
                         for (int c = 0; c < 4; ++c)
-                            sum[i][j][4 * q + c] = __builtin_fmaf(
-                                sc[j], acc[i][j][4 * q + c], __builtin_fmaf(bi[j], xv[c], sum[i][j][4 * q + c]));
+                            pair[i][j][4 * q + c] = __builtin_fmaf(
+                                sc[j], acc[i][j][4 * q + c], __builtin_fmaf(bi[j], xv[c], pair[i][j][4 * q + c]));
                 }
-        } else {
+        }
+    };
+    if constexpr (FOLD) {
+        // the sums of two steps meet before they join the total
+        for (int s = 0; s < nsteps; s += 2) {
+            f16v_t a0[TA][TB] = {}, a1[TA][TB] = {};
+            if constexpr (GROUPED) {
+                step(s, a0, a1);
+                if (s + 1 < nsteps) {
+                    f16v_t a2[TA][TB] = {};
+                    step(s + 1, a2, a1);
+                }
+            } else {
+                step(s, a0, a0);
+                if (s + 1 < nsteps) step(s + 1, a1, a1);
+            }
 #pragma unroll
             for (int i = 0; i < TA; ++i)
 #pragma unroll
-                for (int j = 0; j < TB; ++j) sum[i][j] += acc[i][j];
+                for (int j = 0; j < TB; ++j) {
+                    if constexpr (GROUPED) sum[i][j] += a1[i][j];
+                    else sum[i][j] += a0[i][j] + a1[i][j];
+                }
         }
-    };
-    for (int s = 0; s < nsteps; ++s) {
-#pragma unroll
-        for (int i = 0; i < TA; ++i)
-#pragma unroll
-            for (int j = 0; j < TB; ++j) acc[i][j] = f16v_t{};
-        step(s);
+    } else {
+        for (int s = 0; s < nsteps; ++s) step(s, sum, sum);  // f16 x: one chain over K
     }
     wait_vmcnt<0>();  // the trailing (re-read) DMA, before the block's LDS is given back
 
@@ -402,20 +436,25 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
             for (int r = 0; r < 16; ++r)
                 e[i][r] = -a.xe[min(m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3), a.M - 1)];
     }
+    // output tile j of the wave: columns at n; with ACT the gate tile's columns hold the outputs
+    constexpr int TO = ACT ? 1 : TB;
+    const auto out_col = [&](int j) { return n0 + (ACT ? wn : wn * TB + j) * 32 + r32; };
+    const auto value = [](float v, int ev, float sc, float bi) { return (P == 2 ? ldexpf(v, ev) : v) * sc + bi; };
     bool bad = false;
 #pragma unroll
-    for (int j = 0; j < TB; ++j) {
-        const int n = n0 + (wn * TB + j) * 32 + r32;
+    for (int j = 0; j < TO; ++j) {
+        const int n = out_col(j);
         if (n >= g.n) continue;
         const float sc = column_scale(g, a.sdt, n), bi = g.bias ? g.bias[n] : 0.0f;
+        const float sc1 = ACT ? column_scale(gu, a.sdt, n) : 1.0f, bi1 = ACT && gu.bias ? gu.bias[n] : 0.0f;
 #pragma unroll
         for (int i = 0; i < TA; ++i)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3);
-                float v = sum[i][j][r];
-                if constexpr (P == 2) v = ldexpf(v, e[i][r]);
-                v = v * sc + bi;
+                const int ev = P == 2 ? e[i][r] : 0;
+                float v = value(sum[i][j][r], ev, sc, bi);
+                if constexpr (ACT) v = act_mul(a.act, v, value(sum[i][TB - 1][r], ev, sc1, bi1));
                 if (m < a.M) {
                     g.y[(size_t)m * g.n + n] = v;
                     bad |= !finite_f32(v);
@@ -423,39 +462,51 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
             }
     }
     if (!bad) return;
-    // rolled and rare: this lane's non-finite results again
-    for (int t = 0; t < TA * TB * 16; ++t) {
-        const int i = t / (16 * TB), j = (t / 16) % TB, r = t & 15;
-        const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3), n = n0 + (wn * TB + j) * 32 + r32;
+    // rolled and rare: this lane's non-finite results again (a non-finite gate or up sum makes h non-finite)
+    for (int t = 0; t < TA * TO * 16; ++t) {
+        const int i = t / (16 * TO), j = (t / 16) % TO, r = t & 15;
+        const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3), n = out_col(j);
         if (m >= a.M || n >= g.n || finite_f32(g.y[(size_t)m * g.n + n])) continue;
-        g.y[(size_t)m * g.n + n] =
-            plain_dot<FMT, P>(a, g, m, n) * column_scale(g, a.sdt, n) + (g.bias ? g.bias[n] : 0.0f);
+        g.y[(size_t)m * g.n + n] = plain_output<FMT, P, ACT>(a, g, gu, m, n);
     }
 }
 
 // y of a split GEMM: the splits' sums added in split order, then the epilogue above.  A thread owns four
-// neighbouring columns of one row.
-template <int FMT, int P>
+// neighbouring outputs of one row.
+template <int FMT, int P, bool ACT>
 __global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a, int splits, int bn)
 {
-    const int quads = a.vcols / 4;
-    const size_t stride = (size_t)a.M * quads;
-    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < stride; t += (size_t)gridDim.x * 256) {
-        const int m = (int)(t / quads), vc = (int)(t - (size_t)m * quads) * 4, vt = vc / bn;
-        const int si = (a.nseg > 1 && vt >= a.tile0[1]) + (a.nseg > 2 && vt >= a.tile0[2]);
+    const int quads = a.vcols / (ACT ? 8 : 4);
+    const size_t stride = (size_t)a.M * (a.vcols / 4);
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < (size_t)a.M * quads; t += (size_t)gridDim.x * 256) {
+        const int m = (int)(t / quads), c0 = (int)(t - (size_t)m * quads) * 4;
+        int si = 0, n = c0, vc = c0;
+        if constexpr (ACT) {
+            vc = c0 / 32 * 64 + c0 % 32;  // 32 gate columns, then their 32 up columns
+        } else {
+            const int vt = c0 / bn;
+            si = (a.nseg > 1 && vt >= a.tile0[1]) + (a.nseg > 2 && vt >= a.tile0[2]);
+            n -= a.tile0[si] * bn;
+        }
         const XgSeg g = a.seg[si];
-        const int n = vc - a.tile0[si] * bn;
+        const XgSeg gu = ACT ? a.seg[1] : g;
         if (n >= g.n) continue;
-        const f4_t v = sum_splits_f4(reinterpret_cast<const f4_t*>(a.part) + t, stride, splits);
+        const f4_t* part = reinterpret_cast<const f4_t*>(a.part + (size_t)m * a.vcols + vc);
+        const f4_t v = sum_splits_f4(part, stride, splits);
+        f4_t u{};
+        if constexpr (ACT) u = sum_splits_f4(part + 8, stride, splits);
         const int e = P == 2 ? -a.xe[m] : 0;
         float* y = g.y + (size_t)m * g.n + n;
         f4_t o;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const int nc = min(n + c, g.n - 1);
-            const float sc = column_scale(g, a.sdt, nc), bi = g.bias ? g.bias[nc] : 0.0f;
-            o[c] = (P == 2 ? ldexpf(v[c], e) : v[c]) * sc + bi;
-            if (!finite_f32(o[c])) o[c] = plain_dot<FMT, P>(a, g, m, nc) * sc + bi;
+            o[c] = (P == 2 ? ldexpf(v[c], e) : v[c]) * column_scale(g, a.sdt, nc) + (g.bias ? g.bias[nc] : 0.0f);
+            if constexpr (ACT)
+                o[c] = act_mul(a.act, o[c],
+                               (P == 2 ? ldexpf(u[c], e) : u[c]) * column_scale(gu, a.sdt, nc) +
+                                   (gu.bias ? gu.bias[nc] : 0.0f));
+            if (!finite_f32(o[c])) o[c] = plain_output<FMT, P, ACT>(a, g, gu, m, nc);
         }
         if ((g.n & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
             *reinterpret_cast<f4_t*>(y) = o;
@@ -464,6 +515,20 @@ __global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a,
             for (int c = 0; c < 4; ++c)
                 if (n + c < g.n) y[c] = o[c];
         }
+    }
+}
+
+// f16 rows zero-padded to Kp (K % 8 == 0)
+__global__ __launch_bounds__(256) void pad_x_kernel(const _Float16* __restrict__ x, int K, int Kp, size_t units,
+                                                    _Float16* __restrict__ xp)
+{
+    const int per_row = Kp / 8;
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < units; t += (size_t)gridDim.x * 256) {
+        const size_t m = t / per_row;
+        const int u = (int)(t - m * per_row);
+        u4_t v = {0u, 0u, 0u, 0u};
+        if (u * 8 < K) v = *reinterpret_cast<const u4_t*>(x + m * K + u * 8);
+        reinterpret_cast<u4_t*>(xp)[t] = v;
     }
 }
 
@@ -544,27 +609,30 @@ __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ 
     }
 }
 
-// The tile forms: 0 = 32 rows x 128 columns (2 waves), 1 = 64 x 128 (4 waves), 2 = 128 x 256 (8 waves).
+// The tile forms, rows x columns: f32 x 32 x 128 (2 waves), 64 x 128 (4 waves), 128 x 256 (8 waves); f16 x
+// 32 x 128, 128 x 128, 256 x 256.
 struct XgPlan {
     int form, bm, bn, vtiles, steps_per_split, splits;
     size_t xp_off, sum_off, part_off, bytes;  // workspace: exponents, parts, sums of x', split sums
 };
 
-XgPlan xg_plan(int fmt, const XgSeg* segs, int nseg, int M, int K)
+XgPlan xg_plan(int fmt, int P, const XgSeg* segs, int nseg, bool act, int M, int K)
 {
     XgPlan p{};
     const int steps = (K + kBK - 1) / kBK;
     auto tiles = [&](int bm, int bn) {
         int t = 0;
-        for (int i = 0; i < nseg; ++i) t += (segs[i].n + bn - 1) / bn;
+        if (act) t = (segs[0].n + bn / 2 - 1) / (bn / 2);
+        else
+            for (int i = 0; i < nseg; ++i) t += (segs[i].n + bn - 1) / bn;
         p.bm = bm, p.bn = bn, p.vtiles = t;
         return (int64_t)t * ((M + bm - 1) / bm);
     };
-    int64_t blocks = tiles(128, 256);
+    int64_t blocks = tiles(P == 2 ? 128 : 256, 256);
     p.form = 2;
     if (blocks < 192) {
         p.form = M > 32 ? 1 : 0;
-        blocks = p.form ? tiles(64, 128) : tiles(32, 128);
+        blocks = p.form ? tiles(P == 2 ? 64 : 128, 128) : tiles(32, 128);
     }
     int splits = 1;
     const int64_t want = p.form == 2 ? 256 : 512;
@@ -572,18 +640,18 @@ XgPlan xg_plan(int fmt, const XgSeg* segs, int nseg, int M, int K)
     p.steps_per_split = (steps + splits - 1) / splits;
     p.splits = (steps + p.steps_per_split - 1) / p.steps_per_split;
     const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    p.xp_off = up((size_t)M * 4);
-    p.sum_off = p.xp_off + up((size_t)M * 2 * steps * kBK * 2);
+    p.xp_off = P == 2 ? up((size_t)M * 4) : 0;
+    p.sum_off = p.xp_off + (P == 2 || K % kBK ? up((size_t)M * P * steps * kBK * 2) : 0);
     p.part_off = p.sum_off + (fmt == XG_Q4 ? up((size_t)M * steps * 4) : 0);
     p.bytes = p.part_off + (p.splits > 1 ? (size_t)p.splits * M * p.vtiles * p.bn * 4 : 0);
     return p;
 }
 
-template <int FMT, bool S16, int P, int TA, int TB, int WM, int WN, int NST>
+template <int FMT, bool S16, int P, int TA, int TB, int WM, int WN, int NST, bool ACT>
 hipError_t launch_form(const XgArgs& a, const XgPlan& p, hipStream_t st)
 {
     constexpr int lds = NST * stage_bytes(FMT, P, 32 * TA * WM, 32 * TB * WN, Fmt<FMT>::kStepBytes);
-    auto kern = qgemm_exact_kernel<FMT, S16, P, TA, TB, WM, WN, NST>;
+    auto kern = qgemm_exact_kernel<FMT, S16, P, TA, TB, WM, WN, NST, ACT>;
     if constexpr (lds > 64 * 1024) {
         const hipError_t e = allow_big_lds(kern, lds);
         if (e != hipSuccess) return e;
@@ -593,14 +661,55 @@ hipError_t launch_form(const XgArgs& a, const XgPlan& p, hipStream_t st)
     return hipGetLastError();
 }
 
+template <int FMT, bool S16, int P, bool ACT>
+hipError_t launch_act(const XgArgs& a, const XgPlan& p, hipStream_t st)
+{
+    // f16 rows are twice the bytes: two stages keep two blocks (form 1) or one (form 2) on a CU
+    constexpr int NST = FMT == XG_F16 ? 2 : 3, T1 = P == 2 ? 1 : 2;
+    hipError_t e = p.form == 2   ? launch_form<FMT, S16, P, 2 * T1, 2, 2, 4, NST, ACT>(a, p, st)
+                   : p.form == 1 ? launch_form<FMT, S16, P, T1, 2, 2, 2, NST, ACT>(a, p, st)
+                                 : launch_form<FMT, S16, P, 1, 2, 1, 2, 3, ACT>(a, p, st);
+    if (e != hipSuccess || p.splits == 1) return e;
+    const size_t quads = (size_t)a.M * a.vcols / (ACT ? 8 : 4);
+    const unsigned blocks = (unsigned)std::min<size_t>((quads + 255) / 256, 4096);
+    hipLaunchKernelGGL((qgemm_exact_reduce_kernel<FMT, P, ACT>), dim3(blocks), dim3(256), 0, st, a, p.splits, p.bn);
+    return hipGetLastError();
+}
+
+template <int FMT, bool S16>
+hipError_t launch_f32x(const XgArgs& a, const XgPlan& p, bool act, int32_t* xe, _Float16* xp, float* xsum,
+                       hipStream_t st)
+{
+    hipLaunchKernelGGL((split_x_kernel<Fmt<FMT>::kPairs, FMT == XG_Q4>), dim3(a.M), dim3(256), 0, st,
+                       static_cast<const float*>(a.x), a.K, a.Kp, xp, xe, xsum);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if constexpr (FMT != XG_F16)
+        if (act) return launch_act<FMT, S16, 2, true>(a, p, st);
+    return launch_act<FMT, S16, 2, false>(a, p, st);
+}
+
 }  // namespace
 
-bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int group, int M, int K, const void* x)
+bool qgemm_exact_supported(const XgCall& c, int M, int K)
 {
-    const bool nibbles = fmt == XG_I4 || fmt == XG_Q4;
+    const bool nibbles = c.fmt == XG_I4 || c.fmt == XG_Q4;
     // weight rows start on 16-byte boundaries; a K step has one scale
-    if (M < 5 || K <= 0 || K % (nibbles ? 32 : fmt == XG_I8 ? 16 : 8) != 0) return false;
-    if (fmt == XG_Q4 && (group <= 0 || group % kBK != 0)) return false;
+    if (M < 5 || K <= 0 || K % (nibbles ? 32 : c.fmt == XG_I8 ? 16 : 8) != 0) return false;
+    if (c.fmt == XG_Q4 && (c.group <= 0 || c.group % kBK != 0)) return false;
+    if (c.x_f16 && c.fmt != XG_I8) return false;
+    if (c.act >= 0 && (c.fmt == XG_F16 || c.nseg != 2 || c.segs[0].n != c.segs[1].n)) return false;
+    int64_t n = 0;
+    for (int i = 0; i < c.nseg; ++i) {
+        if (c.segs[i].n <= 0 || (reinterpret_cast<uintptr_t>(c.segs[i].w) & 15) != 0) return false;
+        // group scales and biases are fetched as whole elements
+        if (((reinterpret_cast<uintptr_t>(c.segs[i].gs) | reinterpret_cast<uintptr_t>(c.segs[i].gb)) & 3) != 0) return false;
+        n += c.segs[i].n;
+    }
+    if ((reinterpret_cast<uintptr_t>(c.x) & 15) != 0 || (M + 31) / 32 > 65535) return false;
+    // a tile's byte offsets are 32-bit
+    if ((uint64_t)K * 1024 >= (1ull << 31) || n >= (1 << 30)) return false;
+    if (c.x_f16 && K % kBK == 0) return true;  // no copy of x
     // The kernels of single rows walk the rows one after the other (f16: four at a time), so they take
     // longer with M K (a wave's walk) and with M K N (the whole work); the three launches here take 14-17
     // us at small sizes.  Measured, row kernels against these (us, rows x outputs x k):
@@ -608,56 +717,27 @@ bool qgemm_exact_supported(int fmt, const XgSeg* segs, int nseg, int group, int 
     //   i4    5 x 960 x 960 16.0 / 16.0, 8 x 960 x 960 24.4 / 15.3
     //   f16   8 x 960 x 960 11.3 / 14.9, 12 x 2560 x 960 21.2 / 14.9, 5 x 8192 x 960 19.5 / 14.9
     //   q4    16 x 2560 x 960 13.3 / 17.7, 24 x 1024 x 1024 14.6 / 13.3, 5 x 16384 x 960 17.5 / 17.4
-    const bool affine = fmt == XG_Q4 && segs[0].gb;
-    const int64_t walk = affine ? 24000 : fmt == XG_F16 ? 10000 : nibbles ? 5000 : 7000;
+    const bool affine = c.fmt == XG_Q4 && c.segs[0].gb;
+    const int64_t walk = affine ? 24000 : c.fmt == XG_F16 ? 10000 : nibbles ? 5000 : 7000;
     const double work = affine ? 78e6 : 35e6;
-    if ((int64_t)M * K < walk && (double)M * K * segs[0].n < work) return false;
-    if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 || (M + 31) / 32 > 65535) return false;
-    int64_t n = 0;
-    for (int i = 0; i < nseg; ++i) {
-        if (segs[i].n <= 0 || (reinterpret_cast<uintptr_t>(segs[i].w) & 15) != 0) return false;
-        // group scales and biases are fetched as whole elements
-        if (((reinterpret_cast<uintptr_t>(segs[i].gs) | reinterpret_cast<uintptr_t>(segs[i].gb)) & 3) != 0) return false;
-        n += segs[i].n;
-    }
-    // a tile's byte offsets are 32-bit
-    return (uint64_t)K * 1024 < (1ull << 31) && n < (1 << 30);
+    return (int64_t)M * K * c.nseg >= walk || (double)M * K * n >= work;
 }
 
-size_t qgemm_exact_workspace_bytes(int fmt, const XgSeg* segs, int nseg, int M, int K)
+size_t qgemm_exact_workspace_bytes(const XgCall& c, int M, int K)
 {
-    return xg_plan(fmt, segs, nseg, M, K).bytes;
+    return xg_plan(c.fmt, c.x_f16 ? 1 : 2, c.segs, c.nseg, c.act >= 0, M, K).bytes;
 }
 
-template <int FMT, bool S16>
-static hipError_t launch_fmt(const XgArgs& a, const XgPlan& p, int32_t* xe, _Float16* xp, float* xsum, hipStream_t st)
+hipError_t launch_qgemm_exact(const XgCall& c, int M, int K, void* ws, hipStream_t st)
 {
-    hipLaunchKernelGGL((split_x_kernel<Fmt<FMT>::kPairs, FMT == XG_Q4>), dim3(a.M), dim3(256), 0, st,
-                       static_cast<const float*>(a.x), a.K, a.Kp, xp, xe, xsum);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    // f16 rows are twice the bytes: two stages keep two blocks (form 1) or one (form 2) on a CU
-    constexpr int NST = FMT == XG_F16 ? 2 : 3;
-    e = p.form == 2   ? launch_form<FMT, S16, 2, 2, 2, 2, 4, NST>(a, p, st)
-        : p.form == 1 ? launch_form<FMT, S16, 2, 1, 2, 2, 2, NST>(a, p, st)
-                      : launch_form<FMT, S16, 2, 1, 2, 1, 2, 3>(a, p, st);
-    if (e != hipSuccess || p.splits == 1) return e;
-    const size_t quads = (size_t)a.M * a.vcols / 4;
-    const unsigned blocks = (unsigned)std::min<size_t>((quads + 255) / 256, 4096);
-    hipLaunchKernelGGL((qgemm_exact_reduce_kernel<FMT, 2>), dim3(blocks), dim3(256), 0, st, a, p.splits, p.bn);
-    return hipGetLastError();
-}
-
-hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, int group, int gpr, const float* x, int M,
-                              int K, void* ws, hipStream_t st)
-{
-    const XgPlan p = xg_plan(fmt, segs, nseg, M, K);
+    const bool act = c.act >= 0;
+    const XgPlan p = xg_plan(c.fmt, c.x_f16 ? 1 : 2, c.segs, c.nseg, act, M, K);
     XgArgs a{};
-    a.nseg = nseg;
-    for (int i = 0, t = 0; i < nseg; ++i) {
-        a.seg[i] = segs[i];
-        a.tile0[i] = t;
-        t += (segs[i].n + p.bn - 1) / p.bn;
+    a.nseg = c.nseg;
+    for (int i = 0, t = 0; i < c.nseg; ++i) {
+        a.seg[i] = c.segs[i];
+        a.tile0[i] = act ? 0 : t;
+        t += (c.segs[i].n + p.bn - 1) / p.bn;
     }
     unsigned char* base = static_cast<unsigned char*>(ws);
     int32_t* xe = reinterpret_cast<int32_t*>(base);
@@ -666,23 +746,36 @@ hipError_t launch_qgemm_exact(int fmt, const XgSeg* segs, int nseg, int sdt, int
     a.xe = xe;
     a.xp = xp;
     a.xsum = xsum;
-    a.x = x;
+    a.x = c.x;
     a.part = p.splits > 1 ? reinterpret_cast<float*>(base + p.part_off) : nullptr;
     a.M = M;
     a.K = K;
     a.Kp = (K + kBK - 1) / kBK * kBK;
     a.steps_per_split = p.steps_per_split;
     a.vcols = p.vtiles * p.bn;
-    a.sdt = sdt;
-    a.group = group;
-    a.gpr = gpr;
-    switch (fmt) {
-        case XG_I8: return launch_fmt<XG_I8, false>(a, p, xe, xp, xsum, st);
-        case XG_I4: return launch_fmt<XG_I4, false>(a, p, xe, xp, xsum, st);
-        case XG_F16: return launch_fmt<XG_F16, false>(a, p, xe, xp, xsum, st);
+    a.sdt = c.sdt;
+    a.group = c.group;
+    a.gpr = c.gpr;
+    a.act = c.act;
+    if (c.x_f16) {
+        if (a.Kp == K) {
+            a.xp = static_cast<const _Float16*>(c.x);
+        } else {
+            const size_t units = (size_t)M * a.Kp / 8;
+            hipLaunchKernelGGL(pad_x_kernel, dim3((unsigned)std::min<size_t>((units + 255) / 256, 4096)), dim3(256), 0, st,
+                               static_cast<const _Float16*>(c.x), K, a.Kp, units, xp);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+        return act ? launch_act<XG_I8, false, 1, true>(a, p, st) : launch_act<XG_I8, false, 1, false>(a, p, st);
+    }
+    switch (c.fmt) {
+        case XG_I8: return launch_f32x<XG_I8, false>(a, p, act, xe, xp, xsum, st);
+        case XG_I4: return launch_f32x<XG_I4, false>(a, p, act, xe, xp, xsum, st);
+        case XG_F16: return launch_f32x<XG_F16, false>(a, p, act, xe, xp, xsum, st);
         case XG_Q4:
-            return sdt == DT_F32 ? launch_fmt<XG_Q4, false>(a, p, xe, xp, xsum, st)
-                                 : launch_fmt<XG_Q4, true>(a, p, xe, xp, xsum, st);
+            return c.sdt == DT_F32 ? launch_f32x<XG_Q4, false>(a, p, act, xe, xp, xsum, st)
+                                   : launch_f32x<XG_Q4, true>(a, p, act, xe, xp, xsum, st);
         default: return hipErrorInvalidValue;
     }
 }

@@ -159,7 +159,9 @@ int32_t cellm_hip_qgemv_q4_affine(cellm_hip_ctx_t* ctx, const uint32_t* wq, cons
                                   int64_t m, int64_t n, int64_t k, void* stream);
 
 /* Fused QKV, one launch for m <= 4 (f16/f32 x, cols % 16 == 0, 16-byte
- * aligned W and x; other shapes run three cellm_hip_qgemv_i8 launches):
+ * aligned W and x); f32 x at 5 rows and more runs the MFMA GEMM of
+ * cellm_hip_qgemv_i8 once over the three; other shapes run three
+ * cellm_hip_qgemv_i8 launches:
  *   q = (Wq . x) * sq (+ bq), k and v likewise with rows_kv rows each.
  * Each projection has its own scales (per row when n_s >= rows, per tensor when n_s == 1)
  * and optional bias (NULL = none); all scales share scale_dtype.  Replaces
@@ -173,7 +175,8 @@ int32_t cellm_hip_qgemv_i8_qkv(cellm_hip_ctx_t* ctx, const int8_t* wq, const voi
 
 /* The q, k and v projections of MLX 4-bit affine weights sharing x, in one
  * launch for m <= 4 (f16 or f32 x, cols % 32 == 0, group >= 32, 16-byte
- * aligned x and W); other shapes run one GEMV per projection.  sq/bq ... are
+ * aligned x and W), or by the MFMA GEMM for f32 x at 5 rows and more; other
+ * shapes run one GEMV per projection.  sq/bq ... are
  * each matrix's scales and group biases in sb_dtype (cellm_hip_qgemv_q4_affine);
  * biasq/biask/biasv (f32 [rows], or NULL) are added after each row sum, as
  * add_projection_bias_if_present does (qwen.rs:1132-1139).  No reference
@@ -189,8 +192,9 @@ int32_t cellm_hip_qgemv_q4_affine_qkv(cellm_hip_ctx_t* ctx, const uint32_t* wq, 
 
 /* Gate and up projections with the SiLU * up epilogue:
  *   h = silu((Wg . x) * sg (+ bg)) * ((Wu . x) * su (+ bu)),  silu(g) = g / (1 + exp(-g)).
- * One launch for m <= 4 under the conditions of cellm_hip_qgemv_i8_qkv; other
- * shapes run two GEMVs and an elementwise kernel.  Replaces the gate/up
+ * One launch for m <= 4 under the conditions of cellm_hip_qgemv_i8_qkv; f32 x at
+ * 5 rows and more runs the MFMA GEMM of cellm_hip_qgemv_i8 with the activation
+ * in its epilogue; other shapes run two GEMVs and an elementwise kernel.  Replaces the gate/up
  * encode_mv_i8(_bias) pair plus encode_silu_mul_f32_inplace of the decode
  * graphs (crates/cellm-model/src/llama_graph.rs:318-327,
  * crates/cellm-model/src/qwen.rs:1445-1453; metal.rs:235-245, 956), and the
@@ -203,7 +207,8 @@ int32_t cellm_hip_qgemv_i8_gate_up_silu(cellm_hip_ctx_t* ctx, const int8_t* wg, 
 /* The same for MLX 4-bit affine gate/up weights; sg/bg and su/bu are the affine
  * scales/biases of each matrix.  One launch computes both rows and the SiLU *
  * up for m <= 4 with f16 x, k % 32 == 0, group >= 32 and 16-byte aligned x,
- * wg and wu; other shapes run two cellm_hip_qgemv_q4_affine launches and the
+ * wg and wu, and the MFMA GEMM of cellm_hip_qgemv_q4_affine for f32 x at 5 rows
+ * and more; other shapes run two cellm_hip_qgemv_q4_affine launches and the
  * SiLU * up kernel. */
 int32_t cellm_hip_qgemv_q4_affine_gate_up_silu(cellm_hip_ctx_t* ctx, const uint32_t* wg, const void* sg,
                                                const void* bg, const uint32_t* wu, const void* su, const void* bu,
@@ -225,8 +230,9 @@ int32_t cellm_hip_qgemv_q4_affine_gate_up_gelu(cellm_hip_ctx_t* ctx, const uint3
                                                float* h, int64_t m, int64_t n, int64_t k, void* stream);
 
 /* The same over symmetric i4 gate/up weights (gemma.rs:1446-1471 runs the i4
- * branch of linear_f16_out_in for each): two cellm_hip_qgemv_i4_sym launches
- * (arguments as there, one gs for both) and the GELU * up kernel. */
+ * branch of linear_f16_out_in for each; arguments as cellm_hip_qgemv_i4_sym, one
+ * gs for both): one MFMA GEMM where that call takes it, else two such launches
+ * and the GELU * up kernel. */
 int32_t cellm_hip_qgemv_i4_gate_up_gelu(cellm_hip_ctx_t* ctx, const uint8_t* wg, const uint16_t* sg, int64_t n_sg,
                                         const uint8_t* wu, const uint16_t* su, int64_t n_su, int64_t gs,
                                         const void* x, int32_t x_dtype, float* h, int64_t m, int64_t n, int64_t k,

@@ -217,3 +217,101 @@ def test_captured_calls_use_no_scratch(ops):
         graph.replay()
         torch.cuda.synchronize()
         assert _rel(y.cpu(), ref) <= TOL
+
+
+def _q4(n, k, seed, sdt=torch.float32):
+    g = torch.Generator().manual_seed(seed)
+    w = torch.randint(-2**31, 2**31, (n, k // 8), generator=g, dtype=torch.int64).to(torch.int32)
+    s = (torch.rand(n, -(-k // 64), generator=g) * 0.01 + 1e-3).to(sdt)
+    b = (s.float() * (-7.5 + torch.randn(s.shape, generator=g))).to(sdt)
+    q = ((w[:, :, None] >> torch.arange(0, 32, 4)) & 15).reshape(n, k).double()
+    wide = lambda t: t.double().repeat_interleave(64, 1)[:, :k]
+    return w.cuda(), s.cuda(), b.cuda(), q * wide(s) + wide(b)
+
+
+def _i4(n, k, gs, seed):
+    g = torch.Generator().manual_seed(seed)
+    w = torch.randint(0, 256, (n, k // 2), generator=g, dtype=torch.uint8)
+    s = (torch.rand(n, -(-k // gs), generator=g) * 0.01 + 1e-3).half()
+    q = torch.stack([w & 15, w >> 4], 2).reshape(n, k).double() - 8
+    return w.cuda(), s.cuda(), q * s.double().repeat_interleave(gs, 1)[:, :k]
+
+
+def _act(g, u, act):
+    if act == "silu":
+        return g / (1 + torch.exp(-g)) * u
+    return 0.5 * g * (1 + torch.tanh(0.7978846 * (g + 0.044715 * g * g * g))) * u
+
+
+# segments that end inside a tile, one far smaller than a tile; unsplit, split over k, and the wide form
+QKV = [(40, 130, 33, 224), (77, 896, 128, 896), (512, 300, 260, 2560), (1030, 2500, 520, 320)]
+
+
+@pytest.mark.parametrize("m,rq,rkv,k", QKV)
+def test_qkv_f32_rows(ops, m, rq, rkv, k):
+    x = _x(m, k, m + k)
+    rows, xc = (rq, rkv, rkv), x.cuda()
+    bias = [torch.randn(r, generator=torch.Generator().manual_seed(r)) for r in rows]
+    w = [_i8(r, k, 7 + i) for i, r in enumerate(rows)]
+    y = [torch.full((m, r), float("nan"), device="cuda") for r in rows]
+    dev = [t.cuda() for ws in w for t in ws]
+    ops.encode_qkv_i8(*dev, xc, *y, bq=bias[0].cuda(), bk=None, bv=bias[2].cuda())
+    torch.cuda.synchronize()
+    for i in range(3):
+        ref = x.double() @ w[i][0].double().t() * w[i][1].double() + (bias[i].double() if i != 1 else 0)
+        assert _rel(y[i].cpu(), ref) <= TOL, i
+    q = [_q4(r, k, 17 + i) for i, r in enumerate(rows)]
+    for t in y:
+        t.fill_(float("nan"))
+    ops.encode_qkv_q4_affine(*q[0][:3], *q[1][:3], *q[2][:3], xc, *y, biasq=bias[0].cuda(), biasv=bias[2].cuda())
+    torch.cuda.synchronize()
+    for i in range(3):
+        assert _rel(y[i].cpu(), x.double() @ q[i][3].t() + (bias[i].double() if i != 1 else 0)) <= TOL, i
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("m,n,k", [(40, 70, 224), (77, 33, 896), (200, 4096, 1024), (300, 100, 2560), (1100, 2500, 320)])
+def test_gate_up_f32_rows(ops, m, n, k, act):
+    """One launch of gate and up with the activation, against the 64-bit sums: act(g) * u carries both sums' errors."""
+    x = _x(m, k, m + k) * 0.3
+    xc, h = x.cuda(), torch.full((m, n), float("nan"), device="cuda")
+    (wg, sg), (wu, su) = _i8(n, k, 1), _i8(n, k, 2)
+    sg, su = sg * 0.02, su * 0.02  # sums near 1, where the activation bends
+    bg, bu = (torch.randn(n, generator=torch.Generator().manual_seed(i)) for i in (3, 4))
+    fn = ops.encode_gate_up_silu_i8 if act == "silu" else ops.encode_gate_up_gelu_i8
+    fn(wg.cuda(), sg.cuda(), wu.cuda(), su.cuda(), xc, h, bg=bg.cuda(), bu=bu.cuda())
+    torch.cuda.synchronize()
+    one = lambda w, s, b: x.double() @ w.double().t() * s.double() + b.double()
+    assert _rel(h.cpu(), _act(one(wg, sg, bg), one(wu, su, bu), act)) <= 2 * TOL
+    g, u = _q4(n, k, 5), _q4(n, k, 6)
+    h.fill_(float("nan"))
+    fn = ops.encode_gate_up_silu_q4_affine if act == "silu" else ops.encode_gate_up_gelu_q4_affine
+    fn(*g[:3], *u[:3], xc, h)
+    torch.cuda.synchronize()
+    assert _rel(h.cpu(), _act(x.double() @ g[3].t(), x.double() @ u[3].t(), act)) <= 2 * TOL
+    if act == "gelu":
+        for gs in (k, 64):
+            if gs != k and k % 64:
+                continue
+            g, u = _i4(n, k, gs, 8), _i4(n, k, gs, 9)
+            h.fill_(float("nan"))
+            ops.encode_gate_up_gelu_i4_sym(*g[:2], *u[:2], gs, xc, h, k)
+            torch.cuda.synchronize()
+            assert _rel(h.cpu(), _act(x.double() @ g[2].t(), x.double() @ u[2].t(), act)) <= 2 * TOL, gs
+
+
+@pytest.mark.parametrize("k", [832, 2560])  # unsplit and split over k
+def test_gate_up_non_finite(ops, k):
+    m, n = 9, 70
+    x = _x(m, k, 8) * 0.3
+    x[1, 5], x[2, 7], x[3, 0] = float("inf"), float("nan"), float("-inf")
+    (wg, sg), (wu, su) = _i8(n, k, 1), _i8(n, k, 2)
+    h = torch.empty(m, n, device="cuda")
+    ops.encode_gate_up_silu_i8(wg.cuda(), (sg * 0.02).cuda(), wu.cuda(), (su * 0.02).cuda(), x.cuda(), h)
+    torch.cuda.synchronize()
+    g, u = ((x @ w.float().t()) * (s * 0.02) for w, s in ((wg, sg), (wu, su)))
+    ref, got = g * (1 / (1 + torch.exp(-g))) * u, h.cpu()
+    assert np.array_equal(torch.isnan(got).numpy(), torch.isnan(ref).numpy())
+    assert np.array_equal(torch.isposinf(got).numpy(), torch.isposinf(ref).numpy())
+    assert np.array_equal(torch.isneginf(got).numpy(), torch.isneginf(ref).numpy())
+    assert _rel(got[4:], _act(g[4:].double(), u[4:].double(), "silu")) <= 1e-5  # against f32 sums
