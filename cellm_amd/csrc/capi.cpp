@@ -236,16 +236,18 @@ bool capturing(hipStream_t st)
 
 // The multi-row GEMM (qgemm_exact.hip) where it applies: *done tells whether it was enqueued.  It needs
 // scratch for x's parts, which the one-wave-per-row kernels do without, so a call that cannot have it
-// (captures, no memory) is left to them.
+// (captures, no memory) is left to them.  int8 over f16 x in place (k % 64 == 0) has no such kernel to
+// go back to and needs split sums at most.
 int32_t try_qgemm_exact(cellm_hip_ctx* ctx, const XgCall& c, int64_t m, int64_t k, hipStream_t st, bool* done)
 {
     *done = false;
     if (!qgemm_exact_supported(c, (int)m, (int)k)) return CELLM_HIP_OK;
     const size_t need = qgemm_exact_workspace_bytes(c, (int)m, (int)k);
-    if (need && capturing(st)) return CELLM_HIP_OK;
+    const bool in_place = c.x_f16 && k % 64 == 0;
+    if (need && !in_place && capturing(st)) return CELLM_HIP_OK;
     float* ws = nullptr;
     const int32_t rc = get_workspace(ctx, st, need, &ws);
-    if (rc == CELLM_HIP_ERR_OUT_OF_MEMORY) {
+    if (rc == CELLM_HIP_ERR_OUT_OF_MEMORY && !in_place) {
         (void)hipGetLastError();
         return CELLM_HIP_OK;
     }
@@ -279,16 +281,15 @@ int32_t qgemv_i8_impl(cellm_hip_ctx* ctx, const int8_t* w, const void* scales, i
                 "qgemv_mfma_i8 launch");
         return CELLM_HIP_OK;
     }
-    if ((force_gemm || m > 4) && gemm_ok) {
-        float* ws = nullptr;
-        const size_t need = qgemm_workspace_bytes(1, (int)m, (int)n, (int)k, 64, sdt);
-        if (int32_t rc = get_workspace(ctx, st, need, &ws)) return rc;
-        HIP_TRY(launch_qgemm_i8_ws(w, scales, sdt, per_channel, reinterpret_cast<const _Float16*>(x), bias, y, (int)m,
-                                   (int)n, (int)k, ws, st),
-                "qgemm_i8 launch");
-        return CELLM_HIP_OK;
+    if (xdt == DT_F16 && (force_gemm ? gemm_ok : m > 4)) {
+        const XgSeg seg{w, scales, bias, y, (int)n, per_channel, nullptr, nullptr};
+        const XgCall call{XG_I8, &seg, 1, sdt, x, true, -1, 0, 0};
+        bool done = false;
+        if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
+        if (done) return CELLM_HIP_OK;
     }
-    if (force_gemm) return set_error(CELLM_HIP_ERR_UNSUPPORTED, "qgemm_i8 needs f16 x, k %% 64 == 0, 16-byte alignment");
+    if (force_gemm && !gemm_ok)
+        return set_error(CELLM_HIP_ERR_UNSUPPORTED, "qgemm_i8 needs f16 x, k %% 64 == 0, 16-byte alignment");
     // f32 x over a long output at several rows (the Llama lm_head of a multi-session step,
     // llama.rs:602-643): exact integer sums on int8 MFMA over three x digits per row
     if (xdt == DT_F32 && m >= kI8F32xMfmaMinM && n >= kF32xMfmaMinRows && aligned16(w) && aligned16(x) &&
@@ -393,7 +394,7 @@ int32_t qgemv_q4_impl(cellm_hip_ctx* ctx, const uint32_t* wq, const void* scales
     }
     if ((force_gemm || m > 4) && gemm_ok) {
         float* ws = nullptr;
-        const size_t need = qgemm_workspace_bytes(0, (int)m, (int)n, (int)k, (int)group, sbt);
+        const size_t need = qgemm_workspace_bytes((int)m, (int)n, (int)k, (int)group, sbt);
         if (int32_t rc = get_workspace(ctx, st, need, &ws)) return rc;
         HIP_TRY(launch_qgemm_q4_affine_ws(wq, scales, biases, sbt, (int)group, reinterpret_cast<const _Float16*>(x), y,
                                           (int)m, (int)n, (int)k, ws, st),
@@ -437,12 +438,12 @@ int32_t qkv_i8_impl(cellm_hip_ctx* ctx, const int8_t* const w[3], const void* co
         HIP_TRY(launch_qgemv_i8_fused(segs, 3, false, ACT_SILU, sdt, x, xdt, (int)m, (int)k, st), "qgemv_i8_qkv launch");
         return CELLM_HIP_OK;
     }
-    // many f32 rows: x split once for the three
-    if (xdt == DT_F32) {
+    // many rows: one GEMM over the three (f32: x split once; f16 up to 64 rows: the batched GEMVs)
+    if (xdt == DT_F32 || (xdt == DT_F16 && m > 64)) {
         XgSeg xs[3];
         for (int i = 0; i < 3; ++i)
             xs[i] = XgSeg{w[i], s[i], b[i], y[i], (int)rows[i], n_s[i] >= rows[i] ? 1 : 0, nullptr, nullptr};
-        const XgCall call{XG_I8, xs, 3, sdt, x, false, -1, 0, 0};
+        const XgCall call{XG_I8, xs, 3, sdt, x, xdt == DT_F16, -1, 0, 0};
         bool done = false;
         if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;
@@ -470,10 +471,10 @@ int32_t gate_up_i8_impl(cellm_hip_ctx* ctx, const int8_t* wg, const void* sg, in
         HIP_TRY(launch_qgemv_i8_fused(segs, 2, true, act, sdt, x, xdt, (int)m, (int)k, st), "qgemv_i8 gate/up launch");
         return CELLM_HIP_OK;
     }
-    if (xdt == DT_F32) {
+    if (xdt == DT_F32 || (xdt == DT_F16 && m > 64)) {
         const XgSeg xs[2] = {XgSeg{wg, sg, bg, h, (int)n, n_sg >= n ? 1 : 0, nullptr, nullptr},
                              XgSeg{wu, su, bu, nullptr, (int)n, n_su >= n ? 1 : 0, nullptr, nullptr}};
-        const XgCall call{XG_I8, xs, 2, sdt, x, false, act, 0, 0};
+        const XgCall call{XG_I8, xs, 2, sdt, x, xdt == DT_F16, act, 0, 0};
         bool done = false;
         if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;

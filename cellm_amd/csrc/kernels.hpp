@@ -75,18 +75,15 @@ hipError_t launch_qgemv_q4_segs(const Q4FusedSeg* segs, int nseg, int sbt, int g
 
 // Prefill / batched qGEMM on MFMA: Y[M,N] = X[M,K] . dequant(W)[N,K]^T with
 // W tiles dequantized to f16 in LDS and f32 accumulation.  Requires K % 64 == 0
-// and 16-byte aligned W and X.  `workspace` (qgemm_workspace_bytes: wt 0 = q4
-// affine, 1 = int8) enables split-K; nullptr runs without it.
+// and 16-byte aligned W and X.  `workspace` (qgemm_workspace_bytes) enables split-K; nullptr runs without it.
 int qgemm_splits(int M, int N, int K);
-size_t qgemm_workspace_bytes(int wt, int M, int N, int K, int group_size, int sbt);
+size_t qgemm_workspace_bytes(int M, int N, int K, int group_size, int sbt);
 hipError_t launch_qgemm_q4_affine_ws(const uint32_t* wq, const void* S, const void* B, int sbt, int group_size,
                                      const _Float16* x, float* y, int M, int N, int K, float* workspace,
                                      hipStream_t st);
-hipError_t launch_qgemm_i8_ws(const int8_t* w, const void* S, int sdt, int per_channel, const _Float16* x,
-                              const float* bias, float* y, int M, int N, int K, float* workspace, hipStream_t st);
 
-// Multi-row GEMM over f32 x, weights exact in f16 (qgemm_exact.hip): M >= 5 (and rows enough to pay
-// for its launches), 16-byte aligned W, x and weight rows.  Up to three matrices share x.  `ws` holds
+// Multi-row GEMM, weights exact in f16 (qgemm_exact.hip): f32 x at M >= 5 (and rows enough to pay for its
+// launches), or f16 x over int8; 16-byte aligned W, x and weight rows.  Up to three matrices share x.  `ws` holds
 // x's f16 parts and the split sums.
 enum { XG_I8 = 0, XG_I4 = 1, XG_F16 = 2, XG_Q4 = 3 };
 struct XgSeg {

@@ -1,4 +1,4 @@
-// Quantized-weight GEMM on MFMA for prefill and batched decode (gfx950).
+// MLX 4-bit GEMM on MFMA for prefill and batched decode over f16 activations (gfx950).
 //
 //   Y[M,N] = X[M,K] . dequant(W)[N,K]^T        (f16 X, f32 accumulate, f32 Y)
 //
@@ -13,8 +13,6 @@
 // for K % 128 == 0.  For f16 or bf16 scales, f32(q)*s is exact in f32, so
 // fma(q, s, b) rounds exactly as the reference's mul-then-add does; f32
 // scales take a separate mul and add.
-// int8 weights are exact in f16; their per-row scale is applied in the epilogue
-// (y = acc * s, cpu_kernels.rs:130).
 //
 // Tiling: 256 threads = 4 waves in a 2x2 grid; block tile 128x128, wave tile
 // 64x64 = 4x4 v_mfma_f32_16x16x32_f16 tiles; BK = 64 per LDS stage.  The next
@@ -63,35 +61,21 @@ __device__ __forceinline__ h8_t dequant_word_f16(uint32_t w, float s, float b)
     return h;
 }
 
-__device__ __forceinline__ h8_t int8_to_f16x8(u2_t w)
-{
-    const uint32_t mlo = 0x00FF00FFu, magic = 0x64006400u;
-    const h2_t off = {(_Float16)1152.0f, (_Float16)1152.0f};
-    uint32_t b0 = w[0] ^ 0x80808080u, b1 = w[1] ^ 0x80808080u;
-    // (1152+w0, 1152+w2), (1152+w1, 1152+w3): exact in f16; subtracting 1152 is exact
-    h2_t a0 = as_h2(and_or(b0, mlo, magic)) - off;
-    h2_t a1 = as_h2(and_or(b0 >> 8, mlo, magic)) - off;
-    h2_t a2 = as_h2(and_or(b1, mlo, magic)) - off;
-    h2_t a3 = as_h2(and_or(b1 >> 8, mlo, magic)) - off;
-    h8_t h = {a0[0], a1[0], a0[1], a1[1], a2[0], a3[0], a2[1], a3[1]};
-    return h;
-}
-
 // One K stage (BK = 64) of global data held in registers by one thread:
 // its 32-element halves of one X row and one W row, plus the W row's scale
 // and bias bits for that group (raw, converted when the tile is stored).
 struct StageRegs {
     u4_t x[4];
-    u4_t w0, w1;  // q4: w0 = 32 nibbles; int8: w0, w1 = 32 bytes
+    u4_t w;  // 32 nibbles
     uint32_t s, b;
 };
 
-// WT: 0 = q4 affine (u32 words), 1 = int8.  NS = register prefetch depth.
-template <int WT, int SBT, int NS>
+// q4 affine (u32 words).  NS = register prefetch depth.
+template <int SBT, int NS>
 __global__ __launch_bounds__(kThreads) void qgemm_kernel(const void* __restrict__ W, const void* __restrict__ S,
                                                          const void* __restrict__ Bz, int group_size,
                                                          const _Float16* __restrict__ X, float* __restrict__ Y,
-                                                         int M, int N, int K, int k_per_split, int per_channel)
+                                                         int M, int N, int K, int k_per_split)
 {
     // two LDS buffers: stage s is stored into buffer s&1 while no wave can
     // still read it (every wave passed the barrier after its compute of s-2)
@@ -120,15 +104,10 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const void* __restrict_
         const int kc = kbeg + min(step, nsteps - 1) * BK + ld_half * 32;  // clamped: tail slots reload the last stage
 #pragma unroll
         for (int i = 0; i < 4; ++i) r.x[i] = *reinterpret_cast<const u4_t*>(X + (size_t)xm * K + kc + i * 8);
-        if constexpr (WT == 0) {
-            r.w0 = __builtin_nontemporal_load(w4 + ((size_t)wn_row * K + kc) / 32);
-            const size_t gi = (size_t)wn_row * gpr + (kc >> gshift);
-            r.s = load_raw<SBT>(S, gi);
-            r.b = load_raw<SBT>(Bz, gi);
-        } else {
-            r.w0 = __builtin_nontemporal_load(w4 + ((size_t)wn_row * K + kc) / 16);
-            r.w1 = __builtin_nontemporal_load(w4 + ((size_t)wn_row * K + kc) / 16 + 1);
-        }
+        r.w = __builtin_nontemporal_load(w4 + ((size_t)wn_row * K + kc) / 32);
+        const size_t gi = (size_t)wn_row * gpr + (kc >> gshift);
+        r.s = load_raw<SBT>(S, gi);
+        r.b = load_raw<SBT>(Bz, gi);
     };
 
     auto store_stage = [&](const StageRegs& r, int buf) {
@@ -136,16 +115,9 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const void* __restrict_
 #pragma unroll
         for (int i = 0; i < 4; ++i) *reinterpret_cast<u4_t*>(xd + i * 8) = r.x[i];
         _Float16* wd = ws[buf] + ld_row * LDS_STRIDE + ld_half * 32;
-        if constexpr (WT == 0) {
-            const float sc = raw_to_f32<SBT>(r.s), bi = raw_to_f32<SBT>(r.b);
+        const float sc = raw_to_f32<SBT>(r.s), bi = raw_to_f32<SBT>(r.b);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) *reinterpret_cast<h8_t*>(wd + i * 8) = dequant_word_f16<SBT>(r.w0[i], sc, bi);
-        } else {
-            *reinterpret_cast<h8_t*>(wd + 0) = int8_to_f16x8(u2_t{r.w0[0], r.w0[1]});
-            *reinterpret_cast<h8_t*>(wd + 8) = int8_to_f16x8(u2_t{r.w0[2], r.w0[3]});
-            *reinterpret_cast<h8_t*>(wd + 16) = int8_to_f16x8(u2_t{r.w1[0], r.w1[1]});
-            *reinterpret_cast<h8_t*>(wd + 24) = int8_to_f16x8(u2_t{r.w1[2], r.w1[3]});
-        }
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<h8_t*>(wd + i * 8) = dequant_word_f16<SBT>(r.w[i], sc, bi);
     };
 
     f4_t acc[4][4];
@@ -214,52 +186,35 @@ __global__ __launch_bounds__(kThreads) void qgemm_kernel(const void* __restrict_
     for (int j = 0; j < 4; ++j) {
         const int n = n0 + wn * 64 + j * 16 + ccol;
         if (n >= N) continue;
-        float s = 1.0f;
-        if constexpr (WT == 1) s = load_f32<SBT>(S, per_channel ? (size_t)n : 0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int m = m0 + wm * 64 + i * 16 + crow + e;
-                if (m < M) out[(size_t)m * N + n] = acc[i][j][e] * s;
+                if (m < M) out[(size_t)m * N + n] = acc[i][j][e];
             }
         }
     }
 }
 
-// Sum split-K partials [splits][M*N] in split order, then add the optional bias.
-__global__ void splitk_reduce_kernel(const float* __restrict__ part, float* __restrict__ y, const float* __restrict__ bias,
-                                     int splits, int M, int N)
+// Sum split-K partials [splits][M*N] in split order.
+__global__ void splitk_reduce_kernel(const float* __restrict__ part, float* __restrict__ y, int splits, int M, int N)
 {
     const size_t total = (size_t)M * N;
     if ((N & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
         // four columns of one row per thread: 16-byte loads of every split's partials
         const size_t n4 = total >> 2;
         for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
-            f4_t v = sum_splits_f4(reinterpret_cast<const f4_t*>(part) + i, n4, splits);
-            if (bias) {
-                const size_t n = (4 * i) % (size_t)N;
-                v += f4_t{bias[n], bias[n + 1], bias[n + 2], bias[n + 3]};
-            }
-            reinterpret_cast<f4_t*>(y)[i] = v;
+            reinterpret_cast<f4_t*>(y)[i] = sum_splits_f4(reinterpret_cast<const f4_t*>(part) + i, n4, splits);
         }
         return;
     }
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         float v = part[i];
         for (int s = 1; s < splits; ++s) v += part[(size_t)s * total + i];
-        if (bias) v += bias[i % N];
         y[i] = v;
     }
 }
-
-__global__ void add_bias_kernel(float* __restrict__ y, const float* __restrict__ bias, int M, int N)
-{
-    const size_t total = (size_t)M * N;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x)
-        y[i] += bias[i % N];
-}
-
 
 // ---------------------------------------------------------------------------
 // Direct-to-LDS helpers for the q4 qGEMM below (K % 128 == 0): LDS tiles hold
@@ -536,12 +491,10 @@ int qgemm_splits(int M, int N, int K)
     return splits;
 }
 
-size_t qgemm_workspace_bytes(int wt, int M, int N, int K, int group_size, int sbt)
+size_t qgemm_workspace_bytes(int M, int N, int K, int group_size, int sbt)
 {
-    if (wt == 0) {
-        const dma::Plan p = dma::plan(M, N, K, group_size, sbt, dma::kRegFixedLds);
-        if (p.splits > 0) return p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
-    }
+    const dma::Plan p = dma::plan(M, N, K, group_size, sbt, dma::kRegFixedLds);
+    if (p.splits > 0) return p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
     const int splits = qgemm_splits(M, N, K);
     return splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
 }
@@ -579,10 +532,9 @@ static hipError_t launch_q4_regw(const dma::Plan& p, const uint32_t* wq, const v
     return hipGetLastError();
 }
 
-template <int WT>
 static hipError_t launch_qgemm_common(const void* W, const void* S, const void* B, int sbt, int group_size,
-                                      int per_channel, const _Float16* X, float* Y, const float* bias, int M, int N,
-                                      int K, float* workspace, hipStream_t st)
+                                      const _Float16* X, float* Y, int M, int N, int K, float* workspace,
+                                      hipStream_t st)
 {
     const int splits = workspace ? qgemm_splits(M, N, K) : 1;
     const int ksteps = (K + BK - 1) / BK;
@@ -590,8 +542,8 @@ static hipError_t launch_qgemm_common(const void* W, const void* S, const void* 
     const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM, splits);
     float* out = splits > 1 ? workspace : Y;
 #define CELLM_QGEMM(SBT_)                                                                                          \
-    hipLaunchKernelGGL((qgemm_kernel<WT, SBT_, kStages>), grid, dim3(kThreads), 0, st, W, S, B, group_size, X, out, M, N, K, \
-                       k_per_split, per_channel)
+    hipLaunchKernelGGL((qgemm_kernel<SBT_, kStages>), grid, dim3(kThreads), 0, st, W, S, B, group_size, X, out, M, N, K, \
+                       k_per_split)
     if (sbt == DT_F32) CELLM_QGEMM(DT_F32);
     else if (sbt == DT_F16) CELLM_QGEMM(DT_F16);
     else CELLM_QGEMM(DT_BF16);
@@ -602,10 +554,7 @@ static hipError_t launch_qgemm_common(const void* W, const void* S, const void* 
     unsigned blocks = (unsigned)((total + 255) / 256);
     if (blocks > 4096) blocks = 4096;
     if (splits > 1) {
-        hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, workspace, Y, bias, splits, M, N);
-        e = hipGetLastError();
-    } else if (bias) {
-        hipLaunchKernelGGL(add_bias_kernel, dim3(blocks), dim3(256), 0, st, Y, bias, M, N);
+        hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, workspace, Y, splits, M, N);
         e = hipGetLastError();
     }
     return e;
@@ -628,17 +577,10 @@ hipError_t launch_qgemm_q4_affine_ws(const uint32_t* wq, const void* S, const vo
         const size_t total = (size_t)M * N;
         unsigned blocks = (unsigned)((total + 255) / 256);
         if (blocks > 4096) blocks = 4096;
-        hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, workspace, y, nullptr, p.splits, M,
-                           N);
+        hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, st, workspace, y, p.splits, M, N);
         return hipGetLastError();
     }
-    return launch_qgemm_common<0>(wq, S, B, sbt, group_size, 1, x, y, nullptr, M, N, K, workspace, st);
-}
-
-hipError_t launch_qgemm_i8_ws(const int8_t* w, const void* S, int sdt, int per_channel, const _Float16* x,
-                              const float* bias, float* y, int M, int N, int K, float* workspace, hipStream_t st)
-{
-    return launch_qgemm_common<1>(w, S, nullptr, sdt, 64, per_channel, x, y, bias, M, N, K, workspace, st);
+    return launch_qgemm_common(wq, S, B, sbt, group_size, x, y, M, N, K, workspace, st);
 }
 
 }  // namespace cellm

@@ -695,7 +695,7 @@ bool qgemm_exact_supported(const XgCall& c, int M, int K)
 {
     const bool nibbles = c.fmt == XG_I4 || c.fmt == XG_Q4;
     // weight rows start on 16-byte boundaries; a K step has one scale
-    if (M < 5 || K <= 0 || K % (nibbles ? 32 : c.fmt == XG_I8 ? 16 : 8) != 0) return false;
+    if (M < (c.x_f16 ? 1 : 5) || K <= 0 || K % (nibbles ? 32 : c.fmt == XG_I8 ? 16 : 8) != 0) return false;
     if (c.fmt == XG_Q4 && (c.group <= 0 || c.group % kBK != 0)) return false;
     if (c.x_f16 && c.fmt != XG_I8) return false;
     if (c.act >= 0 && (c.fmt == XG_F16 || c.nseg != 2 || c.segs[0].n != c.segs[1].n)) return false;

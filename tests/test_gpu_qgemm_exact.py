@@ -315,3 +315,45 @@ def test_gate_up_non_finite(ops, k):
     assert np.array_equal(torch.isposinf(got).numpy(), torch.isposinf(ref).numpy())
     assert np.array_equal(torch.isneginf(got).numpy(), torch.isneginf(ref).numpy())
     assert _rel(got[4:], _act(g[4:].double(), u[4:].double(), "silu")) <= 1e-5  # against f32 sums
+
+
+# f16 activations over int8: products are exact, one f32 chain over K (a rounding per 8 or 16 products):
+# sqrt(K / 8) * 2^-24 is 1.9e-6 at K = 8192
+@pytest.mark.parametrize("m,n,k", SIZES + [(70, 300, 8192), (2049, 6200, 192), (129, 64, 64)])
+@pytest.mark.parametrize("sdt", [torch.float32, torch.bfloat16])
+def test_i8_f16_rows(ops, m, n, k, sdt):
+    x = _x(m, k, m * 7 + k).half()
+    w, s = _i8(n, k, n * 3 + k)
+    s = s.to(sdt)
+    bias = torch.randn(n, generator=torch.Generator().manual_seed(n))
+    ref = x.double() @ w.double().t() * s.double() + bias.double()
+    y = torch.full((m, n), float("nan"), device="cuda")
+    ops.encode_qgemv_i8(w.cuda(), s.cuda(), x.cuda(), y, bias=bias.cuda())
+    torch.cuda.synchronize()
+    assert _rel(y.cpu(), ref) <= 2e-6
+    if k % 64 == 0:  # the qGEMM entry point takes any number of rows
+        for rows in (1, m):
+            y.fill_(float("nan"))
+            ops.encode_qgemm_i8(w.cuda(), s.cuda(), x[:rows].cuda(), y[:rows], bias=bias.cuda())
+            torch.cuda.synchronize()
+            assert _rel(y[:rows].cpu(), ref[:rows]) <= 2e-6
+
+
+@pytest.mark.parametrize("m,rq,rkv,k", [s for s in QKV if s[0] > 64])
+def test_qkv_and_gate_up_f16_rows(ops, m, rq, rkv, k):
+    x = _x(m, k, m + k).half()
+    rows = (rq, rkv, rkv)
+    w = [_i8(r, k, 7 + i) for i, r in enumerate(rows)]
+    y = [torch.full((m, r), float("nan"), device="cuda") for r in rows]
+    ops.encode_qkv_i8(*[t.cuda() for ws in w for t in ws], x.cuda(), *y)
+    torch.cuda.synchronize()
+    for i in range(3):
+        assert _rel(y[i].cpu(), x.double() @ w[i][0].double().t() * w[i][1].double()) <= 2e-6, i
+    x = (x * 0.3).half()
+    (wg, sg), (wu, su) = _i8(rq, k, 1), _i8(rq, k, 2)
+    sg, su = sg * 0.02, su * 0.02
+    h = torch.full((m, rq), float("nan"), device="cuda")
+    ops.encode_gate_up_silu_i8(wg.cuda(), sg.cuda(), wu.cuda(), su.cuda(), x.cuda(), h)
+    torch.cuda.synchronize()
+    g, u = (x.double() @ t.double().t() * s.double() for t, s in ((wg, sg), (wu, su)))
+    assert _rel(h.cpu(), _act(g, u, "silu")) <= 4e-6
