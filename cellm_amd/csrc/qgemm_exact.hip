@@ -635,7 +635,9 @@ XgPlan xg_plan(int fmt, int P, const XgSeg* segs, int nseg, bool act, int M, int
         blocks = p.form ? tiles(P == 2 ? 64 : 128, 128) : tiles(32, 128);
     }
     int splits = 1;
-    const int64_t want = p.form == 2 ? 256 : 512;
+    // f16 x: a second block per CU does not pay for the split sums (2048 rows of 2048 -> 2048 34.5 us unsplit on
+    // 256 blocks, 43.0 split in two); f32 x: it does or is even (512 rows of 960 -> 960 20.0 against 20.3)
+    const int64_t want = p.form == 2 || P == 1 ? 256 : 512;
     while (blocks * splits * 2 <= want && steps / (splits * 2) >= 4) splits *= 2;
     p.steps_per_split = (steps + splits - 1) / splits;
     p.splits = (steps + p.steps_per_split - 1) / p.steps_per_split;
