@@ -1836,6 +1836,20 @@ hipError_t launch_attention_gqa_f16kv(const float* q, const uint16_t* kcache, co
     const bool one_launch = rows * n_kv_heads <= kAttnCounters;
     const int cap = max_blocks * tokens_per_block;
     const dim3 hgrid((unsigned)(rows * n_heads));
+    // The MFMA kernel reads K and V once for all query vectors that share them and starts later than the
+    // others (8 us at any size): it takes the calls with much to read, and long contexts, whose many 64-position
+    // chunks cost the split form's last block.  Measured, us, vector kernels / MFMA (rows, heads / kv heads,
+    // head_dim, positions): 16, 15/5, 64, 512: 8.4 / 12.5; 64, 14/2, 64, 512: 20.0 / 13.9; 16, 32/8, 128, 512:
+    // 24.6 / 17.9; 4, 15/5, 64, 2048: 13.2 / 15.2; 16, 32/8, 128, 2048: 43.5 / 32.3; 1, 14/2, 64, 16384: 32.8 /
+    // 17.9; 8, 32/8, 128, window 512 of 4096: 14.6 / 20.9; prompts of 64 and 512 tokens, 14/2, 64: 11.0 / 8.8 and
+    // 90 / 15.
+    const double reads = (double)rows * n_heads * head_dim * (window > 0 ? std::min(window, cap) : cap);
+    const bool vec16 = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kcache) |
+                         reinterpret_cast<uintptr_t>(vcache) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+    if (vec16 && (reads >= (rows >= 32 ? 3e6 : 20e6) || (window == 0 && cap >= 8192)))
+        return launch_attention_mma(q, kcache, vcache, block_tables, max_blocks, total_blocks, pos, rows, n_heads,
+                                    n_kv_heads, head_dim, n_layers, tokens_per_block, layer, scale, soft_cap, window,
+                                    one_launch && cap > 2 * kAttnBlockSub ? 64 : 1, part, counters, out, st);
     auto go = [&](auto hd, auto g) {
         constexpr int HD = decltype(hd)::value, GG = decltype(g)::value;
         // caches of up to 512 positions: the whole sequence in one block per query head

@@ -1,0 +1,153 @@
+"""The MFMA attention (attention.hip) against 64-bit results, at the sizes where it
+chooses between shared tiles, single rows and splits.
+
+The bar, 2e-6 in the 2-norm: scores are f32 dot products (a few 2^-24 of |q||k|,
+here up to 10 * 6e-8 in the exponent), weights and V products f32 sums; the
+measured error is 2e-7 to 4e-7."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-6
+
+
+def _cache(total, layers, tpb, nkv, hd, seed):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(total, layers, tpb, nkv, hd, generator=g).half() for _ in range(2)]
+
+
+def _reference(q, kc, vc, bt, pos, layer, scale=None, cap=0.0, window=0):
+    """f64; a missing page counts as zero keys and values."""
+    rows, nh, hd = q.shape
+    total, _, tpb, nkv, _ = kc.shape
+    out = torch.zeros(rows, nh, hd, dtype=torch.float64)
+    for r in range(rows):
+        seq = min(int(pos[r]) + 1, bt.shape[1] * tpb)
+        if seq <= 0:
+            continue
+        t = torch.arange(max(seq - window, 0) if window else 0, seq)
+        blk = bt[r][t // tpb].long()
+        there = (blk < total)[:, None, None]
+        k, v = (torch.where(there, c[blk.clamp(max=total - 1), layer, t % tpb], 0.0).double() for c in (kc, vc))
+        g = nh // nkv
+        for h in range(nh):
+            s = (k[:, h // g] @ q[r, h].double()) * (scale or 1 / math.sqrt(hd))
+            if cap:
+                s = torch.tanh(s / cap) * cap
+            out[r, h] = torch.softmax(s, 0) @ v[:, h // g]
+    return out
+
+
+def _run(ops, q, kc, vc, bt, pos, layer, **kw):
+    rows, nh, hd = q.shape
+    total, layers, tpb, nkv, _ = kc.shape
+    out = torch.full((rows, nh * hd), 7.0, device="cuda")
+    ops.encode_attention(q.reshape(rows, -1).cuda(), kc.cuda(), vc.cuda(), bt.to(torch.int32).cuda(),
+                         pos.to(torch.int32).cuda(), out, nh, nkv, hd, total, layers, tpb, layer, **kw)
+    torch.cuda.synchronize()
+    return out.cpu().view(rows, nh, hd)
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+# rows, heads, kv heads, head_dim, tokens per page: tiles of 16 rows with full and short last tiles (fewer rows
+# than heads per kv head among them), every group size, pages of odd sizes
+@pytest.mark.parametrize("rows,nh,nkv,hd,tpb", [(32, 14, 2, 64, 16), (33, 16, 2, 128, 16), (50, 5, 5, 64, 5),
+                                                (47, 12, 4, 64, 32), (100, 10, 2, 64, 7), (64, 6, 3, 128, 16),
+                                                (35, 8, 1, 128, 3), (40, 12, 2, 64, 16)])
+def test_prompt_rows_share_pages(ops, rows, nh, nkv, hd, tpb):
+    past = 1 + int(3.2e6 / (rows * nh * hd))  # positions before the prompt: enough for the MFMA form
+    n = past + rows
+    per = -(-n // tpb)
+    g = torch.Generator().manual_seed(rows)
+    kc, vc = _cache(per + 3, 2, tpb, nkv, hd, rows)
+    bt = (torch.randperm(per + 3, generator=g)[:per])[None].repeat(rows, 1)
+    pos = torch.arange(past, n)
+    q = torch.randn(rows, nh, hd, generator=g) * 1.5
+    for kw in ({}, dict(window=33), dict(soft_cap=5.0, attn_scale=0.2)):
+        got = _run(ops, q, kc, vc, bt, pos, 1, **kw)
+        ref = _reference(q, kc, vc, bt, pos, 1, kw.get("attn_scale"), kw.get("soft_cap", 0.0), kw.get("window", 0))
+        assert _rel(got, ref) <= TOL, kw
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_mixed_tiles(ops, seed):
+    """Rows of one tile with equal tables, tables that part after the first page, pages of their own, missing
+    pages, positions out of order, and rows without a position (their output is left as it was)."""
+    rows, nh, nkv, hd, tpb, per = 53, 6, 2, 64, 4, 48
+    g = torch.Generator().manual_seed(seed)
+    total = 400
+    kc, vc = _cache(total, 1, tpb, nkv, hd, seed)
+    base = torch.randperm(total, generator=g)[:per]
+    bt = base[None].repeat(rows, 1)
+    for r in range(rows):
+        kind = int(torch.randint(0, 5, (1,), generator=g)) if r < 48 else 0
+        if kind == 1:
+            bt[r, 1 + r % 40:] = torch.randperm(total, generator=g)[:per - 1 - r % 40]
+        elif kind == 2:
+            bt[r] = torch.randperm(total, generator=g)[:per]
+        elif kind == 3:
+            bt[r, r % per] = total + 5
+    pos = torch.randint(-1, per * tpb, (rows,), generator=g)
+    pos[7] = -1
+    pos[9] = per * tpb + 50  # past the table: the table's positions
+    q = torch.randn(rows, nh, hd, generator=g)
+    got = _run(ops, q, kc, vc, bt, pos, 0)
+    ref = _reference(q, kc, vc, bt, pos, 0)
+    none = pos < 0
+    assert bool((got[none] == 7.0).all())
+    assert _rel(got[~none], ref[~none]) <= TOL
+
+
+# sessions with pages of their own, split over positions: one split, several, contexts that end inside the first
+@pytest.mark.parametrize("rows,nh,nkv,hd,ctx", [(1, 8, 1, 64, 8192), (3, 32, 8, 128, 2100), (16, 16, 2, 128, 1300),
+                                                (40, 8, 8, 64, 1030), (2, 4, 4, 128, 9000)])
+def test_long_contexts_in_splits(ops, rows, nh, nkv, hd, ctx):
+    tpb = 16
+    per = -(-ctx // tpb)
+    g = torch.Generator().manual_seed(ctx)
+    kc, vc = _cache(per * rows, 1, tpb, nkv, hd, ctx)
+    bt = torch.randperm(per * rows, generator=g).view(rows, per)
+    pos = torch.randint(ctx // 2, ctx, (rows,), generator=g)
+    if rows > 2:
+        pos[0], pos[1] = 0, 511
+    q = torch.randn(rows, nh, hd, generator=g)
+    for _ in range(2):  # the counters are back at zero
+        assert _rel(_run(ops, q, kc, vc, bt, pos, 0), _reference(q, kc, vc, bt, pos, 0)) <= TOL
+
+
+@pytest.mark.parametrize("rows,ctx", [(40, 320), (2, 8192)])  # a shared tile; splits
+def test_non_finite_keys_values_and_queries(ops, rows, ctx):
+    """An infinite or NaN element reaches the outputs it reaches in a plain f32 softmax: a key of -inf score has
+    weight 0, and an infinite value its sign."""
+    nh, nkv, hd, tpb = 8, 2, 64, 16
+    per = ctx // tpb
+    g = torch.Generator().manual_seed(1)
+    kc, vc = _cache(per, 1, tpb, nkv, hd, 2)
+    bt = torch.arange(per)[None].repeat(rows, 1)
+    pos = torch.full((rows,), ctx - 1)
+    q = torch.randn(rows, nh, hd, generator=g)
+    q[:, :, 0] = q[:, :, 0].abs() + 0.5
+    kc[0, 0, 3, 0, 0] = float("-inf")      # weight 0 for every query of kv head 0
+    vc[0, 0, 5, 0, 1] = float("inf")       # value +inf in dim 1 of kv head 0
+    vc[0, 0, 6, 1, 2] = float("nan")
+    q[1, 5] = float("nan")
+    got = _run(ops, q, kc, vc, bt, pos, 0)
+    ref = torch.zeros_like(got)
+    for h in range(nh):
+        k, v = (c[bt[0], 0].reshape(-1, nkv, hd)[:, h // 4].float() for c in (kc, vc))
+        s = (q[:, h, None, :] * k[None]).sum(2) / 8.0
+        p = torch.exp(s - s.max(1, keepdim=True).values)
+        ref[:, h] = (p @ v) / p.sum(1, keepdim=True)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.isinf(got), torch.isinf(ref))
+    fine = torch.isfinite(ref)
+    assert bool((got[:, :4, 1] == float("inf")).all())
+    assert _rel(got[fine], ref[fine].double()) <= 5e-6  # the reference here is f32 too
