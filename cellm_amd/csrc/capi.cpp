@@ -243,7 +243,7 @@ int32_t try_qgemm_exact(cellm_hip_ctx* ctx, const XgCall& c, int64_t m, int64_t 
     *done = false;
     if (!qgemm_exact_supported(c, (int)m, (int)k)) return CELLM_HIP_OK;
     const size_t need = qgemm_exact_workspace_bytes(c, (int)m, (int)k);
-    const bool in_place = c.x_f16 && k % 64 == 0;
+    const bool in_place = c.x_f16 && c.fmt == XG_I8 && k % 64 == 0;
     if (need && !in_place && capturing(st)) return CELLM_HIP_OK;
     float* ws = nullptr;
     const int32_t rc = get_workspace(ctx, st, need, &ws);
@@ -504,10 +504,18 @@ int32_t gate_up_q4_impl(cellm_hip_ctx* ctx, const uint32_t* wg, const void* sg, 
                 "qgemv_q4 gate/up launch");
         return CELLM_HIP_OK;
     }
-    if (xdt == DT_F32) {
+    if (xdt == DT_F16 && m > 64) {
+        const Q4FusedSeg fs[2] = {Q4FusedSeg{wg, sg, bg, nullptr, h, (int)n}, Q4FusedSeg{wu, su, bu, nullptr, nullptr, (int)n}};
+        const _Float16* xh = reinterpret_cast<const _Float16*>(x);
+        if (qgemm_q4_fused_supported(fs, 2, true, sbt, (int)group, xh, (int)m, (int)k)) {
+            HIP_TRY(launch_qgemm_q4_fused(fs, 2, act, sbt, (int)group, xh, (int)m, (int)k, st), "qgemm_q4 gate/up launch");
+            return CELLM_HIP_OK;
+        }
+    }
+    if (xdt == DT_F32 || (xdt == DT_F16 && (m > 64 ? k % 128 != 0 : k % 64 != 0))) {
         const XgSeg xs[2] = {XgSeg{wg, nullptr, nullptr, h, (int)n, 0, sg, bg},
                              XgSeg{wu, nullptr, nullptr, nullptr, (int)n, 0, su, bu}};
-        const XgCall call{XG_Q4, xs, 2, sbt, x, false, act, (int)group, (int)((k + group - 1) / group)};
+        const XgCall call{XG_Q4, xs, 2, sbt, x, xdt == DT_F16, act, (int)group, (int)((k + group - 1) / group)};
         bool done = false;
         if (int32_t rc = try_qgemm_exact(ctx, call, m, k, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;
@@ -863,10 +871,17 @@ int32_t cellm_hip_qgemv_q4_affine_qkv(cellm_hip_ctx_t* ctx, const uint32_t* wq, 
                 "qgemv_q4_qkv launch");
         return CELLM_HIP_OK;
     }
-    if (x_dtype == DT_F32) {
+    if (x_dtype == DT_F16 && m > 64) {
+        const _Float16* xh = reinterpret_cast<const _Float16*>(x);
+        if (qgemm_q4_fused_supported(segs, 3, false, sb_dtype, (int)group, xh, (int)m, (int)cols)) {
+            HIP_TRY(launch_qgemm_q4_fused(segs, 3, -1, sb_dtype, (int)group, xh, (int)m, (int)cols, st), "qgemm_q4_qkv launch");
+            return CELLM_HIP_OK;
+        }
+    }
+    if (x_dtype == DT_F32 || (x_dtype == DT_F16 && (m > 64 ? cols % 128 != 0 : cols % 64 != 0))) {
         XgSeg xs[3];
         for (int i = 0; i < 3; ++i) xs[i] = XgSeg{w[i], nullptr, pb[i], y[i], (int)rows[i], 0, s[i], b[i]};
-        const XgCall call{XG_Q4, xs, 3, sb_dtype, x, false, -1, (int)group, (int)((cols + group - 1) / group)};
+        const XgCall call{XG_Q4, xs, 3, sb_dtype, x, x_dtype == DT_F16, -1, (int)group, (int)((cols + group - 1) / group)};
         bool done = false;
         if (int32_t rc = try_qgemm_exact(ctx, call, m, cols, st, &done)) return rc;
         if (done) return CELLM_HIP_OK;

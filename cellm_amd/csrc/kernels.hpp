@@ -82,6 +82,13 @@ hipError_t launch_qgemm_q4_affine_ws(const uint32_t* wq, const void* S, const vo
                                      const _Float16* x, float* y, int M, int N, int K, float* workspace,
                                      hipStream_t st);
 
+// Several q4 matrices over one f16 x in one launch, or (act >= 0, two matrices) act(seg 0) * seg 1 into seg 0's
+// y; f16 weight tiles as launch_qgemm_q4_affine_ws, K % 128 == 0, no workspace.
+bool qgemm_q4_fused_supported(const Q4FusedSeg* segs, int nseg, bool act, int sbt, int group, const _Float16* x, int M,
+                              int K);
+hipError_t launch_qgemm_q4_fused(const Q4FusedSeg* segs, int nseg, int act, int sbt, int group, const _Float16* x, int M,
+                                 int K, hipStream_t st);
+
 // Multi-row GEMM, weights exact in f16 (qgemm_exact.hip): f32 x at M >= 5 (and rows enough to pay for its
 // launches), or f16 x over int8; 16-byte aligned W, x and weight rows.  Up to three matrices share x.  `ws` holds
 // x's f16 parts and the split sums.

@@ -266,14 +266,26 @@ constexpr int kRegStageBytes = kStageHalves * 2 + kRawStepBytes;    // 40 KB
 constexpr size_t kRegFixedLds = (size_t)kRegStages * kRegStageBytes;
 constexpr size_t kRegExchangeBytes = 8 * 2 * 16 * 64 * 4;  // k-half exchange after the loop (64 KB)
 
-template <int SBT>
-__global__ __launch_bounds__(kRegThreads) void qgemm_q4_regw_kernel(const uint32_t* __restrict__ W,
-                                                                   const void* __restrict__ S,
-                                                                   const void* __restrict__ Bz, int gshift,
-                                                                   const _Float16* __restrict__ X,
-                                                                   float* __restrict__ out, int M, int N, int K,
-                                                                   int k_per_split)
+struct RegArgs {
+    Q4FusedSeg seg[3];
+    int tile0[3];  // first column tile of each segment; of an absent one, past every tile
+    int gshift, M, K, k_per_split, act;
+    const _Float16* X;
+    float* part;   // split sums [split][M][N] of the one segment, or nullptr
+};
+
+// REG_MANY: up to three matrices share X, column tiles of one grid, with their biases.  REG_ACT: segments 0 and 1
+// are gate and up, a tile's four 32-column slices are gate, up, gate, up of the same 64 outputs, and
+// h = act(gate) * up leaves the tile (both unsplit only).  At 512 rows of 896, 2 x 4864 columns took 13.2 us twice
+// and 5 us for the activation over three f32 matrices, now 26.3 (304 tiles are two rounds of 256 blocks); q/k/v of
+// 896 and 2 x 16 columns 32.2 -> 11.6.  One matrix has an instance of its own, without the selects and the bias:
+// with them 10.9 -> 11.3 us at 512 x 896 x 896.
+enum RegMode { REG_ONE, REG_MANY, REG_ACT };
+
+template <int SBT, RegMode MODE>
+__global__ __launch_bounds__(kRegThreads) void qgemm_q4_regw_kernel(const RegArgs a)
 {
+    constexpr bool ACT = MODE == REG_ACT;
     extern __shared__ __align__(16) unsigned char smem[];
     // stage t: X tile at t * kRegStageBytes, W raw at + kStageHalves * 2; then the scales/biases
     uint32_t* sbl = reinterpret_cast<uint32_t*>(smem + kRegFixedLds);  // [BN][groups] as in the DMA kernel
@@ -282,11 +294,28 @@ __global__ __launch_bounds__(kRegThreads) void qgemm_q4_regw_kernel(const uint32
     const int tid = threadIdx.x, lane = tid & 63, wn = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kh = wn >> 2, ns = wn & 3;
     const int r32 = lane & 31, h32 = lane >> 5;
-    const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
-    const int kbeg = blockIdx.z * k_per_split;
-    const int kend = min(K, kbeg + k_per_split);
+    const int M = a.M, K = a.K, gshift = a.gshift, vt = blockIdx.x;
+    // selects between arguments that are all loaded at once, not a chain of loads through an index
+    const Q4FusedSeg su = a.seg[1];
+    Q4FusedSeg sg = a.seg[0];
+    int tile0 = 0;
+    if constexpr (MODE == REG_MANY) {
+        const Q4FusedSeg s2 = a.seg[2];
+        const int t1 = a.tile0[1], t2 = a.tile0[2];
+        const bool c1 = vt >= t1, c2 = vt >= t2;
+        const auto pick = [&](auto x0, auto x1, auto x2) { return c2 ? x2 : c1 ? x1 : x0; };
+        sg = Q4FusedSeg{pick(sg.w, su.w, s2.w),    pick(sg.S, su.S, s2.S), pick(sg.B, su.B, s2.B),
+                        pick(sg.bias, su.bias, s2.bias), pick(sg.y, su.y, s2.y), pick(sg.n, su.n, s2.n)};
+        tile0 = pick(0, t1, t2);
+    }
+    const int N = sg.n;
+    const int n0 = ACT ? vt * (BN / 2) : (vt - tile0) * BN, m0 = blockIdx.y * BM;
+    // tile column -> matrix column past n0
+    const auto column = [](int c) { return ACT ? (c >> 6) * 32 + (c & 31) : c; };
+    const int kbeg = blockIdx.z * a.k_per_split;
+    const int kend = min(K, kbeg + a.k_per_split);
     const int nsteps = (kend - kbeg) / BK;
-    float* o = out + (size_t)blockIdx.z * M * N;
+    float* o = a.part ? a.part + (size_t)blockIdx.z * M * N : sg.y;
     if (nsteps <= 0) return;  // the launcher never makes an empty split
     const int last = nsteps - 1;
     const int gpr = (K + (1 << gshift) - 1) >> gshift;
@@ -305,9 +334,9 @@ __global__ __launch_bounds__(kRegThreads) void qgemm_q4_regw_kernel(const uint32
     // W DMA: 1 per wave per stage, covering columns wn * 16 .. +16, 64 bytes each (columns past N
     // re-read the last one: computed, never stored); byte offsets from W + kbeg / 2
     const uint32_t woff =
-        (uint32_t)((size_t)min(n0 + wn * 16 + (lane >> 2), N - 1) * (K / 2) + 16 * (lane & 3));
-    const unsigned char* xbase = reinterpret_cast<const unsigned char*>(X) + (size_t)kbeg * 2;
-    const unsigned char* wbase = reinterpret_cast<const unsigned char*>(W) + kbeg / 2;
+        (uint32_t)((size_t)min(n0 + column(wn * 16 + (lane >> 2)), N - 1) * (K / 2) + 16 * (lane & 3));
+    const unsigned char* xbase = reinterpret_cast<const unsigned char*>(a.X) + (size_t)kbeg * 2;
+    const unsigned char* wbase = reinterpret_cast<const unsigned char*>(ACT && (wn & 2) ? su.w : sg.w) + kbeg / 2;
     const uint32_t lds0 = lds_addr(smem);
     auto issue = [&](int step) {
         const int sc = min(step, last), st = step % kRegStages;
@@ -330,9 +359,9 @@ __global__ __launch_bounds__(kRegThreads) void qgemm_q4_regw_kernel(const uint32
             for (int u = 0; u < PB; ++u) {
                 const int i = min(base + u * kRegThreads, total - 1);
                 const int col = i / ng, gi = i - col * ng;
-                const size_t idx = (size_t)min(n0 + col, N - 1) * gpr + g0 + gi;
-                sv[u] = load_raw<SBT>(S, idx);
-                bv[u] = load_raw<SBT>(Bz, idx);
+                const size_t idx = (size_t)min(n0 + column(col), N - 1) * gpr + g0 + gi;
+                sv[u] = load_raw<SBT>(ACT && (col & 32) ? su.S : sg.S, idx);
+                bv[u] = load_raw<SBT>(ACT && (col & 32) ? su.B : sg.B, idx);
             }
 #pragma unroll
             for (int u = 0; u < PB; ++u) {
@@ -408,9 +437,13 @@ __global__ __launch_bounds__(kRegThreads) void qgemm_q4_regw_kernel(const uint32
     // exchanges with lane l of the partner, 8 KB per wave.  All partner values are read before any
     // add or store (one LDS round trip instead of one per store).
     float* xch = reinterpret_cast<float*>(smem);
-    const int ncol = n0 + lcol;
+    const int ncol = n0 + column(lcol);
     auto finish = [&](auto keep_c) {
         constexpr int KEEP = decltype(keep_c)::value, GIVE = 2 - KEEP;  // constant indices: no scratch
+        // arrived before the stores: a load still pending there makes every guarded store wait for the one
+        // before it (10.9 against 14.0 us at 512 x 896 x 896)
+        float bias = MODE == REG_MANY && sg.bias ? sg.bias[min(ncol, N - 1)] : 0.0f;
+        asm volatile("" : "+v"(bias));
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -421,14 +454,43 @@ __global__ __launch_bounds__(kRegThreads) void qgemm_q4_regw_kernel(const uint32
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r) other[t][r] = xch[((((wn ^ 4) * 2 + t) * 16 + r) * 64) + lane];
+        if constexpr (ACT) {
+            // every wave's sums back to LDS, then half a gate tile and its up tile for each: the waves that hold
+            // the gate slices sit on two of the four SIMDs, which took 15.4 us at 65 x 896 x 2 x 896, this 12.9
+            float* mine = xch + kRegExchangeBytes / 4 + (size_t)wn * 2 * 16 * 64;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mine[(t * 16 + r) * 64 + lane] = acc[KEEP + t][r] + other[t][r];
+            __syncthreads();
+            const int t = ns & 1, n = n0 + (ns >> 1) * 32 + r32;
+            const float* gate = xch + kRegExchangeBytes / 4 + (size_t)((wn & ~1) * 2 + t) * 16 * 64 + lane;
+            const float* up = gate + 2 * 16 * 64;
+            if (n >= N) return;
+            const auto rows = [&](auto act) {
+#pragma unroll 8
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + (KEEP + t) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3);
+                    const float v = act_mul(decltype(act)::value, gate[r * 64], up[r * 64]);
+                    if (m < M) __builtin_nontemporal_store(v, o + (size_t)m * N + n);
+                }
+            };
+            if (a.act == ACT_GELU_TANH)
+                rows(std::integral_constant<int, ACT_GELU_TANH>{});
+            else
+                rows(std::integral_constant<int, ACT_SILU>{});
+            return;
+        }
         if (ncol >= N) return;
+        const bool biased = MODE == REG_MANY && sg.bias;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 // register r of a 32x32 tile: row (r/4)*8 + (lane/32)*4 + r%4, column lane%32
                 const int m = m0 + (KEEP + t) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3);
-                if (m < M) __builtin_nontemporal_store(acc[KEEP + t][r] + other[t][r], o + (size_t)m * N + ncol);
+                const float v = acc[KEEP + t][r] + other[t][r];
+                if (m < M) __builtin_nontemporal_store(biased ? v + bias : v, o + (size_t)m * N + ncol);
             }
     };
     if (kh == 0)
@@ -519,17 +581,67 @@ static hipError_t allow_lds(Kern kern, size_t bytes)
     return e;
 }
 
-template <int SBT>
-static hipError_t launch_q4_regw(const dma::Plan& p, const uint32_t* wq, const void* S, const void* B, int gshift,
-                                 const _Float16* x, float* out, int M, int N, int K, hipStream_t st)
+template <dma::RegMode MODE>
+static hipError_t launch_q4_regw(const dma::RegArgs& a, int sbt, int vtiles, int splits, size_t lds, hipStream_t st)
 {
-    auto kern = dma::qgemm_q4_regw_kernel<SBT>;
-    hipError_t e = allow_lds(kern, p.lds);
-    if (e != hipSuccess) return e;
-    const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM, p.splits);
-    hipLaunchKernelGGL(kern, grid, dim3(dma::kRegThreads), p.lds, st, wq, S, B, gshift, x, out, M, N, K,
-                       p.k_per_split);
-    return hipGetLastError();
+    auto go = [&](auto kern) {
+        const hipError_t e = allow_lds(kern, lds);
+        if (e != hipSuccess) return e;
+        const dim3 grid(vtiles, (a.M + BM - 1) / BM, splits);
+        hipLaunchKernelGGL(kern, grid, dim3(dma::kRegThreads), lds, st, a);
+        return hipGetLastError();
+    };
+    return sbt == DT_F16   ? go(dma::qgemm_q4_regw_kernel<DT_F16, MODE>)
+           : sbt == DT_F32 ? go(dma::qgemm_q4_regw_kernel<DT_F32, MODE>)
+                           : go(dma::qgemm_q4_regw_kernel<DT_BF16, MODE>);
+}
+
+// LDS of an unsplit tile, 0 if its scales and biases do not fit
+static size_t fused_lds(int K, int group, int sbt)
+{
+    const size_t lds = dma::kRegFixedLds + (size_t)BN * ((K + group - 1) / group) * (sbt == DT_F32 ? 8 : 4);
+    return lds <= dma::kMaxLds ? std::max(lds, dma::kRegExchangeBytes * 2) : 0;
+}
+
+bool qgemm_q4_fused_supported(const Q4FusedSeg* segs, int nseg, bool act, int sbt, int group, const _Float16* x, int M,
+                              int K)
+{
+    if (M < 1 || K <= 0 || K % dma::BK != 0 || group < 32 || (reinterpret_cast<uintptr_t>(x) & 15) != 0 ||
+        (uint64_t)M * K * 2 >= (1ull << 32) || !fused_lds(K, group, sbt) || (act && segs[0].n != segs[1].n))
+        return false;
+    int64_t tiles = 0;
+    for (int i = 0; i < nseg; ++i) {
+        if (segs[i].n <= 0 || (reinterpret_cast<uintptr_t>(segs[i].w) & 15) != 0 ||
+            (uint64_t)segs[i].n * K / 2 >= (1ull << 32))
+            return false;
+        tiles += (segs[i].n + BN - 1) / BN;
+    }
+    tiles *= (M + BM - 1) / BM;
+    // unsplit: 1.04 us per 128 k, against launches of their own with split sums where tiles are few
+    return K / dma::BK <= 20 || tiles >= 128;
+}
+
+hipError_t launch_qgemm_q4_fused(const Q4FusedSeg* segs, int nseg, int act, int sbt, int group, const _Float16* x, int M,
+                                 int K, hipStream_t st)
+{
+    dma::RegArgs a{};
+    int vtiles = 0;
+    for (int i = 0; i < 3; ++i) {
+        a.tile0[i] = i < nseg ? vtiles : INT32_MAX;
+        if (i >= nseg) continue;
+        a.seg[i] = segs[i];
+        vtiles += (segs[i].n + BN - 1) / BN;
+    }
+    if (act >= 0) vtiles = (segs[0].n + BN / 2 - 1) / (BN / 2);
+    a.gshift = __builtin_ctz((unsigned)group);
+    a.M = M;
+    a.K = K;
+    a.k_per_split = K;
+    a.act = act;
+    a.X = x;
+    const size_t lds = fused_lds(K, group, sbt);
+    return act >= 0 ? launch_q4_regw<dma::REG_ACT>(a, sbt, vtiles, 1, lds, st)
+                    : launch_q4_regw<dma::REG_MANY>(a, sbt, vtiles, 1, lds, st);
 }
 
 static hipError_t launch_qgemm_common(const void* W, const void* S, const void* B, int sbt, int group_size,
@@ -568,11 +680,16 @@ hipError_t launch_qgemm_q4_affine_ws(const uint32_t* wq, const void* S, const vo
     p.lds = std::max(p.lds, dma::kRegExchangeBytes);
     const bool offsets_fit = (uint64_t)M * K * 2 < (1ull << 32) && (uint64_t)N * K / 2 < (1ull << 32);
     if (p.splits > 0 && (p.splits == 1 || workspace) && offsets_fit) {
-        const int gshift = __builtin_ctz((unsigned)group_size);
-        float* out = p.splits > 1 ? workspace : y;
-        hipError_t e = sbt == DT_F16   ? launch_q4_regw<DT_F16>(p, wq, S, B, gshift, x, out, M, N, K, st)
-                       : sbt == DT_F32 ? launch_q4_regw<DT_F32>(p, wq, S, B, gshift, x, out, M, N, K, st)
-                                       : launch_q4_regw<DT_BF16>(p, wq, S, B, gshift, x, out, M, N, K, st);
+        dma::RegArgs a{};
+        a.seg[0] = Q4FusedSeg{wq, S, B, nullptr, y, N};
+        a.tile0[1] = a.tile0[2] = INT32_MAX;
+        a.gshift = __builtin_ctz((unsigned)group_size);
+        a.M = M;
+        a.K = K;
+        a.k_per_split = p.k_per_split;
+        a.X = x;
+        a.part = p.splits > 1 ? workspace : nullptr;
+        const hipError_t e = launch_q4_regw<dma::REG_ONE>(a, sbt, (N + BN - 1) / BN, p.splits, p.lds, st);
         if (e != hipSuccess || p.splits == 1) return e;
         const size_t total = (size_t)M * N;
         unsigned blocks = (unsigned)((total + 255) / 256);

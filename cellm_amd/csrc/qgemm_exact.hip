@@ -64,8 +64,7 @@ constexpr int kBK = 64;
 
 struct XgArgs {
     XgSeg seg[3];
-    int tile0[3];  // first column tile of each segment
-    int nseg;
+    int tile0[3];  // first column tile of each segment; of an absent one, past every tile
     const _Float16* xp;   // [M][P][Kp] activation parts
     const int32_t* xe;    // [M] row exponents e (x' = x 2^e); P == 2
     const void* x;        // the caller's activations [M][K], for the recomputed sums
@@ -78,6 +77,20 @@ struct XgArgs {
     int group, gpr;       // XG_Q4: elements per scale, scales per row
     int act;              // ACT: h = act(seg 0) * seg 1, written to seg 0's y
 };
+
+// The segment of column tile vt and its first tile: selects between arguments that are all loaded at once, not
+// a chain of loads through an index
+__device__ __forceinline__ XgSeg segment_of(const XgArgs& a, int vt, int& tile0)
+{
+    const XgSeg s0 = a.seg[0], s1 = a.seg[1], s2 = a.seg[2];
+    const int t1 = a.tile0[1], t2 = a.tile0[2];
+    const bool c1 = vt >= t1, c2 = vt >= t2;
+    const auto pick = [&](auto x0, auto x1, auto x2) { return c2 ? x2 : c1 ? x1 : x0; };
+    tile0 = pick(0, t1, t2);
+    return XgSeg{pick(s0.w, s1.w, s2.w), pick(s0.s, s1.s, s2.s), pick(s0.bias, s1.bias, s2.bias), pick(s0.y, s1.y, s2.y),
+                 pick(s0.n, s1.n, s2.n), pick(s0.s_stride, s1.s_stride, s2.s_stride), pick(s0.gs, s1.gs, s2.gs),
+                 pick(s0.gb, s1.gb, s2.gb)};
+}
 
 template <int FMT>
 struct Fmt;
@@ -218,10 +231,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
     const int step0 = blockIdx.z * a.steps_per_split, total = a.Kp / kBK;
     const int nsteps = min(a.steps_per_split, total - step0);
     if (nsteps <= 0) return;  // the launcher makes no empty split
-    const int si = ACT ? 0 : (a.nseg > 1 && vt >= a.tile0[1]) + (a.nseg > 2 && vt >= a.tile0[2]);
-    const XgSeg g = a.seg[si];
-    const XgSeg gu = ACT ? a.seg[1] : g;
-    const int n0 = (vt - a.tile0[si]) * (ACT ? BN / 2 : BN);
+    int tile0 = 0;
+    const XgSeg gu = a.seg[1], g = ACT ? a.seg[0] : segment_of(a, vt, tile0);
+    const int n0 = (vt - tile0) * (ACT ? BN / 2 : BN);
     const size_t rbytes = row_bytes<FMT>(a.K);
 
     // X DMA: load j of a wave covers 8 part rows (128 bytes each); part row p BM + i is part p of row
@@ -391,7 +403,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
         // the sums of two steps meet before they join the total
         for (int s = 0; s < nsteps; s += 2) {
             f16v_t a0[TA][TB] = {}, a1[TA][TB] = {};
-            if constexpr (GROUPED) {
+            if constexpr (GROUPED && P == 1) {
+                step(s, a0, sum);  // f16 x: each step onto the total (a second set of sums costs the registers)
+                if (s + 1 < nsteps) step(s + 1, a1, sum);
+                continue;
+            } else if constexpr (GROUPED) {
                 step(s, a0, a1);
                 if (s + 1 < nsteps) {
                     f16v_t a2[TA][TB] = {};
@@ -480,16 +496,9 @@ __global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a,
     const size_t stride = (size_t)a.M * (a.vcols / 4);
     for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < (size_t)a.M * quads; t += (size_t)gridDim.x * 256) {
         const int m = (int)(t / quads), c0 = (int)(t - (size_t)m * quads) * 4;
-        int si = 0, n = c0, vc = c0;
-        if constexpr (ACT) {
-            vc = c0 / 32 * 64 + c0 % 32;  // 32 gate columns, then their 32 up columns
-        } else {
-            const int vt = c0 / bn;
-            si = (a.nseg > 1 && vt >= a.tile0[1]) + (a.nseg > 2 && vt >= a.tile0[2]);
-            n -= a.tile0[si] * bn;
-        }
-        const XgSeg g = a.seg[si];
-        const XgSeg gu = ACT ? a.seg[1] : g;
+        int tile0 = 0;
+        const XgSeg gu = a.seg[1], g = ACT ? a.seg[0] : segment_of(a, c0 / bn, tile0);
+        const int n = c0 - tile0 * bn, vc = ACT ? c0 / 32 * 64 + c0 % 32 : c0;  // ACT: 32 gate, then their 32 up columns
         if (n >= g.n) continue;
         const f4_t* part = reinterpret_cast<const f4_t*>(a.part + (size_t)m * a.vcols + vc);
         const f4_t v = sum_splits_f4(part, stride, splits);
@@ -609,8 +618,26 @@ __global__ __launch_bounds__(256) void split_x_kernel(const float* __restrict__ 
     }
 }
 
+// f16 rows in the nibbles' order, zero-padded to Kp, with each step's sum (K % 8 == 0): a thread per eight
+// elements, eight threads per step
+__global__ __launch_bounds__(256) void pair_x_kernel(const _Float16* __restrict__ x, int M, int K, int Kp,
+                                                     _Float16* __restrict__ xp, float* __restrict__ xsum)
+{
+    const int per_row = Kp / 8;
+    const size_t units = (size_t)M * per_row;  // a multiple of 8: a step's threads are all here or none
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < units; t += (size_t)gridDim.x * 256) {
+        const int m = (int)(t / per_row), u = (int)(t - (size_t)m * per_row);
+        h8_t v = {};
+        if (u * 8 < K) v = *reinterpret_cast<const h8_t*>(x + (size_t)m * K + u * 8);
+        const float s = oct_sum((((float)v[0] + (float)v[1]) + ((float)v[2] + (float)v[3])) +
+                                (((float)v[4] + (float)v[5]) + ((float)v[6] + (float)v[7])));
+        if ((u & 7) == 0) xsum[(size_t)(u >> 3) * M + m] = s;
+        reinterpret_cast<h8_t*>(xp)[t] = h8_t{v[0], v[4], v[1], v[5], v[2], v[6], v[3], v[7]};
+    }
+}
+
 // The tile forms, rows x columns: f32 x 32 x 128 (2 waves), 64 x 128 (4 waves), 128 x 256 (8 waves); f16 x
-// 32 x 128, 128 x 128, 256 x 256.
+// 32 x 128, 128 x 128, 256 x 256 (group-scaled nibbles, with their second accumulators, 128 x 256).
 struct XgPlan {
     int form, bm, bn, vtiles, steps_per_split, splits;
     size_t xp_off, sum_off, part_off, bytes;  // workspace: exponents, parts, sums of x', split sums
@@ -628,7 +655,7 @@ XgPlan xg_plan(int fmt, int P, const XgSeg* segs, int nseg, bool act, int M, int
         p.bm = bm, p.bn = bn, p.vtiles = t;
         return (int64_t)t * ((M + bm - 1) / bm);
     };
-    int64_t blocks = tiles(P == 2 ? 128 : 256, 256);
+    int64_t blocks = tiles(P == 2 || fmt == XG_Q4 ? 128 : 256, 256);
     p.form = 2;
     if (blocks < 192) {
         p.form = M > 32 ? 1 : 0;
@@ -643,7 +670,7 @@ XgPlan xg_plan(int fmt, int P, const XgSeg* segs, int nseg, bool act, int M, int
     p.splits = (steps + p.steps_per_split - 1) / p.steps_per_split;
     const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     p.xp_off = P == 2 ? up((size_t)M * 4) : 0;
-    p.sum_off = p.xp_off + (P == 2 || K % kBK ? up((size_t)M * P * steps * kBK * 2) : 0);
+    p.sum_off = p.xp_off + (P == 2 || K % kBK || fmt == XG_Q4 ? up((size_t)M * P * steps * kBK * 2) : 0);
     p.part_off = p.sum_off + (fmt == XG_Q4 ? up((size_t)M * steps * 4) : 0);
     p.bytes = p.part_off + (p.splits > 1 ? (size_t)p.splits * M * p.vtiles * p.bn * 4 : 0);
     return p;
@@ -667,8 +694,8 @@ template <int FMT, bool S16, int P, bool ACT>
 hipError_t launch_act(const XgArgs& a, const XgPlan& p, hipStream_t st)
 {
     // f16 rows are twice the bytes: two stages keep two blocks (form 1) or one (form 2) on a CU
-    constexpr int NST = FMT == XG_F16 ? 2 : 3, T1 = P == 2 ? 1 : 2;
-    hipError_t e = p.form == 2   ? launch_form<FMT, S16, P, 2 * T1, 2, 2, 4, NST, ACT>(a, p, st)
+    constexpr int NST = FMT == XG_F16 ? 2 : 3, T1 = P == 2 ? 1 : 2, T2 = P == 1 && FMT != XG_Q4 ? 4 : 2;
+    hipError_t e = p.form == 2   ? launch_form<FMT, S16, P, T2, 2, 2, 4, NST, ACT>(a, p, st)
                    : p.form == 1 ? launch_form<FMT, S16, P, T1, 2, 2, 2, NST, ACT>(a, p, st)
                                  : launch_form<FMT, S16, P, 1, 2, 1, 2, 3, ACT>(a, p, st);
     if (e != hipSuccess || p.splits == 1) return e;
@@ -697,9 +724,9 @@ bool qgemm_exact_supported(const XgCall& c, int M, int K)
 {
     const bool nibbles = c.fmt == XG_I4 || c.fmt == XG_Q4;
     // weight rows start on 16-byte boundaries; a K step has one scale
-    if (M < (c.x_f16 ? 1 : 5) || K <= 0 || K % (nibbles ? 32 : c.fmt == XG_I8 ? 16 : 8) != 0) return false;
+    if (M < (c.x_f16 && c.fmt == XG_I8 ? 1 : 5) || K <= 0 || K % (nibbles ? 32 : c.fmt == XG_I8 ? 16 : 8) != 0) return false;
     if (c.fmt == XG_Q4 && (c.group <= 0 || c.group % kBK != 0)) return false;
-    if (c.x_f16 && c.fmt != XG_I8) return false;
+    if (c.x_f16 && c.fmt != XG_I8 && (c.fmt != XG_Q4 || !c.segs[0].gb)) return false;
     if (c.act >= 0 && (c.fmt == XG_F16 || c.nseg != 2 || c.segs[0].n != c.segs[1].n)) return false;
     int64_t n = 0;
     for (int i = 0; i < c.nseg; ++i) {
@@ -711,7 +738,7 @@ bool qgemm_exact_supported(const XgCall& c, int M, int K)
     if ((reinterpret_cast<uintptr_t>(c.x) & 15) != 0 || (M + 31) / 32 > 65535) return false;
     // a tile's byte offsets are 32-bit
     if ((uint64_t)K * 1024 >= (1ull << 31) || n >= (1 << 30)) return false;
-    if (c.x_f16 && K % kBK == 0) return true;  // no copy of x
+    if (c.x_f16 && (c.fmt == XG_I8 ? K % kBK == 0 : M > 64)) return true;  // x in place; over the tile kernels of f16 weights
     // The kernels of single rows walk the rows one after the other (f16: four at a time), so they take
     // longer with M K (a wave's walk) and with M K N (the whole work); the three launches here take 14-17
     // us at small sizes.  Measured, row kernels against these (us, rows x outputs x k):
@@ -735,10 +762,10 @@ hipError_t launch_qgemm_exact(const XgCall& c, int M, int K, void* ws, hipStream
     const bool act = c.act >= 0;
     const XgPlan p = xg_plan(c.fmt, c.x_f16 ? 1 : 2, c.segs, c.nseg, act, M, K);
     XgArgs a{};
-    a.nseg = c.nseg;
-    for (int i = 0, t = 0; i < c.nseg; ++i) {
+    for (int i = 0, t = 0; i < 3; ++i) {
+        a.tile0[i] = i < c.nseg && !act ? t : INT32_MAX;
+        if (i >= c.nseg) continue;
         a.seg[i] = c.segs[i];
-        a.tile0[i] = act ? 0 : t;
         t += (c.segs[i].n + p.bn - 1) / p.bn;
     }
     unsigned char* base = static_cast<unsigned char*>(ws);
@@ -759,6 +786,15 @@ hipError_t launch_qgemm_exact(const XgCall& c, int M, int K, void* ws, hipStream
     a.group = c.group;
     a.gpr = c.gpr;
     a.act = c.act;
+    if (c.x_f16 && c.fmt == XG_Q4) {
+        const size_t units = (size_t)M * a.Kp / 8;
+        hipLaunchKernelGGL(pair_x_kernel, dim3((unsigned)std::min<size_t>((units + 255) / 256, 4096)), dim3(256), 0, st,
+                           static_cast<const _Float16*>(c.x), M, K, a.Kp, xp, xsum);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        if (c.sdt == DT_F32) return act ? launch_act<XG_Q4, false, 1, true>(a, p, st) : launch_act<XG_Q4, false, 1, false>(a, p, st);
+        return act ? launch_act<XG_Q4, true, 1, true>(a, p, st) : launch_act<XG_Q4, true, 1, false>(a, p, st);
+    }
     if (c.x_f16) {
         if (a.Kp == K) {
             a.xp = static_cast<const _Float16*>(c.x);

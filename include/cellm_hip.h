@@ -175,8 +175,9 @@ int32_t cellm_hip_qgemv_i8_qkv(cellm_hip_ctx_t* ctx, const int8_t* wq, const voi
 
 /* The q, k and v projections of MLX 4-bit affine weights sharing x, in one
  * launch for m <= 4 (f16 or f32 x, cols % 32 == 0, group >= 32, 16-byte
- * aligned x and W), or by the MFMA GEMM for f32 x at 5 rows and more; other
- * shapes run one GEMV per projection.  sq/bq ... are
+ * aligned x and W), or by an MFMA GEMM: f32 x at 5 rows and more, f16 x above
+ * 64 rows (cols % 32 == 0, except few columns over a long cols, whose sums are
+ * better split); other shapes run one GEMV per projection.  sq/bq ... are
  * each matrix's scales and group biases in sb_dtype (cellm_hip_qgemv_q4_affine);
  * biasq/biask/biasv (f32 [rows], or NULL) are added after each row sum, as
  * add_projection_bias_if_present does (qwen.rs:1132-1139).  No reference
@@ -207,7 +208,8 @@ int32_t cellm_hip_qgemv_i8_gate_up_silu(cellm_hip_ctx_t* ctx, const int8_t* wg, 
 /* The same for MLX 4-bit affine gate/up weights; sg/bg and su/bu are the affine
  * scales/biases of each matrix.  One launch computes both rows and the SiLU *
  * up for m <= 4 with f16 x, k % 32 == 0, group >= 32 and 16-byte aligned x,
- * wg and wu, and the MFMA GEMM of cellm_hip_qgemv_q4_affine for f32 x at 5 rows
+ * wg and wu, and an MFMA GEMM with the activation in its epilogue for f16 x
+ * above 64 rows as in cellm_hip_qgemv_q4_affine_qkv and for f32 x at 5 rows
  * and more; other shapes run two cellm_hip_qgemv_q4_affine launches and the
  * SiLU * up kernel. */
 int32_t cellm_hip_qgemv_q4_affine_gate_up_silu(cellm_hip_ctx_t* ctx, const uint32_t* wg, const void* sg,

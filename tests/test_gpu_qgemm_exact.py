@@ -357,3 +357,29 @@ def test_qkv_and_gate_up_f16_rows(ops, m, rq, rkv, k):
     torch.cuda.synchronize()
     g, u = (x.double() @ t.double().t() * s.double() for t, s in ((wg, sg), (wu, su)))
     assert _rel(h.cpu(), _act(g, u, "silu")) <= 4e-6
+
+
+# f16 activations over MLX q4 at more than 64 rows: k % 128 == 0 runs f16 weight tiles (2^-11 per weight, 2e-4 in
+# the sum; f32, f16 and bf16 scales), other k the exact nibbles
+@pytest.mark.parametrize("m,rq,rkv,k", [(65, 130, 33, 128), (77, 896, 128, 896), (300, 300, 260, 2560), (513, 2500, 520, 384),
+                                        (128, 1000, 64, 6400), (77, 896, 128, 960), (200, 300, 40, 1056), (40, 300, 40, 1056)])
+@pytest.mark.parametrize("sdt", [torch.float16, torch.float32, torch.bfloat16])
+def test_q4_qkv_and_gate_up_f16_rows(ops, m, rq, rkv, k, sdt):
+    tol = 5e-4 if k % 128 == 0 else TOL
+    x = _x(m, k, m + k).half()
+    rows, xc = (rq, rkv, rkv), x.cuda()
+    bias = [torch.randn(r, generator=torch.Generator().manual_seed(r)) for r in rows]
+    y = [torch.full((m, r), float("nan"), device="cuda") for r in rows]
+    q = [_q4(r, k, 17 + i, sdt) for i, r in enumerate(rows)]
+    ops.encode_qkv_q4_affine(*q[0][:3], *q[1][:3], *q[2][:3], xc, *y, biasq=bias[0].cuda(), biasv=bias[2].cuda())
+    torch.cuda.synchronize()
+    for i in range(3):
+        assert _rel(y[i].cpu(), x.double() @ q[i][3].t() + (bias[i].double() if i != 1 else 0)) <= tol, i
+    x = (x * 0.3).half()
+    g, u = _q4(rq, k, 5, sdt), _q4(rq, k, 6, sdt)
+    h = torch.full((m, rq), float("nan"), device="cuda")
+    for act, fn in (("silu", ops.encode_gate_up_silu_q4_affine), ("gelu", ops.encode_gate_up_gelu_q4_affine)):
+        h.fill_(float("nan"))
+        fn(*g[:3], *u[:3], x.cuda(), h)
+        torch.cuda.synchronize()
+        assert _rel(h.cpu(), _act(x.double() @ g[3].t(), x.double() @ u[3].t(), act)) <= 2 * tol, act
