@@ -456,27 +456,54 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
     constexpr int TO = ACT ? 1 : TB;
     const auto out_col = [&](int j) { return n0 + (ACT ? wn : wn * TB + j) * 32 + r32; };
     const auto value = [](float v, int ev, float sc, float bi) { return (P == 2 ? ldexpf(v, ev) : v) * sc + bi; };
-    bool bad = false;
+    // every load of the epilogue before its first store: one still pending there makes each guarded store wait for
+    // the one before it (int8 over f16 rows, 2048 x 12288 x 4096: 237 -> 223 us)
+    float sc[TO], bi[TO], sc1 = 1.0f, bi1 = 0.0f;
 #pragma unroll
     for (int j = 0; j < TO; ++j) {
-        const int n = out_col(j);
-        if (n >= g.n) continue;
-        const float sc = column_scale(g, a.sdt, n), bi = g.bias ? g.bias[n] : 0.0f;
-        const float sc1 = ACT ? column_scale(gu, a.sdt, n) : 1.0f, bi1 = ACT && gu.bias ? gu.bias[n] : 0.0f;
+        const int n = min(out_col(j), g.n - 1);
+        sc[j] = column_scale(g, a.sdt, n);
+        bi[j] = g.bias ? g.bias[n] : 0.0f;
+        if constexpr (ACT) {
+            sc1 = column_scale(gu, a.sdt, n);
+            bi1 = gu.bias ? gu.bias[n] : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < TO; ++j) asm volatile("" : "+v"(sc[j]), "+v"(bi[j]));
+    asm volatile("" : "+v"(sc1), "+v"(bi1));
+    if constexpr (P == 2) {
 #pragma unroll
         for (int i = 0; i < TA; ++i)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3);
-                const int ev = P == 2 ? e[i][r] : 0;
-                float v = value(sum[i][j][r], ev, sc, bi);
-                if constexpr (ACT) v = act_mul(a.act, v, value(sum[i][TB - 1][r], ev, sc1, bi1));
-                if (m < a.M) {
-                    g.y[(size_t)m * g.n + n] = v;
-                    bad |= !finite_f32(v);
-                }
-            }
+            for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(e[i][r]));
     }
+    bool bad = false;
+    const auto store = [&](auto act) {
+#pragma unroll
+        for (int j = 0; j < TO; ++j) {
+            const int n = out_col(j);
+            if (n >= g.n) continue;
+#pragma unroll
+            for (int i = 0; i < TA; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3);
+                    const int ev = P == 2 ? e[i][r] : 0;
+                    float v = value(sum[i][j][r], ev, sc[j], bi[j]);
+                    if constexpr (ACT)
+                        v = act_mul(decltype(act)::value, v, value(sum[i][TB - 1][r], ev, sc1, bi1));
+                    if (m < a.M) {
+                        g.y[(size_t)m * g.n + n] = v;
+                        bad |= !finite_f32(v);
+                    }
+                }
+        }
+    };
+    if (ACT && a.act == ACT_GELU_TANH)  // outside the loops: no branch between neighbouring values
+        store(std::integral_constant<int, ACT_GELU_TANH>{});
+    else
+        store(std::integral_constant<int, ACT_SILU>{});
     if (!bad) return;
     // rolled and rare: this lane's non-finite results again (a non-finite gate or up sum makes h non-finite)
     for (int t = 0; t < TA * TO * 16; ++t) {
