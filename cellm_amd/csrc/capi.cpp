@@ -236,22 +236,29 @@ bool capturing(hipStream_t st)
 
 // The multi-row GEMM (qgemm_exact.hip) where it applies: *done tells whether it was enqueued.  It needs
 // scratch for x's parts, which the one-wave-per-row kernels do without, so a call that cannot have it
-// (captures, no memory) is left to them.  int8 over f16 x in place (k % 64 == 0) has no such kernel to
-// go back to and needs split sums at most.
+// (captures, no memory) is left to them.  int8 over f16 x in place (k % 64 == 0) needs split sums at most
+// and runs unsplit without them: a capture uses the stream's workspace as it stands and never grows it.
 int32_t try_qgemm_exact(cellm_hip_ctx* ctx, const XgCall& c, int64_t m, int64_t k, hipStream_t st, bool* done)
 {
     *done = false;
     if (!qgemm_exact_supported(c, (int)m, (int)k)) return CELLM_HIP_OK;
     const size_t need = qgemm_exact_workspace_bytes(c, (int)m, (int)k);
     const bool in_place = c.x_f16 && c.fmt == XG_I8 && k % 64 == 0;
-    if (need && !in_place && capturing(st)) return CELLM_HIP_OK;
     float* ws = nullptr;
-    const int32_t rc = get_workspace(ctx, st, need, &ws);
-    if (rc == CELLM_HIP_ERR_OUT_OF_MEMORY && !in_place) {
-        (void)hipGetLastError();
-        return CELLM_HIP_OK;
+    if (need && capturing(st)) {
+        if (!in_place) return CELLM_HIP_OK;
+        const auto it = ctx->workspaces.find(st);
+        if (it != ctx->workspaces.end() && it->second.bytes >= need) ws = reinterpret_cast<float*>(it->second.ptr);
+    } else {
+        const int32_t rc = get_workspace(ctx, st, need, &ws);
+        if (rc == CELLM_HIP_ERR_OUT_OF_MEMORY) {
+            (void)hipGetLastError();
+            if (!in_place) return CELLM_HIP_OK;
+            ws = nullptr;
+        } else if (rc) {
+            return rc;
+        }
     }
-    if (rc) return rc;
     HIP_TRY(launch_qgemm_exact(c, (int)m, (int)k, ws, st), "qgemm_exact launch");
     *done = true;
     return CELLM_HIP_OK;

@@ -787,7 +787,11 @@ size_t qgemm_exact_workspace_bytes(const XgCall& c, int M, int K)
 hipError_t launch_qgemm_exact(const XgCall& c, int M, int K, void* ws, hipStream_t st)
 {
     const bool act = c.act >= 0;
-    const XgPlan p = xg_plan(c.fmt, c.x_f16 ? 1 : 2, c.segs, c.nseg, act, M, K);
+    XgPlan p = xg_plan(c.fmt, c.x_f16 ? 1 : 2, c.segs, c.nseg, act, M, K);
+    if (!ws && p.splits > 1) {  // x in place and no workspace for split sums
+        p.steps_per_split *= p.splits;
+        p.splits = 1;
+    }
     XgArgs a{};
     for (int i = 0, t = 0; i < 3; ++i) {
         a.tile0[i] = i < c.nseg && !act ? t : INT32_MAX;

@@ -219,6 +219,27 @@ def test_captured_calls_use_no_scratch(ops):
         assert _rel(y.cpu(), ref) <= TOL
 
 
+def test_captured_f16_rows_on_a_fresh_stream(ops):
+    """int8 over f16 rows whose eager form splits K: a capture on a stream without a workspace allocates none and
+    runs unsplit.  One f32 chain of 2560 / 16 MFMA roundings stays within TOL."""
+    m, n, k = 129, 200, 2560
+    x, (w, s) = _x(m, k, 1).half(), _i8(n, k, 2)
+    ref = x.double() @ w.double().t() * s.double()
+    wd, sd, xd, y = w.cuda(), s.cuda(), x.cuda(), torch.zeros(m, n, device="cuda")
+    ops.encode_qgemm_i8(wd, sd, xd, y)  # the kernels' modules are loaded
+    torch.cuda.synchronize()
+    assert _rel(y.cpu(), ref) <= TOL
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        ops.encode_qgemm_i8(wd, sd, xd, y, stream=torch.cuda.current_stream())
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _rel(y.cpu(), ref) <= TOL
+
+
 def _q4(n, k, seed, sdt=torch.float32):
     g = torch.Generator().manual_seed(seed)
     w = torch.randint(-2**31, 2**31, (n, k // 8), generator=g, dtype=torch.int64).to(torch.int32)
