@@ -47,6 +47,7 @@ namespace cellm {
 namespace {
 
 constexpr int kWaves = 4, kThreads = kWaves * 64, kCols = 16, kChunk = 32;
+constexpr int kMinSplit = kWaves * kChunk;  // positions: a chunk per wave
 constexpr int kVStride = kChunk + 4;  // halves between the dims of a transposed V chunk
 
 struct AttnArgs {
@@ -58,7 +59,7 @@ struct AttnArgs {
     int max_blocks, total_blocks, n_layers, tpb, tpb_shift;  // tpb_shift: log2(tpb), or -1
     int rows, n_heads, n_kv, group, layer, window, tiles;
     float scale, soft_cap;
-    int per_split, nsplit;  // positions of a split (a multiple of kChunk)
+    int nsplit, cap;        // splits of a row's positions at most; positions of a table
     float* part;            // [row][kv head][split][group][HD + 2]
     uint32_t* counters;     // per (row, kv head): splits done, zero between calls
     float* out;
@@ -190,13 +191,13 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
     __shared__ long long bases_s[kWaves][kChunk];
     __shared__ float ml[kWaves][2][kCols];
     __shared__ uint32_t flags;                        // tile rows that differ; then columns to compute plainly
-    __shared__ int last;
+    __shared__ int last, splits_s;                    // splits_s: of this pass (a scalar register fewer over the loop)
 
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int c = lane & 15, g4 = lane >> 4;
     const int r = block_row(a, blockIdx.x / a.n_kv), kvh = blockIdx.x % a.n_kv, sp = blockIdx.y;
     const int gid = r * a.n_kv + kvh;
-    const int cap = a.max_blocks * a.tpb, kvd = a.n_kv * HD;
+    const int cap = a.cap, kvd = a.n_kv * HD;
 
     // ---- positions and first pages of the tile's rows, and the first chunk's page entry
     const int tile0 = r & ~(kCols - 1), sub = r & (kCols - 1), nr = min(kCols, a.rows - tile0);
@@ -278,13 +279,23 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
             lo = __builtin_amdgcn_readfirstlane(lo);
         }
         const int table = solo ? r : tile0 + leader;
-        const int split0 = solo ? lo / a.per_split : 0, split1 = solo ? (hi - 1) / a.per_split : 0;
-        int t0 = lo & ~(kChunk - 1), t1 = hi;
+        int t0 = lo & ~(kChunk - 1), t1 = hi, splits = 1;
         if (solo) {
-            if (sp < split0 || sp > split1) continue;
-            t0 = max(t0, sp * a.per_split);
-            t1 = min(hi, (sp + 1) * a.per_split);
+            // Rows past half their table take shares of the table, the others (and windows) spread their own
+            // positions over all splits.  us, shares / spread: 8 rows, 32/8 heads of 128, table of 8192, positions
+            // 500 16.1 / 13.1, 2000 29.3 / 23.5, 4096..8191 56.4 / 57.6; 16 rows, 8/8 of 128, 9000 of 16384 116 /
+            // 122; 1 row, 14/2 of 64, 1000 of 32768 14.9 / 11.3 (at least 256 a split 12.6); 16 rows, 32/8 of 128,
+            // window 2048 of 8192 47.3 / 33.9
+            const int len = hi - t0, over = 2 * len >= a.cap ? a.cap : len;
+            // (the divisions run on the vector unit: their results go back to scalars)
+            const int per = __builtin_amdgcn_readfirstlane(
+                max(kMinSplit, ((over + a.nsplit - 1) / a.nsplit + kChunk - 1) & ~(kChunk - 1)));
+            splits = __builtin_amdgcn_readfirstlane((len + per - 1) / per);
+            if (sp >= splits) continue;
+            t0 += sp * per;
+            t1 = min(hi, t0 + per);
         }
+        if (t == 0) splits_s = splits;  // read after the barriers below
 
         // ---- q: two f16 parts of every column in LDS (wave 0; lane (c, g4): dims 32 kk + 8 g4 + 0..7)
         if (wave == 0) {
@@ -471,7 +482,8 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
         }
         if (t == 0) flags = 0;
         __syncthreads();
-        const bool split = solo && split1 > split0;
+        const int nsp = __builtin_amdgcn_readfirstlane(splits_s);
+        const bool split = nsp > 1;
         float* const grp = a.part + (size_t)gid * a.nsplit * a.group * (HD + 2);
         for (int i = t; i < kCols * (HD / 4); i += kThreads) {
             const int oc = i / (HD / 4), d4 = i % (HD / 4);
@@ -509,12 +521,12 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
             __syncthreads();
             if (t == 0)
                 last = __hip_atomic_fetch_add(a.counters + gid, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                       (uint32_t)(split1 - split0);
+                       (uint32_t)(nsp - 1);
             __syncthreads();
             if (!last) return;  // the pass of this row's heads is the last one
             // split maxima and sums to LDS, then weights e^(m_k - M), then HD values per head, eight loads at a time
-            const int n = split1 - split0 + 1;
-            const float* base = grp + (size_t)split0 * a.group * (HD + 2);
+            const int n = nsp;
+            const float* base = grp;
             const size_t step = (size_t)a.group * (HD + 2);
             float* mk = reinterpret_cast<float*>(wave_lds);   // [group][n], then the weights
             float* lk = mk + a.group * n;
@@ -595,13 +607,13 @@ hipError_t launch_attention_mma(const float* q, const uint16_t* kcache, const ui
     a.scale = scale;
     a.soft_cap = soft_cap;
     const int cap = max_blocks * tokens_per_block;
-    // splits of at least 512 positions (four chunks per wave), and no more than make 512 blocks: a split that
-    // has no work still reads positions and pages (4 rows of 15 / 5 heads over 2048 positions: 256 / 512 / 1024
+    // at least 512 positions of the table per split (four chunks per wave), and no more splits than make 512
+    // blocks: a split that has no work still reads positions and pages (4 rows of 15 / 5 heads over 2048 positions: 256 / 512 / 1024
     // per split 17.3 / 15.3 / 21.5 us; 8 rows of 32 / 8 heads of 128 over 8192: 512 / 768 / 1024 65 / 64 / 60 us;
     // a 2048-token prompt of 14 / 2 heads with four splits 186 us, with one 126)
     const int want = std::min(max_splits, std::max(1, 512 / (rows * n_kv_heads)));
-    a.per_split = want > 1 ? std::max(512, ((cap + want - 1) / want + kChunk - 1) / kChunk * kChunk) : cap;
-    a.nsplit = (cap + a.per_split - 1) / a.per_split;
+    a.nsplit = std::min(want, (cap + 511) / 512);
+    a.cap = cap;
     a.part = part;
     a.counters = counters;
     a.out = out;

@@ -123,6 +123,24 @@ def test_long_contexts_in_splits(ops, rows, nh, nkv, hd, ctx):
         assert _rel(_run(ops, q, kc, vc, bt, pos, 0), _reference(q, kc, vc, bt, pos, 0)) <= TOL
 
 
+# lengths at the edges of the shortest split (128), below, at and past half the table, and the whole of it
+@pytest.mark.parametrize("nh,nkv,hd,window", [(14, 2, 64, 0), (8, 1, 128, 0), (4, 2, 128, 700), (8, 8, 64, 5000)])
+def test_short_contexts_in_large_tables(ops, nh, nkv, hd, window):
+    tpb, per = 16, 512
+    lens = [1, 127, 128, 129, 257, 1025, 4095, 4096, 4097, 8192]
+    rows = len(lens)
+    g = torch.Generator().manual_seed(hd + nh)
+    kc, vc = _cache(per * rows, 1, tpb, nkv, hd, nh)
+    bt = torch.randperm(per * rows, generator=g).view(rows, per)
+    pos = torch.tensor(lens) - 1
+    q = torch.randn(rows, nh, hd, generator=g)
+    ref = _reference(q, kc, vc, bt, pos, 0, window=window)
+    for _ in range(2):
+        got = _run(ops, q, kc, vc, bt, pos, 0, window=window)
+        for r in range(rows):
+            assert _rel(got[r], ref[r]) <= TOL, lens[r]
+
+
 @pytest.mark.parametrize("rows,ctx", [(40, 320), (2, 8192)])  # a shared tile; splits
 def test_non_finite_keys_values_and_queries(ops, rows, ctx):
     """An infinite or NaN element reaches the outputs it reaches in a plain f32 softmax: a key of -inf score has
