@@ -90,8 +90,8 @@ hipError_t launch_qgemm_q4_fused(const Q4FusedSeg* segs, int nseg, int act, int 
                                  int K, hipStream_t st);
 
 // Multi-row GEMM, weights exact in f16 (qgemm_exact.hip): f32 x at M >= 5 (and rows enough to pay for its
-// launches), or f16 x over int8; 16-byte aligned W, x and weight rows.  Up to three matrices share x.  `ws` holds
-// x's f16 parts and the split sums.
+// launches), or f16 x over int8 and q4; 16-byte aligned W, x and weight rows.  Up to three matrices share x.  `ws` holds
+// x's f16 parts and the split sums; int8 over f16 x with K % 64 == 0 has x in place and, without `ws`, runs unsplit.
 enum { XG_I8 = 0, XG_I4 = 1, XG_F16 = 2, XG_Q4 = 3 };
 struct XgSeg {
     const void* w;
@@ -108,7 +108,7 @@ struct XgCall {
     const XgSeg* segs;
     int nseg;
     int sdt;
-    const void* x;      // [M][K] f32, or f16 (int8 weights only)
+    const void* x;      // [M][K] f32, or f16 (XG_I8, XG_Q4 with biases)
     bool x_f16;
     int act;            // -1, or ACT_*: y of seg 0 = act(seg 0) * seg 1
     int group, gpr;     // XG_Q4: elements per scale (a multiple of 64) and scales per row
