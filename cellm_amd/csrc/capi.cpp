@@ -83,6 +83,7 @@ int32_t hip_error(hipError_t e, const char* what)
 struct DeviceBuffer {
     void* ptr = nullptr;
     size_t bytes = 0;
+    bool captured = false;  // a captured graph holds its address
 };
 
 bool valid_dtype(int32_t d) { return d == DT_F32 || d == DT_F16 || d == DT_BF16; }
@@ -102,6 +103,7 @@ struct cellm_hip_ctx {
     std::unordered_map<hipStream_t, DeviceBuffer> aux;         // unfused gate/up: the up rows, one per stream
     std::unordered_map<hipStream_t, DeviceBuffer> attn;        // split-sequence attention partials, one per stream
     std::unordered_map<hipStream_t, DeviceBuffer> argmax;      // argmax row counters + chunk partials, one per stream
+    std::vector<void*> retired;                                // outgrown scratch that captured graphs still write to
     float* attn_static = nullptr;  // this device's static attention scratch (cellm_hip_attention_gqa_f16kv_noalloc)
     std::atomic<int> rope_interleaved{0};  // RoPE pairs of the fused decode ops (cellm_hip_set_rope_interleaved)
 };
@@ -177,11 +179,26 @@ int32_t check_n_scales(int64_t n_scales, int64_t n, const char* what)
                      (long long)n_scales, what, (long long)n);
 }
 
+// Whether the stream is under graph capture (or cannot be asked: the null stream during another's capture)
+bool capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
 // Per-stream scratch (split-K partials, unfused gate/up rows, attention
 // partials), grown on demand.  The caller holds ctx->mu from this call until
 // every kernel that uses the buffer is enqueued: calls on one stream then
 // queue their scratch users back to back, and a grow (which waits for the
 // stream, then frees) cannot happen between a get and its launches.
+// A buffer that was handed to a capture is never freed before the context is:
+// the graph writes to it on every replay, so a grow sets it aside.  A capture
+// itself takes the buffer as it stands; one that is too small is refused before
+// anything is done to the stream.
 // zero_prefix: bytes at the start of a freshly allocated buffer that are cleared
 // on this stream before first use (the attention's group counters, which its
 // kernels then return to zero themselves).
@@ -193,7 +210,18 @@ int32_t get_stream_buffer(cellm_hip_ctx* ctx, std::unordered_map<hipStream_t, De
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     DeviceBuffer& b = map[st];
     const bool grow = b.bytes < need;
-    if (grow) {
+    if ((grow || !b.captured) && capturing(st)) {
+        if (grow)
+            return set_error(CELLM_HIP_ERR_DEVICE,
+                             "stream under capture: the call needs %zu bytes of scratch, the stream has %zu (run the "
+                             "call once on the stream before the capture)",
+                             need, b.bytes);
+        b.captured = true;
+    }
+    if (grow && b.captured) {
+        ctx->retired.push_back(b.ptr);
+        b = DeviceBuffer{};
+    } else if (grow) {
         // The old buffer may still be read by queued work on this stream.
         HIP_TRY(hipStreamSynchronize(st), "hipStreamSynchronize(workspace grow)");
     }
@@ -221,43 +249,23 @@ int32_t get_workspace(cellm_hip_ctx* ctx, hipStream_t st, size_t need, float** o
     return get_stream_buffer(ctx, ctx->workspaces, st, need, out);
 }
 
-// A stream under graph capture.  Calls whose scratch is only a matter of speed take the form without it
-// there: a workspace cannot grow during a capture, and one that grows later would leave the graph with
-// the address of the freed one.
-bool capturing(hipStream_t st)
-{
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &status) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;
-    }
-    return status != hipStreamCaptureStatusNone;
-}
-
 // The multi-row GEMM (qgemm_exact.hip) where it applies: *done tells whether it was enqueued.  It needs
 // scratch for x's parts, which the one-wave-per-row kernels do without, so a call that cannot have it
 // (captures, no memory) is left to them.  int8 over f16 x in place (k % 64 == 0) needs split sums at most
-// and runs unsplit without them: a capture uses the stream's workspace as it stands and never grows it.
+// and runs unsplit where it cannot have them.
 int32_t try_qgemm_exact(cellm_hip_ctx* ctx, const XgCall& c, int64_t m, int64_t k, hipStream_t st, bool* done)
 {
     *done = false;
     if (!qgemm_exact_supported(c, (int)m, (int)k)) return CELLM_HIP_OK;
     const size_t need = qgemm_exact_workspace_bytes(c, (int)m, (int)k);
     const bool in_place = c.x_f16 && c.fmt == XG_I8 && k % 64 == 0;
+    if (need && !in_place && capturing(st)) return CELLM_HIP_OK;
     float* ws = nullptr;
-    if (need && capturing(st)) {
+    if (const int32_t rc = get_workspace(ctx, st, need, &ws)) {
+        if (rc != CELLM_HIP_ERR_OUT_OF_MEMORY && !capturing(st)) return rc;
+        (void)hipGetLastError();
         if (!in_place) return CELLM_HIP_OK;
-        const auto it = ctx->workspaces.find(st);
-        if (it != ctx->workspaces.end() && it->second.bytes >= need) ws = reinterpret_cast<float*>(it->second.ptr);
-    } else {
-        const int32_t rc = get_workspace(ctx, st, need, &ws);
-        if (rc == CELLM_HIP_ERR_OUT_OF_MEMORY) {
-            (void)hipGetLastError();
-            if (!in_place) return CELLM_HIP_OK;
-            ws = nullptr;
-        } else if (rc) {
-            return rc;
-        }
+        ws = nullptr;
     }
     HIP_TRY(launch_qgemm_exact(c, (int)m, (int)k, ws, st), "qgemm_exact launch");
     *done = true;
@@ -677,6 +685,7 @@ void cellm_hip_destroy(cellm_hip_ctx_t* ctx)
             (void)hipStreamSynchronize(kv.first);
             if (kv.second.ptr) (void)hipFree(kv.second.ptr);
         }
+    for (void* p : ctx->retired) (void)hipFree(p);
     for (auto& kv : ctx->weights)
         if (kv.second.ptr) (void)hipFree(kv.second.ptr);
     if (ctx->x_buf.ptr) (void)hipFree(ctx->x_buf.ptr);

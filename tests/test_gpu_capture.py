@@ -1,0 +1,98 @@
+"""Graph capture and the context's per-stream scratch: a graph keeps the address of the scratch that its calls
+used, so that memory stays allocated when a later call needs more, and every replay gives the eager result."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from cellm_amd import HipOps
+from cellm_amd._lib import CellmHipError
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def own():
+    """A context of its own: no scratch of other tests."""
+    o = HipOps(0)
+    yield o
+    torch.cuda.synchronize()
+    o.close()
+
+
+def _i8(n, k, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randint(-128, 128, (n, k), generator=g, device="cuda", dtype=torch.int8),
+            torch.rand(n, generator=g, device="cuda") * 0.01 + 1e-3)
+
+
+def _q4(n, k, seed, dtype=torch.float16):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    w = torch.randint(-2**31, 2**31, (n, k // 8), generator=g, device="cuda", dtype=torch.int64).to(torch.int32)
+    s = (torch.rand(n, k // 64, generator=g, device="cuda") * 0.01 + 1e-3).to(dtype)
+    return w, s, (s.float() * -7.5).to(dtype)
+
+
+def _x(m, k, seed, dtype=torch.float32):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(m, k, generator=g, device="cuda").to(dtype)
+
+
+def _capture(stream, call):
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        call(torch.cuda.current_stream())
+    return graph
+
+
+def _replays(graph, y, ref, between=lambda: None):
+    for _ in range(3):
+        y.zero_()
+        between()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref)
+
+
+def test_scratch_of_a_graph_outlives_a_grow(own):
+    """A split q4 qGEMM is captured; an eager f32 call on that stream then needs more scratch.  The grow takes new
+    memory and keeps the old: the free memory tells, before a replay could write to it."""
+    side = torch.cuda.Stream()
+    (w8, s8), (wq, s, b) = _i8(64, 8192, 1), _q4(896, 4864, 2)
+    x = _x(128, 4864, 3, torch.float16)
+    small, large = _x(1024, 8192, 4), _x(2048, 8192, 5)
+    y, y8 = torch.zeros(128, 896, device="cuda"), torch.zeros(2048, 64, device="cuda")
+    gemm = lambda st: own.encode_qgemm_q4_affine(wq, s, b, x, y, stream=st)
+    rows = lambda v, st: own.encode_qgemv_i8(w8, s8, v, y8[:v.shape[0]], stream=st)
+    rows(large, torch.cuda.current_stream())  # the kernels' modules are loaded, another stream's scratch taken
+    rows(small, side)                         # 1024 rows of two f16 parts: 32 MiB on this stream
+    gemm(side)
+    torch.cuda.synchronize()
+    ref = y.clone()
+    graph = _capture(side, gemm)
+    before = torch.cuda.mem_get_info()[0]
+    rows(large, side)                         # 64 MiB
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] >= 60 * 2**20  # 32 MiB where the old scratch was freed
+    _replays(graph, y, ref, lambda: rows(large, side))
+
+
+def test_call_short_of_scratch_is_refused_and_the_capture_goes_on(own):
+    side = torch.cuda.Stream()
+    wq, s, b = _q4(896, 4864, 2)
+    x, y = _x(128, 4864, 3, torch.float16), torch.zeros(128, 896, device="cuda")
+    g, up = _x(16, 64, 6), _x(16, 64, 7)
+    own.encode_qgemm_q4_affine(wq, s, b, x, y)  # the scratch of another stream
+    h = g.clone()
+    own.encode_silu_mul(h, up)
+    ref = h.clone()
+
+    def calls(st):
+        with pytest.raises(CellmHipError, match="scratch"):
+            own.encode_qgemm_q4_affine(wq, s, b, x, y, stream=st)
+        h.copy_(g)
+        own.encode_silu_mul(h, up, stream=st)
+
+    _replays(_capture(side, calls), h, ref)
