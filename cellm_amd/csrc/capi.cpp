@@ -250,16 +250,17 @@ int32_t get_workspace(cellm_hip_ctx* ctx, hipStream_t st, size_t need, float** o
 }
 
 // The multi-row GEMM (qgemm_exact.hip) where it applies: *done tells whether it was enqueued.  It needs
-// scratch for x's parts, which the one-wave-per-row kernels do without, so a call that cannot have it
-// (captures, no memory) is left to them.  int8 over f16 x in place (k % 64 == 0) needs split sums at most
-// and runs unsplit where it cannot have them.
+// scratch for x's parts, which the one-wave-per-row kernels do without, so a call that cannot have it (no
+// memory, a capture on a stream with too little) is left to them.  int8 over f16 x in place (k % 64 == 0)
+// needs split sums at most and runs unsplit where it cannot have them.  A capture after an eager call of the
+// same shape runs the same launches: the gate/up rows and split sums of the other kernels' launches were not
+// reserved by that call.
 int32_t try_qgemm_exact(cellm_hip_ctx* ctx, const XgCall& c, int64_t m, int64_t k, hipStream_t st, bool* done)
 {
     *done = false;
     if (!qgemm_exact_supported(c, (int)m, (int)k)) return CELLM_HIP_OK;
     const size_t need = qgemm_exact_workspace_bytes(c, (int)m, (int)k);
     const bool in_place = c.x_f16 && c.fmt == XG_I8 && k % 64 == 0;
-    if (need && !in_place && capturing(st)) return CELLM_HIP_OK;
     float* ws = nullptr;
     if (const int32_t rc = get_workspace(ctx, st, need, &ws)) {
         if (rc != CELLM_HIP_ERR_OUT_OF_MEMORY && !capturing(st)) return rc;

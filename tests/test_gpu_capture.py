@@ -96,3 +96,73 @@ def test_call_short_of_scratch_is_refused_and_the_capture_goes_on(own):
         own.encode_silu_mul(h, up, stream=st)
 
     _replays(_capture(side, calls), h, ref)
+
+
+def _i4(n, k, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.randint(0, 256, (n, k // 2), generator=g, device="cuda", dtype=torch.uint8),
+            (torch.rand(n, 1, generator=g, device="cuda") * 0.01 + 1e-3).half())
+
+
+M, N, K = 77, 200, 960  # k % 128 == 64: q4 over f16 rows takes the GEMM that needs scratch
+
+
+def _gate_up_i8(ops, x, y):
+    g, u = _i8(N, K, 1), _i8(N, K, 2)
+    return lambda st: ops.encode_gate_up_silu_i8(*g, *u, x, y, stream=st)
+
+
+def _gate_up_q4(ops, x, y):
+    g, u = _q4(N, K, 1, x.dtype), _q4(N, K, 2, x.dtype)
+    return lambda st: ops.encode_gate_up_silu_q4_affine(*g, *u, x, y, stream=st)
+
+
+def _gate_up_i4(ops, x, y):
+    g, u = _i4(N, K, 1), _i4(N, K, 2)
+    return lambda st: ops.encode_gate_up_gelu_i4_sym(*g, *u, K, x, y, K, stream=st)
+
+
+def _qkv_q4(ops, x, y):
+    w = [t for i, n in enumerate((N - 80, 40, 40)) for t in _q4(n, K, 3 + i, x.dtype)]
+    q, k, v = (t.view(M, -1) for t in y.view(-1).split([M * (N - 80), M * 40, M * 40]))
+    return lambda st: ops.encode_qkv_q4_affine(*w, x, q, k, v, stream=st)
+
+
+def _qkv_i8(ops, x, y):
+    w = [t for i, n in enumerate((N - 80, 40, 40)) for t in _i8(n, K, 3 + i)]
+    q, k, v = (t.view(M, -1) for t in y.view(-1).split([M * (N - 80), M * 40, M * 40]))
+    return lambda st: ops.encode_qkv_i8(*w, x, q, k, v, stream=st)
+
+
+def _one_i8(ops, x, y):
+    w = _i8(N, K, 9)
+    return lambda st: ops.encode_qgemv_i8(*w, x, y, stream=st)
+
+
+def _one_i4(ops, x, y):
+    w = _i4(N, K, 9)
+    return lambda st: ops.encode_qgemv_i4_sym(*w, K, x, y, K, stream=st)
+
+
+def _one_f16(ops, x, y):
+    w = _x(N, K, 9, torch.float16)
+    return lambda st: ops.encode_qgemv_f16(w, x, y, stream=st)
+
+
+@pytest.mark.parametrize("make,dtype", [(_gate_up_i8, torch.float32), (_gate_up_q4, torch.float32),
+                                        (_gate_up_i4, torch.float32), (_gate_up_q4, torch.float16),
+                                        (_gate_up_i8, torch.float16), (_qkv_q4, torch.float16),
+                                        (_qkv_q4, torch.float32), (_qkv_i8, torch.float32),
+                                        (_one_i8, torch.float32), (_one_i4, torch.float32),
+                                        (_one_f16, torch.float32)])
+def test_one_eager_call_makes_the_capture_possible_and_equal(own, make, dtype):
+    """The scratch of one eager call on the capture stream is all that the capture of that call needs, and the
+    graph runs the same launches."""
+    y = torch.zeros(M, N, device="cuda")
+    call, side = make(own, _x(M, K, 5, dtype) * 0.1, y), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    call(side)
+    torch.cuda.synchronize()
+    ref = y.clone()
+    assert bool(ref.any())
+    _replays(_capture(side, call), y, ref)
