@@ -190,6 +190,17 @@ bool capturing(hipStream_t st)
     return status != hipStreamCaptureStatusNone;
 }
 
+// Memory is waited for, freed and taken beside captures of other streams, on this thread or another: in the
+// default (global) mode those calls would fail while any capture lasts, and end it.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool ok = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~RelaxedCapture()
+    {
+        if (ok) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 // Per-stream scratch (split-K partials, unfused gate/up rows, attention
 // partials), grown on demand.  The caller holds ctx->mu from this call until
 // every kernel that uses the buffer is enqueued: calls on one stream then
@@ -218,16 +229,21 @@ int32_t get_stream_buffer(cellm_hip_ctx* ctx, std::unordered_map<hipStream_t, De
                              need, b.bytes);
         b.captured = true;
     }
-    if (grow && b.captured) {
+    if (!grow) {
+        *out = reinterpret_cast<float*>(b.ptr);
+        return CELLM_HIP_OK;
+    }
+    const RelaxedCapture relaxed;
+    if (b.captured) {
         ctx->retired.push_back(b.ptr);
         b = DeviceBuffer{};
-    } else if (grow) {
+    } else {
         // The old buffer may still be read by queued work on this stream.
         HIP_TRY(hipStreamSynchronize(st), "hipStreamSynchronize(workspace grow)");
     }
     int32_t rc = ensure_buffer(b, need);
     if (rc) return rc;
-    if (grow && zero_prefix) HIP_TRY(hipMemsetAsync(b.ptr, 0, std::min(zero_prefix, need), st), "hipMemsetAsync(counters)");
+    if (zero_prefix) HIP_TRY(hipMemsetAsync(b.ptr, 0, std::min(zero_prefix, need), st), "hipMemsetAsync(counters)");
     *out = reinterpret_cast<float*>(b.ptr);
     return CELLM_HIP_OK;
 }

@@ -166,3 +166,30 @@ def test_one_eager_call_makes_the_capture_possible_and_equal(own, make, dtype):
     ref = y.clone()
     assert bool(ref.any())
     _replays(_capture(side, call), y, ref)
+
+
+@pytest.mark.parametrize("warm", [False, True])  # first scratch of the stream; a grow
+def test_scratch_grows_beside_the_capture_of_another_stream(own, warm):
+    """An eager call that needs scratch runs while another stream is captured in torch's (global) mode, and the
+    capture goes on."""
+    w, s = _i8(64, 512, 1)
+    x, y = _x(64, 512, 2), torch.zeros(64, 64, device="cuda")
+    h, up = _x(16, 64, 6), _x(16, 64, 7)
+    src, other = h.clone(), torch.cuda.Stream()
+    own.encode_silu_mul(h, up)
+    ref = h.clone()
+    own.encode_qgemv_i8(w, s, x, y)  # scratch of the current stream
+    expected = y.clone()
+    if warm:
+        own.encode_qgemv_i8(w, s, x[:32], y[:32], stream=other)
+    y.zero_()
+
+    def calls(st):
+        h.copy_(src)
+        own.encode_qgemv_i8(w, s, x, y, stream=other)
+        own.encode_silu_mul(h, up, stream=st)
+
+    graph = _capture(torch.cuda.Stream(), calls)
+    torch.cuda.synchronize()
+    assert torch.equal(y, expected)
+    _replays(graph, h, ref)
