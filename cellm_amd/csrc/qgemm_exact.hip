@@ -208,13 +208,15 @@ __device__ __forceinline__ float plain_output(const XgArgs& a, const XgSeg& g, c
     return act_mul(a.act, v, plain_dot<FMT, P>(a, gu, m, n) * column_scale(gu, a.sdt, n) + (gu.bias ? gu.bias[n] : 0.0f));
 }
 
-// S16: XG_Q4's scales are 16 bits wide.  ACT: segments 0 and 1 are gate and up; each wave's 64 columns are 32
+// S16: XG_Q4's scales are 16 bits wide.  FOLD: the sums of two K steps (int8 over f16 rows: four) meet before they
+// join the total, else one chain over K.  ACT: segments 0 and 1 are gate and up; each wave's 64 columns are 32
 // gate columns and the same 32 up columns, so both sums of an output end in one lane.
-template <int FMT, bool S16, int P, int TA, int TB, int WM, int WN, int NST, bool ACT>
+template <int FMT, bool S16, int P, bool FOLD, int TA, int TB, int WM, int WN, int NST, bool ACT>
 __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgArgs a)
 {
     constexpr int NW = WM * WN, BM = 32 * TA * WM, BN = 32 * TB * WN, RB = Fmt<FMT>::kStepBytes;
-    constexpr bool GROUPED = FMT == XG_Q4, FOLD = P == 2 || GROUPED;
+    constexpr bool GROUPED = FMT == XG_Q4;
+    static_assert(FOLD || !GROUPED, "group scales are folded per step");
     static_assert(!ACT || TB == 2, "a gate and an up tile per wave");
     // a stage: X parts, raw weights, and the step's group scales, group biases and sums of x'
     constexpr int kXBytes = BM * P * 128, kWBytes = BN * RB, kGroupAt = kXBytes + kWBytes, kSumAt = kGroupAt + 8 * BN;
@@ -400,14 +402,29 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
         }
     };
     if constexpr (FOLD) {
-        // the sums of two steps meet before they join the total
+        if constexpr (P == 1 && !GROUPED) {
+            for (int s = 0; s < nsteps; s += 4) {
+                f16v_t few[TA][TB] = {};
+                step(s, few, few);
+#pragma unroll
+                for (int u = 1; u < 4; ++u) {
+                    if (s + u >= nsteps) break;
+                    f16v_t a0[TA][TB] = {};
+                    step(s + u, a0, a0);
+#pragma unroll
+                    for (int i = 0; i < TA; ++i)
+#pragma unroll
+                        for (int j = 0; j < TB; ++j) few[i][j] += a0[i][j];
+                }
+#pragma unroll
+                for (int i = 0; i < TA; ++i)
+#pragma unroll
+                    for (int j = 0; j < TB; ++j) sum[i][j] += few[i][j];
+            }
+        } else
         for (int s = 0; s < nsteps; s += 2) {
             f16v_t a0[TA][TB] = {}, a1[TA][TB] = {};
-            if constexpr (GROUPED && P == 1) {
-                step(s, a0, sum);  // f16 x: each step onto the total (a second set of sums costs the registers)
-                if (s + 1 < nsteps) step(s + 1, a1, sum);
-                continue;
-            } else if constexpr (GROUPED) {
+            if constexpr (GROUPED) {
                 step(s, a0, a1);
                 if (s + 1 < nsteps) {
                     f16v_t a2[TA][TB] = {};
@@ -426,7 +443,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
                 }
         }
     } else {
-        for (int s = 0; s < nsteps; ++s) step(s, sum, sum);  // f16 x: one chain over K
+        for (int s = 0; s < nsteps; ++s) step(s, sum, sum);
     }
     wait_vmcnt<0>();  // the trailing (re-read) DMA, before the block's LDS is given back
 
@@ -670,10 +687,20 @@ struct XgPlan {
     size_t xp_off, sum_off, part_off, bytes;  // workspace: exponents, parts, sums of x', split sums
 };
 
+// f16 rows over int8 in place run one chain over K, as in the tile kernel that took them before (error at 4096 k,
+// 2048 rows, 4.2e-7 in both).  k % 64 != 0 came from the one-wave-per-row kernel's tree sums (976 / 2032 / 4080 /
+// 8176 k: 8.3e-8 / 9.3e-8 / 1.1e-7 / 1.5e-7), which sums of four steps keep (8.4e-8 / 9.4e-8 / 1.1e-7 / 1.3e-7) and a
+// chain does not (2.1e-7 / 2.9e-7 / 4.1e-7 / 5.7e-7); four steps need tiles of half the rows (2048 rows of 8176 ->
+// 8192 260 us chained, 344 so; single rows take tens of ms).  q4 over f16 rows: a step at a time onto the total 1.2e-7
+// / 1.4e-7 / 2.0e-7 / 2.9e-7 at 992 / 2016 / 4064 / 8160 k, in pairs 7.7e-8 / 8.7e-8 / 1.1e-7 / 1.6e-7 (single rows
+// 9.7e-8 / 1.2e-7 / 1.6e-7 / 2.1e-7), 3 to 5 % slower.
+bool xg_chained(int fmt, int P, int K) { return P == 1 && fmt == XG_I8 && K % kBK == 0; }
+
 XgPlan xg_plan(int fmt, int P, const XgSeg* segs, int nseg, bool act, int M, int K)
 {
     XgPlan p{};
     const int steps = (K + kBK - 1) / kBK;
+    const bool chained = xg_chained(fmt, P, K);
     auto tiles = [&](int bm, int bn) {
         int t = 0;
         if (act) t = (segs[0].n + bn / 2 - 1) / (bn / 2);
@@ -682,7 +709,7 @@ XgPlan xg_plan(int fmt, int P, const XgSeg* segs, int nseg, bool act, int M, int
         p.bm = bm, p.bn = bn, p.vtiles = t;
         return (int64_t)t * ((M + bm - 1) / bm);
     };
-    int64_t blocks = tiles(P == 2 || fmt == XG_Q4 ? 128 : 256, 256);
+    int64_t blocks = tiles(chained ? 256 : 128, 256);
     p.form = 2;
     if (blocks < 192) {
         p.form = M > 32 ? 1 : 0;
@@ -703,11 +730,11 @@ XgPlan xg_plan(int fmt, int P, const XgSeg* segs, int nseg, bool act, int M, int
     return p;
 }
 
-template <int FMT, bool S16, int P, int TA, int TB, int WM, int WN, int NST, bool ACT>
+template <int FMT, bool S16, int P, bool FOLD, int TA, int TB, int WM, int WN, int NST, bool ACT>
 hipError_t launch_form(const XgArgs& a, const XgPlan& p, hipStream_t st)
 {
     constexpr int lds = NST * stage_bytes(FMT, P, 32 * TA * WM, 32 * TB * WN, Fmt<FMT>::kStepBytes);
-    auto kern = qgemm_exact_kernel<FMT, S16, P, TA, TB, WM, WN, NST, ACT>;
+    auto kern = qgemm_exact_kernel<FMT, S16, P, FOLD, TA, TB, WM, WN, NST, ACT>;
     if constexpr (lds > 64 * 1024) {
         const hipError_t e = allow_big_lds(kern, lds);
         if (e != hipSuccess) return e;
@@ -717,14 +744,14 @@ hipError_t launch_form(const XgArgs& a, const XgPlan& p, hipStream_t st)
     return hipGetLastError();
 }
 
-template <int FMT, bool S16, int P, bool ACT>
+template <int FMT, bool S16, int P, bool ACT, bool FOLD = true>
 hipError_t launch_act(const XgArgs& a, const XgPlan& p, hipStream_t st)
 {
     // f16 rows are twice the bytes: two stages keep two blocks (form 1) or one (form 2) on a CU
-    constexpr int NST = FMT == XG_F16 ? 2 : 3, T1 = P == 2 ? 1 : 2, T2 = P == 1 && FMT != XG_Q4 ? 4 : 2;
-    hipError_t e = p.form == 2   ? launch_form<FMT, S16, P, T2, 2, 2, 4, NST, ACT>(a, p, st)
-                   : p.form == 1 ? launch_form<FMT, S16, P, T1, 2, 2, 2, NST, ACT>(a, p, st)
-                                 : launch_form<FMT, S16, P, 1, 2, 1, 2, 3, ACT>(a, p, st);
+    constexpr int NST = FMT == XG_F16 ? 2 : 3, T1 = P == 2 ? 1 : 2, T2 = FOLD ? 2 : 4;
+    hipError_t e = p.form == 2   ? launch_form<FMT, S16, P, FOLD, T2, 2, 2, 4, NST, ACT>(a, p, st)
+                   : p.form == 1 ? launch_form<FMT, S16, P, FOLD, T1, 2, 2, 2, NST, ACT>(a, p, st)
+                                 : launch_form<FMT, S16, P, FOLD, 1, 2, 1, 2, 3, ACT>(a, p, st);
     if (e != hipSuccess || p.splits == 1) return e;
     const size_t quads = (size_t)a.M * a.vcols / (ACT ? 8 : 4);
     const unsigned blocks = (unsigned)std::min<size_t>((quads + 255) / 256, 4096);
@@ -826,16 +853,16 @@ hipError_t launch_qgemm_exact(const XgCall& c, int M, int K, void* ws, hipStream
         if (c.sdt == DT_F32) return act ? launch_act<XG_Q4, false, 1, true>(a, p, st) : launch_act<XG_Q4, false, 1, false>(a, p, st);
         return act ? launch_act<XG_Q4, true, 1, true>(a, p, st) : launch_act<XG_Q4, true, 1, false>(a, p, st);
     }
+    if (c.x_f16 && xg_chained(c.fmt, 1, K)) {
+        a.xp = static_cast<const _Float16*>(c.x);
+        return act ? launch_act<XG_I8, false, 1, true, false>(a, p, st) : launch_act<XG_I8, false, 1, false, false>(a, p, st);
+    }
     if (c.x_f16) {
-        if (a.Kp == K) {
-            a.xp = static_cast<const _Float16*>(c.x);
-        } else {
-            const size_t units = (size_t)M * a.Kp / 8;
-            hipLaunchKernelGGL(pad_x_kernel, dim3((unsigned)std::min<size_t>((units + 255) / 256, 4096)), dim3(256), 0, st,
-                               static_cast<const _Float16*>(c.x), K, a.Kp, units, xp);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-        }
+        const size_t units = (size_t)M * a.Kp / 8;
+        hipLaunchKernelGGL(pad_x_kernel, dim3((unsigned)std::min<size_t>((units + 255) / 256, 4096)), dim3(256), 0, st,
+                           static_cast<const _Float16*>(c.x), K, a.Kp, units, xp);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
         return act ? launch_act<XG_I8, false, 1, true>(a, p, st) : launch_act<XG_I8, false, 1, false>(a, p, st);
     }
     switch (c.fmt) {

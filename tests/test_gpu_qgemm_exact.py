@@ -404,3 +404,33 @@ def test_q4_qkv_and_gate_up_f16_rows(ops, m, rq, rkv, k, sdt):
         fn(*g[:3], *u[:3], x.cuda(), h)
         torch.cuda.synchronize()
         assert _rel(h.cpu(), _act(x.double() @ g[3].t(), x.double() @ u[3].t(), act)) <= 2 * tol, act
+
+
+# The bar is the error of kernels whose lanes sum a row's products in a tree, on the same x: int8 in calls of four f32
+# rows (1.0e-7 to 1.1e-7 here; sums of four 64-k steps 8.2e-8 to 1.1e-7, one chain over K 1.6e-7 to 4.2e-7), q4 the
+# single call, which runs one wave per row at k % 64 == 32 (1.3e-7 / 1.6e-7; steps in pairs 9.2e-8 / 1.2e-7, each onto
+# the total 1.5e-7 / 2.1e-7)
+@pytest.mark.parametrize("m,n,k", [(1100, 2048, 976), (300, 2560, 2032), (1100, 2048, 4080)])
+def test_i8_f16_rows_ragged_k_sum_as_well_as_single_rows(ops, m, n, k):
+    x = _x(m, k, k).half().cuda()
+    w, s = (t.cuda() for t in _i8(n, k, 3))
+    ref = torch.matmul(x.double(), w.double().t().contiguous()) * s.double()
+    y, rows = (torch.full((m, n), float("nan"), device="cuda") for _ in range(2))
+    ops.encode_qgemv_i8(w, s, x, y)
+    for r in range(0, m, 4):
+        ops.encode_qgemv_i8(w, s, x[r:r + 4].float(), rows[r:r + 4])
+    torch.cuda.synchronize()
+    assert _rel(y, ref) <= 1.05 * _rel(rows, ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(300, 2560, 2016), (1100, 2048, 4064)])
+def test_q4_f16_rows_ragged_k_sum_as_well_as_single_rows(ops, m, n, k):
+    x = _x(m, k, k).half().cuda()
+    w, s, b, dense = _q4(n, k, 3)
+    ref = torch.matmul(x.double(), dense.cuda().t().contiguous())
+    y, rows, *kv = (torch.full((m, n), float("nan"), device="cuda") for _ in range(4))
+    ops.encode_qkv_q4_affine(w, s, b, w, s, b, w, s, b, x, y, *kv)
+    ops.encode_qgemv_q4_affine(w, s, b, x, rows)
+    torch.cuda.synchronize()
+    assert _rel(y, ref) <= 1.05 * _rel(rows, ref)
+    assert torch.equal(kv[0], y) and torch.equal(kv[1], y)
