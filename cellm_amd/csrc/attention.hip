@@ -8,12 +8,12 @@
 //   - the G query heads of one (row, kv head), or
 //   - one query head of up to 16 neighbouring rows whose block tables agree over
 //     their positions: the tokens of a prompt.
-// Which of the two is found on the device: a row joins its 16-row tile if its
-// table equals the table of the tile's furthest row over its own positions.  A
-// tile of at least two such rows is computed by one block per query head (blocks
-// of those rows past the heads leave at once); any other row by its own block.
-// Sessions with pages of their own differ in their first page, which one load
-// per row shows.
+// Which of the two is found on the device: a row joins its 16-row tile's set if
+// its table equals the table of the tile's furthest row over its own positions,
+// and the set is worth sharing (rule below).  A set is computed in units of one
+// query head and one range of positions, spread over the blocks of the tile's
+// rows; any other row by its own blocks.  Sessions with pages of their own differ
+// in their first page, which one load per row shows.
 //
 // Wave w of 4 takes chunks of 32 positions, w, w + 4, ...  A chunk is
 //   S^T [32 positions][16 columns] = K . Q^T       v_mfma_f32_16x16x32_f16
@@ -31,9 +31,10 @@
 // that is not finite (an infinity or NaN in q, K or V: inf * lo may be NaN where
 // inf * v is not) is computed again by plain f32 sums.
 //
-// Long contexts split their positions over blocks: partial sums (HD values, the
-// maximum, the sum) go to the workspace with agent-coherent stores and the
-// group's last block adds them in split order, as in attn_partial_kernel.
+// Long contexts split their positions over blocks, a row's and a set's: partial
+// sums (HD values, the maximum, the sum) go to the workspace with agent-coherent
+// stores and the last block of the row's or of the set's head adds them in split
+// order, as in attn_partial_kernel.
 #include <algorithm>
 #include <cmath>
 
@@ -46,8 +47,13 @@ namespace cellm {
 
 namespace {
 
+typedef float f2_t __attribute__((ext_vector_type(2)));
+
 constexpr int kWaves = 4, kThreads = kWaves * 64, kCols = 16, kChunk = 32;
 constexpr int kMinSplit = kWaves * kChunk;  // positions: a chunk per wave
+// rows share where their own positions have no splits, or up to kShareSplits of at least kSharePositions
+constexpr int kShareSplits = 6, kSharePositions = 1024;
+constexpr int kMinTileSplit = 256, kMaxTileSplits = 32;  // positions of a set's split, splits
 constexpr int kVStride = kChunk + 4;  // halves between the dims of a transposed V chunk
 
 struct AttnArgs {
@@ -60,7 +66,8 @@ struct AttnArgs {
     int rows, n_heads, n_kv, group, layer, window, tiles;
     float scale, soft_cap;
     int nsplit, cap;        // splits of a row's positions at most; positions of a table
-    float* part;            // [row][kv head][split][group][HD + 2]
+    int tsplit, slots;      // splits of a shared tile's positions at most; slots for splits in `part`
+    float* part;            // [row][kv head][slot][group][HD + 2]
     uint32_t* counters;     // per (row, kv head): splits done, zero between calls
     float* out;
 };
@@ -68,6 +75,10 @@ struct AttnArgs {
 __device__ __forceinline__ bool finite_f32(float v) { return (__builtin_bit_cast(uint32_t, v) & 0x7F800000u) != 0x7F800000u; }
 __device__ __forceinline__ void st_agent(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float ld_agent(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ f2_t ld_agent2(const float* p)  // 8-byte aligned
+{
+    return __builtin_bit_cast(f2_t, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
 __device__ __forceinline__ int first_position(int seq, int window) { return window > 0 ? max(seq - window, 0) : 0; }
 // LDS of one wave, written and read across its lanes: the wave's LDS operations run in order, and the
 // compiler moves none across this
@@ -172,7 +183,7 @@ __device__ __forceinline__ int block_row(const AttnArgs& a, int i)
 
 // Registers: four waves per SIMD at HD 64 (a 2048-token prompt of 14 / 2 heads 74 us at three, 67 at four); HD 128
 // needs the registers of three.  Measured, us, vector kernels -> this: prompts of 512 and 2048 tokens, 14 / 2 heads
-// of 64, 90 -> 15 and 589 -> 67; 1024 tokens at 2048 positions, 32 / 8 heads of 128, 1586 -> 182; 8 sessions at
+// of 64, 90 -> 13 and 589 -> 58; 1024 tokens at 2048 positions, 32 / 8 heads of 128, 1586 -> 182; 8 sessions at
 // 4096..8192 positions, 32 / 8 heads of 128, 86 -> 56 (3.6 TB/s), 16 sessions at 8192..16384, 8 / 8 heads of 128,
 // 190 -> 176 (4.6 TB/s).  Prompts are bound by the latency of a chunk (page, K, scores, maximum, weights, V in LDS)
 // at about two waves per SIMD, long contexts by memory.  The error against 64 bits is no larger than the vector
@@ -196,7 +207,6 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int c = lane & 15, g4 = lane >> 4;
     const int r = block_row(a, blockIdx.x / a.n_kv), kvh = blockIdx.x % a.n_kv, sp = blockIdx.y;
-    const int gid = r * a.n_kv + kvh;
     const int cap = a.cap, kvd = a.n_kv * HD;
 
     // ---- positions and first pages of the tile's rows, and the first chunk's page entry
@@ -226,12 +236,21 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
         const uint32_t* lead = a.bt + (size_t)(tile0 + leader) * a.max_blocks;
         lead_first = lead[b_first];
         members = (uint32_t)__ballot(pj > 0 && first == (uint32_t)__builtin_amdgcn_readlane((int)first, leader)) & 0xFFFFu;
-        if (__popc(members) >= 2) {
+        // Worth sharing: a row by itself fills `group` of the 16 columns, a set one per row, and its last block adds
+        // 16 columns where a row's adds `group`.  us, each row by itself / a set, 1 set and 2 and 4 (16, 32, 64 rows of
+        // one session): 14/2 heads of 64, 8192 positions 20.6 / 28.1, 25.7 / 29.7, 38.2 / 33.9; 2048 16.7 / 17.3, 17.8 /
+        // 18.4, 19.1 / 19.6; 32/8 of 128, 8192 64.9 / 42.8, 110 / 51, 154 / 73; 1024 20.4 / 21.4, 27.0 / 22.9, 26.7 / 26.7.
+        // Two rows of 14/2 heads at 8192 positions took 371 us as a set with one block per head, 17 so.
+        const int span = a.window > 0 ? min(seq_lead, a.window) : seq_lead;
+        if (__popc(members) < max(a.group, 2) ||
+            (a.nsplit > 1 && (a.nsplit > kShareSplits || span < a.nsplit * kSharePositions)))
+            members = 0;
+        if (members) {
             // whole tables: thread t compares entries t / 16, t / 16 + 16, ... of tile row t % 16 (that is c); of
             // every candidate where this block needs the set, of its own row where that is all
             if (t == 0) flags = 0;
             __syncthreads();
-            const bool mine = (members >> c & 1) && c != leader && (c == sub || sub < a.group || sub == leader);
+            const bool mine = (members >> c & 1) && c != leader && (c == sub || sub < a.group || sub == leader || a.tsplit > 1);
             const int nb = mine ? (pj + a.tpb - 1) / a.tpb : 0;
             const uint32_t* own = a.bt + (size_t)jr * a.max_blocks;
             bool differ = false;
@@ -261,25 +280,35 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
     _Float16* const vt = reinterpret_cast<_Float16*>(my_lds);
     const bool in_set = members >> sub & 1;
 
-    // pass h < group: the tile's rows, query head h; pass group: this row's heads
-    for (int h = 0; h <= a.group; ++h) {
-        const bool solo = h == a.group;
-        if (solo ? in_set : (members == 0 || sp != 0 || h % nr != sub)) continue;
+    // The shared set: positions lo_set..seq_lead in `tsplits` parts, one unit per query head and part
+    int lo_set = 0, tsplits = 1, tper = 0;
+    if (members) {
+        if (a.window > 0) {
+            lo_set = members >> c & 1 ? first_position(pj, a.window) : cap;
+#pragma unroll
+            for (int o = 8; o > 0; o >>= 1) lo_set = min(lo_set, __shfl_xor(lo_set, o));
+            lo_set = __builtin_amdgcn_readfirstlane(lo_set) & ~(kChunk - 1);
+        }
+        const int len = seq_lead - lo_set;
+        const int n = len < 4 * kMinTileSplit ? 1 : max(1, min(min(a.tsplit, nr * a.nsplit / a.group), len / kMinTileSplit));
+        tper = __builtin_amdgcn_readfirstlane(((len + n - 1) / n + kChunk - 1) & ~(kChunk - 1));
+        tsplits = __builtin_amdgcn_readfirstlane((len + tper - 1) / tper);
+    }
+    const int units = members ? a.group * tsplits : 0;
+
+    // the set's units, spread over the blocks of the tile's rows, then this row's heads if it is not in the set
+    for (int u = sub + nr * sp;; u += nr * a.nsplit) {
+        const bool solo = u >= units;
+        if (solo && in_set) break;
+        const int ts = solo ? sp : __builtin_amdgcn_readfirstlane(u / a.group), h = solo ? 0 : u - ts * a.group;
         // column c: its positions, and those of the whole block
         const bool has = solo ? c < a.group : members >> c & 1;
         const int seq_c = has ? (solo ? seq_own : pj) : 0;
         const int s0_c = first_position(seq_c, a.window);
         const int hi = solo ? seq_own : seq_lead;
-        if (hi <= 0) continue;  // no position: nothing written
-        int lo = 0;
-        if (a.window > 0) {
-            lo = has ? s0_c : cap;
-#pragma unroll
-            for (int o = 8; o > 0; o >>= 1) lo = min(lo, __shfl_xor(lo, o));
-            lo = __builtin_amdgcn_readfirstlane(lo);
-        }
+        if (hi <= 0) break;  // no position: nothing written
         const int table = solo ? r : tile0 + leader;
-        int t0 = lo & ~(kChunk - 1), t1 = hi, splits = 1;
+        int t0 = solo ? first_position(hi, a.window) & ~(kChunk - 1) : lo_set, t1 = hi, splits = tsplits, per = tper;
         if (solo) {
             // Rows past half their table take shares of the table, the others (and windows) spread their own
             // positions over all splits.  us, shares / spread: 8 rows, 32/8 heads of 128, table of 8192, positions
@@ -288,13 +317,13 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
             // window 2048 of 8192 47.3 / 33.9
             const int len = hi - t0, over = 2 * len >= a.cap ? a.cap : len;
             // (the divisions run on the vector unit: their results go back to scalars)
-            const int per = __builtin_amdgcn_readfirstlane(
+            per = __builtin_amdgcn_readfirstlane(
                 max(kMinSplit, ((over + a.nsplit - 1) / a.nsplit + kChunk - 1) & ~(kChunk - 1)));
             splits = __builtin_amdgcn_readfirstlane((len + per - 1) / per);
-            if (sp >= splits) continue;
-            t0 += sp * per;
-            t1 = min(hi, t0 + per);
+            if (sp >= splits) break;
         }
+        t0 += ts * per;
+        t1 = min(hi, t0 + per);
         if (t == 0) splits_s = splits;  // read after the barriers below
 
         // ---- q: two f16 parts of every column in LDS (wave 0; lane (c, g4): dims 32 kk + 8 g4 + 0..7)
@@ -484,7 +513,12 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
         __syncthreads();
         const int nsp = __builtin_amdgcn_readfirstlane(splits_s);
         const bool split = nsp > 1;
-        float* const grp = a.part + (size_t)gid * a.nsplit * a.group * (HD + 2);
+        // column oc's partials of split 0, and the floats between splits
+        const auto partial_of = [&](int oc) {
+            const int row = solo ? r : tile0 + oc, head = solo ? oc : h;
+            return a.part + ((size_t)(row * a.n_kv + kvh) * a.slots * a.group + head) * (HD + 2);
+        };
+        const size_t split_step = (size_t)a.group * (HD + 2);
         for (int i = t; i < kCols * (HD / 4); i += kThreads) {
             const int oc = i / (HD / 4), d4 = i % (HD / 4);
             if (solo ? oc >= a.group : !(members >> oc & 1)) continue;
@@ -500,7 +534,7 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
                 acc = acc + *reinterpret_cast<const f4_t*>(reinterpret_cast<const float*>(wave_lds + w * kWaveLds) + oc * OS + 4 * d4) * ew;
             }
             if (split) {
-                float* p = grp + ((size_t)sp * a.group + oc) * (HD + 2);
+                float* p = partial_of(oc) + ts * split_step;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) st_agent(p + 4 * d4 + k, acc[k]);
                 if (d4 == 0) {
@@ -516,27 +550,36 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
                 atomicOr(&flags, 1u << oc);
         }
         if (split) {
-            // this block's partials are performed at the coherence point before it counts itself
+            // this block's partials are performed at the coherence point before it counts itself.  A row counts on its
+            // own counter; head h of a set on byte h % 4 of the counter of the set's first row, or second for h >= 4
+            // (a set has two rows or more, and they count nothing of their own)
+            const uint32_t rest = members & (members - 1);
+            const int crow = solo ? r : tile0 + __builtin_ctz(h < 4 ? members : rest), shift = solo ? 0 : 8 * (h & 3);
+            uint32_t* const counter = a.counters + crow * a.n_kv + kvh;
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
             if (t == 0)
-                last = __hip_atomic_fetch_add(a.counters + gid, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                last = (__hip_atomic_fetch_add(counter, 1u << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> shift & 255u) ==
                        (uint32_t)(nsp - 1);
             __syncthreads();
-            if (!last) return;  // the pass of this row's heads is the last one
-            // split maxima and sums to LDS, then weights e^(m_k - M), then HD values per head, eight loads at a time
-            const int n = nsp;
-            const float* base = grp;
-            const size_t step = (size_t)a.group * (HD + 2);
-            float* mk = reinterpret_cast<float*>(wave_lds);   // [group][n], then the weights
-            float* lk = mk + a.group * n;
-            for (int i = t; i < a.group * n; i += kThreads) {
-                const float* p = base + (size_t)(i % n) * step + (size_t)(i / n) * (HD + 2) + HD;
+            if (!last) {
+                if (solo) break;
+                continue;
+            }
+            // split maxima and sums to LDS, then weights e^(m_k - M), then HD values per column, eight loads at a time
+            const int n = nsp, cols = solo ? a.group : kCols;
+            float* mk = reinterpret_cast<float*>(wave_lds);   // [column][n], then the weights
+            float* lk = mk + cols * n;
+            for (int i = t; i < cols * n; i += kThreads) {
+                const int oc = i / n;
+                if (!solo && !(members >> oc & 1)) continue;
+                const float* p = partial_of(oc) + (size_t)(i - oc * n) * split_step + HD;
                 mk[i] = ld_agent(p);
                 lk[i] = ld_agent(p + 1);
             }
             __syncthreads();
-            for (int oc = wave; oc < a.group; oc += kWaves) {
+            for (int oc = wave; oc < cols; oc += kWaves) {
+                if (!solo && !(members >> oc & 1)) continue;
                 float mm = -INFINITY, ll = 0.0f;
                 for (int k = lane; k < n; k += 64) mm = fmaxf(mm, mk[oc * n + k]);
                 mm = group_max<64>(mm);
@@ -549,24 +592,26 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
                 if (lane == 0) ml[0][0][oc] = ll;
             }
             __syncthreads();
-            for (int i = t; i < a.group * HD; i += kThreads) {
-                const int oc = i / HD;
-                const float* p = base + (size_t)oc * (HD + 2) + i % HD;
-                float acc = 0.0f;
+            for (int i = t; i < cols * (HD / 2); i += kThreads) {
+                const int oc = i / (HD / 2), d = 2 * (i % (HD / 2));
+                if (!solo && !(members >> oc & 1)) continue;
+                const float* p = partial_of(oc) + d;
+                f2_t acc = {0.0f, 0.0f};
                 for (int k = 0; k < n; k += 8) {
-                    float v[8];
+                    f2_t v[8];
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) v[j] = ld_agent(p + (size_t)min(k + j, n - 1) * step);
+                    for (int j = 0; j < 8; ++j) v[j] = ld_agent2(p + (size_t)min(k + j, n - 1) * split_step);
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
                         if (k + j < n) acc = acc + v[j] * mk[oc * n + k + j];
                 }
                 const float ll = ml[0][0][oc];
                 acc = acc * (ll > 0.0f ? 1.0f / ll : 0.0f);
-                a.out[((size_t)r * a.n_heads + kvh * a.group + oc) * HD + i % HD] = acc;
-                if (!finite_f32(acc) || !finite_f32(ll)) atomicOr(&flags, 1u << oc);
+                const int row = solo ? r : tile0 + oc, head = kvh * a.group + (solo ? oc : h);
+                *reinterpret_cast<f2_t*>(a.out + ((size_t)row * a.n_heads + head) * HD + d) = acc;
+                if (!finite_f32(acc[0]) || !finite_f32(acc[1]) || !finite_f32(ll)) atomicOr(&flags, 1u << oc);
             }
-            if (t == 0) __hip_atomic_store(a.counters + gid, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (t == 0) __hip_atomic_fetch_sub(counter, (uint32_t)n << shift, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
         const uint32_t again = flags;
@@ -574,6 +619,7 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
             if (again >> oc & 1)
                 plain_attention<HD>(a, solo ? r : tile0 + oc, kvh * a.group + (solo ? oc : h),
                                     reinterpret_cast<float*>(wave_lds));
+        if (solo) break;
         __syncthreads();
     }
 }
@@ -613,6 +659,10 @@ hipError_t launch_attention_mma(const float* q, const uint16_t* kcache, const ui
     // a 2048-token prompt of 14 / 2 heads with four splits 186 us, with one 126)
     const int want = std::min(max_splits, std::max(1, 512 / (rows * n_kv_heads)));
     a.nsplit = std::min(want, (cap + 511) / 512);
+    a.slots = (cap + 63) / 64;  // as attention_workspace_bytes counts them
+    // sets of all tiles' heads: 512 blocks
+    const int tiles = (rows + kCols - 1) / kCols;
+    a.tsplit = max_splits == 1 ? 1 : std::min({kMaxTileSplits, a.slots, std::max(1, 512 / (tiles * n_heads))});
     a.cap = cap;
     a.part = part;
     a.counters = counters;
