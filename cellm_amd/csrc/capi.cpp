@@ -1730,7 +1730,7 @@ int32_t cellm_hip_argmax_f32(cellm_hip_ctx_t* ctx, const float* logits, int64_t 
     // and returned to zero by every launch
     float* scratch = nullptr;
     if (int32_t rc = get_stream_buffer(ctx, ctx->argmax, st, argmax_scratch_bytes((int)rows, (int)n), &scratch,
-                                       argmax_counter_bytes((int)rows)))
+                                       argmax_counter_bytes()))
         return rc;
     HIP_TRY(launch_argmax(logits, (int)rows, (int)n, out_index, out_value, scratch, st), "argmax launch");
     return CELLM_HIP_OK;

@@ -2263,12 +2263,14 @@ hipError_t launch_qgemv_q4_x32(const uint32_t* wq, const float* S, const float* 
 
 int argmax_chunks(int n) { return std::max(1, (n + kArgmaxChunk - 1) / kArgmaxChunk); }
 
-size_t argmax_counter_bytes(int rows) { return (((size_t)rows * sizeof(uint32_t)) + 255) & ~(size_t)255; }
+// of 65536 rows, whatever the call has: scratch that held fewer rows' counters holds their partials where more
+// rows count
+size_t argmax_counter_bytes() { return 65536 * sizeof(uint32_t); }
 
 size_t argmax_scratch_bytes(int rows, int n)
 {
     const int nch = argmax_chunks(n);
-    return nch == 1 ? 0 : argmax_counter_bytes(rows) + (size_t)rows * nch * sizeof(float2);
+    return nch == 1 ? 0 : argmax_counter_bytes() + (size_t)rows * nch * sizeof(float2);
 }
 
 hipError_t launch_argmax_keys(const float* logits, int rows, int n, uint64_t* keys, hipStream_t st)
@@ -2283,7 +2285,7 @@ hipError_t launch_argmax(const float* logits, int rows, int n, int32_t* idx, flo
     if (nch > 1 && !scratch) return hipErrorInvalidValue;
     uint32_t* cnt = reinterpret_cast<uint32_t*>(scratch);
     float2* part = nch > 1 ? reinterpret_cast<float2*>(reinterpret_cast<unsigned char*>(scratch) +
-                                                        argmax_counter_bytes(rows))
+                                                        argmax_counter_bytes())
                            : nullptr;
     hipLaunchKernelGGL(argmax_kernel, dim3(nch, rows), dim3(kArgmaxThreads), 0, st, logits, n, idx, val, cnt, part);
     return hipGetLastError();

@@ -188,7 +188,7 @@ hipError_t launch_attention_mma(const float* q, const uint16_t* kcache, const ui
 // one chunk need scratch of argmax_scratch_bytes whose first argmax_counter_bytes (the per-row
 // counters) are zero before the first call and are left at zero by every call.
 size_t argmax_scratch_bytes(int rows, int n);
-size_t argmax_counter_bytes(int rows);
+size_t argmax_counter_bytes();
 hipError_t launch_argmax(const float* logits, int rows, int n, int32_t* idx, float* val, void* scratch, hipStream_t st);
 // The same first maximum per row as a packed key (value order in the high word, 0xffffffff - index
 // in the low word) merged into keys[r] by one 64-bit atomic max per chunk block: keys start at zero;

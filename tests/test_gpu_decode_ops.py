@@ -830,3 +830,23 @@ def test_attention_workspace_growth():
                     assert rel_err(got[r], ref) <= 1e-5, (rep, rows, r)
     finally:
         o.close()
+
+
+def test_argmax_of_more_rows_in_the_scratch_of_longer_ones():
+    """Four rows of 64 chunks leave their partials where a later call of 100 rows, in the same scratch, counts."""
+    import torch
+
+    from cellm_amd import HipOps
+
+    own = HipOps(0)
+    try:
+        g = torch.Generator(device="cuda").manual_seed(3)
+        for rows, n in ((4, 262144), (100, 5000), (100, 5000), (4, 262144)):
+            z = torch.randn(rows, n, generator=g, device="cuda")
+            idx = torch.full((rows,), -1, dtype=torch.int32, device="cuda")
+            val = torch.empty(rows, device="cuda")
+            own.encode_argmax(z, idx, val)
+            torch.cuda.synchronize()
+            assert torch.equal(idx.long(), z.argmax(1)) and torch.equal(val, z.max(1).values), (rows, n)
+    finally:
+        own.close()
