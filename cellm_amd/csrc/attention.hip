@@ -67,6 +67,7 @@ struct AttnArgs {
     float scale, soft_cap;
     int nsplit, cap;        // splits of a row's positions at most; positions of a table
     int tsplit, slots;      // splits of a shared tile's positions at most; slots for splits in `part`
+    int busy;               // rows of a shared tile whose blocks have a unit of it, at most
     float* part;            // [row][kv head][slot][group][HD + 2]
     uint32_t* counters;     // per (row, kv head): splits done, zero between calls
     float* out;
@@ -163,12 +164,12 @@ __device__ __forceinline__ void plain_attention(const AttnArgs& a, int row, int 
 }
 
 // Row of the i-th block of a kv head.  The last tile first (in a prompt its rows see the most positions), and
-// the rows a shared tile needs blocks of (one per query head) before those whose blocks then leave at once:
-// blocks go to the XCDs in turn, and with the rows in order one XCD in four had half the others' work (a
+// the rows a shared tile needs blocks of (one per query head and split) before those whose blocks then leave at
+// once: blocks go to the XCDs in turn, and with the rows in order one XCD in four had half the others' work (a
 // 2048-token prompt of 14 / 2 heads 126 us in row order, 74 so).
 __device__ __forceinline__ int block_row(const AttnArgs& a, int i)
 {
-    const int full = a.rows / kCols, rem = a.rows - full * kCols, g = a.group, first = min(rem, g);
+    const int full = a.rows / kCols, rem = a.rows - full * kCols, g = a.busy, first = min(rem, g);
     const int active = full * g + first;
     if (i < active) {
         if (i < first) return full * kCols + i;
@@ -663,6 +664,7 @@ hipError_t launch_attention_mma(const float* q, const uint16_t* kcache, const ui
     // sets of all tiles' heads: 512 blocks
     const int tiles = (rows + kCols - 1) / kCols;
     a.tsplit = max_splits == 1 ? 1 : std::min({kMaxTileSplits, a.slots, std::max(1, 512 / (tiles * n_heads))});
+    a.busy = std::min(kCols, a.group * a.tsplit);
     a.cap = cap;
     a.part = part;
     a.counters = counters;
