@@ -1816,6 +1816,34 @@ size_t attention_workspace_bytes(int rows, int n_heads, int n_kv_heads, int head
 
 size_t attention_counter_bytes() { return kAttnCounterBytes; }
 
+// The MFMA kernel reads K and V once for the query heads of a kv head, and for rows that share their pages, but
+// starts later than the others and takes 1.4 us (heads of 64) or 2 us (128) per 128 positions of a block.
+// Tables of up to 512 positions: the others run a block per row and query head, 6 us up to about 500 blocks and 10
+// more per 1000.  Larger tables: they take their time by the elements read, the MFMA kernel by the positions, and
+// more than most with one to three heads per kv head, where its 16 columns are mostly empty unless rows share pages.
+// Tables of 8192 and more go to it at any size: many 64-position chunks cost the others' last block.
+// us, others / MFMA, rows (P: of one prompt), heads / kv heads, head_dim, table:
+//   P 64, 14/2, 64, 64      11.0 / 7.9    P 128, 8/8, 64, 128    10.4 / 8.5    P 32, 14/2, 64, 512     8.8 / 12.9
+//   P 64, 14/2, 64, 512     15.1 / 12.9   P 128, 4/1, 64, 512     8.8 / 13.1   128, 8/8, 64, 512      20.7 / 24.8
+//   P 64, 8/1, 128, 256      8.9 / 13.5   35, 16/2, 128, 224     15.1 / 12.2   P 256, 8/8, 64, 384    26.4 / 11.9
+//   P 32, 8/1, 128, 512      9.5 / 17.8   13, 32/4, 128, 432     20.2 / 16.9   64, 8/8, 128, 256      12.0 / 17.1
+//   32, 14/2, 64, 1024      18.7 / 15.2   P 32, 15/5, 64, 1024   14.3 / 16.8   P 64, 8/8, 64, 1536    26.7 / 18.7
+//   P 32, 8/8, 128, 1024    16.2 / 26.6   P 64, 8/8, 128, 1024   25.6 / 25.8   P 128, 8/8, 128, 1024  42.6 / 26.0
+//   32, 6/2, 128, 1024      13.7 / 19.0   64, 6/2, 128, 1536     23.5 / 23.1   32, 12/2, 128, 768     20.3 / 17.7
+//   8, 6/2, 128, 4096       21.3 / 19.0   16, 8/8, 64, 4096      26.1 / 25.7   4, 15/5, 64, 8192       38.2 / 18.7
+static bool attention_mma_faster(int rows, int n_heads, int group, int head_dim, int cap, int window)
+{
+    const int64_t blocks = (int64_t)rows * n_heads;
+    if (cap <= 2 * kAttnBlockSub)
+        return blocks >= (head_dim == 64 ? (group == 1 ? 1536 : 704) : cap > kAttnBlockSub ? (group == 1 ? 768 : 320)
+                                                                                          : (group == 1 ? 1024 : 544));
+    if (window == 0 && cap >= 8192) return true;
+    const int span = window > 0 ? std::min(window, cap) : cap;
+    const double reads = (double)blocks * head_dim * span;
+    const double from = head_dim == 64 ? (group >= 4 ? 24e6 : 36e6) : (group >= 4 ? 30e6 : group == 3 ? 45e6 : 90e6);
+    return reads >= (span >= 4096 ? std::min(from, 28e6) : from);
+}
+
 hipError_t launch_attention_gqa_f16kv(const float* q, const uint16_t* kcache, const uint16_t* vcache,
                                       const uint32_t* block_tables, int max_blocks, int total_blocks,
                                       const int32_t* pos, int rows, int n_heads, int n_kv_heads, int head_dim,
@@ -1836,17 +1864,9 @@ hipError_t launch_attention_gqa_f16kv(const float* q, const uint16_t* kcache, co
     const bool one_launch = rows * n_kv_heads <= kAttnCounters;
     const int cap = max_blocks * tokens_per_block;
     const dim3 hgrid((unsigned)(rows * n_heads));
-    // The MFMA kernel reads K and V once for all query vectors that share them and starts later than the
-    // others (8 us at any size): it takes the calls with much to read, and long contexts, whose many 64-position
-    // chunks cost the split form's last block.  Measured, us, vector kernels / MFMA (rows, heads / kv heads,
-    // head_dim, positions): 16, 15/5, 64, 512: 8.4 / 12.5; 64, 14/2, 64, 512: 20.0 / 13.9; 16, 32/8, 128, 512:
-    // 24.6 / 17.9; 4, 15/5, 64, 2048: 13.2 / 15.2; 16, 32/8, 128, 2048: 43.5 / 32.3; 1, 14/2, 64, 16384: 32.8 /
-    // 17.9; 8, 32/8, 128, window 512 of 4096: 14.6 / 20.9; prompts of 64 and 512 tokens, 14/2, 64: 11.0 / 8.8 and
-    // 90 / 15.
-    const double reads = (double)rows * n_heads * head_dim * (window > 0 ? std::min(window, cap) : cap);
     const bool vec16 = ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kcache) |
                          reinterpret_cast<uintptr_t>(vcache) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    if (vec16 && (reads >= (rows >= 32 ? 3e6 : 20e6) || (window == 0 && cap >= 8192)))
+    if (vec16 && attention_mma_faster(rows, n_heads, G, head_dim, cap, window))
         return launch_attention_mma(q, kcache, vcache, block_tables, max_blocks, total_blocks, pos, rows, n_heads,
                                     n_kv_heads, head_dim, n_layers, tokens_per_block, layer, scale, soft_cap, window,
                                     one_launch && cap > 2 * kAttnBlockSub ? 64 : 1, part, counters, out, st);

@@ -503,13 +503,11 @@ int32_t cellm_hip_decode_q4_affine_gate_up_silu(cellm_hip_ctx_t* ctx, const floa
  * owned by the context, per stream: 64 KB of group counters, zeroed when the
  * workspace is allocated and left at zero by every call, then the partials).
  * More than 16384 (row, kv head) groups take a second combine launch.
- * Calls with much to read (rows * n_heads * head_dim * positions >= 20e6, or
- * >= 3e6 at 32 rows and more; positions = window or the table's) and tables of
- * 8192 positions and more, with 16-byte aligned q, caches and out, run on f16
- * MFMA instead: neighbouring rows whose tables agree over their positions (the
- * tokens of a prompt) share each K and V read, q and the softmax weights are
- * multiplied as two f16 parts each, and the same workspace holds the partials
- * of splits of at least 512 positions. */
+ * Calls with much to read and tables of 8192 positions and more, with 16-byte
+ * aligned q, caches and out, run on f16 MFMA instead: many neighbouring rows
+ * whose tables agree over their positions (the tokens of a prompt) share each
+ * K and V read, q and the softmax weights are multiplied as two f16 parts each,
+ * and the same workspace holds the partials of splits of the positions. */
 int32_t cellm_hip_attention_gqa_f16kv(cellm_hip_ctx_t* ctx, const float* q, const uint16_t* kcache,
                                       const uint16_t* vcache, const uint32_t* block_tables, int64_t max_blocks,
                                       int64_t total_blocks, const int32_t* positions, int64_t rows, int64_t n_heads,
