@@ -298,3 +298,65 @@ def test_dispatch_takes_no_slower_kernel(ops, rows, nh, nkv, hd, ctx, shared):
     chosen, others = _time(lambda: call(out), 30), _time(lambda: call(other), 30)
     assert _rel(out, other.double()) <= 2 * TOL
     assert chosen <= 1.5 * others, (chosen, others)
+
+
+# rows by themselves in splits, one and with pages of their own; a set in splits; a set without (masked positions among
+# its chunks)
+@pytest.mark.parametrize("rows,nh,nkv,hd,ctx,shared", [(1, 8, 2, 64, 8192, True), (3, 8, 2, 128, 8192, False),
+                                                       (16, 32, 8, 64, 5000, True), (100, 8, 2, 64, 304, True)])
+def test_non_finite_elements_in_splits_and_sets(ops, rows, nh, nkv, hd, ctx, shared):
+    """Infinities and NaN of K, V and q reach the outputs that they reach in a plain f32 softmax over the row's own
+    positions: not those of rows that end before them."""
+    tpb = 8
+    per = ctx // tpb
+    g = torch.Generator().manual_seed(ctx)
+    kc, vc = _cache(per * (1 if shared else rows), 1, tpb, nkv, hd, ctx)
+    bt = torch.arange(per)[None].repeat(rows, 1) if shared else torch.arange(per * rows).view(rows, per)
+    pos = torch.arange(ctx - rows, ctx)
+    q = torch.randn(rows, nh, hd, generator=g)
+    q[:, :, 0] = q[:, :, 0].abs() + 0.5
+    late = per - 2  # of the last pages: past the positions of the first rows of a long session
+    for r in range(1 if shared else rows):
+        base = int(bt[r, 0])
+        kc[base, 0, 3, 0, 0] = float("-inf")            # weight 0 for the queries of kv head 0
+        vc[base + 1, 0, 5, 0, 1] = float("inf")         # a value of +inf in dim 1 of kv head 0
+        vc[base + per // 2, 0, 6, 1, 2] = float("nan")  # dim 2 of kv head 1
+        kc[base + late, 0, 1, 1, 0] = float("inf")      # a score of +inf: NaN
+        vc[base + per - 1, 0, 7, 0, 3] = float("-inf")
+    if rows > 2:
+        q[2, nh - 1, 5] = float("nan")
+    got = _run(ops, q, kc, vc, bt, pos, 0)
+    got2 = _run(ops, q, kc, vc, bt, pos, 0)
+    ref = torch.zeros_like(got)
+    for r in range(rows):
+        t = torch.arange(int(pos[r]) + 1)
+        for h in range(nh):
+            k, v = (c[bt[r, t // tpb], 0, t % tpb, h // (nh // nkv)].float() for c in (kc, vc))
+            s = (k * q[r, h]).sum(1) * (1 / math.sqrt(hd))
+            p = torch.exp(s - s.nan_to_num(-math.inf, math.inf, -math.inf).max())
+            ref[r, h] = (p[:, None] * v).sum(0) / p.sum()
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(torch.isposinf(got), torch.isposinf(ref)) and torch.equal(torch.isneginf(got), torch.isneginf(ref))
+    fine = torch.isfinite(ref)
+    assert _rel(got[fine], ref[fine].double()) <= 5e-6  # the reference is f32 too
+    assert torch.equal(got2.nan_to_num(7.0), got.nan_to_num(7.0))  # the counters are back at zero
+
+
+# the time of a call with one NaN in its first page, in times of the call without: 21 and 6 where the plain sums run over
+# the block's positions with a score a thread; 550 and 2500 where one block summed whole rows with a score per output
+@pytest.mark.parametrize("rows,nh,nkv,hd,ctx,shared", [(512, 14, 2, 64, 512, True), (8, 32, 8, 128, 8192, False)])
+def test_non_finite_value_costs_no_more_than_its_blocks(ops, rows, nh, nkv, hd, ctx, shared):
+    tpb = 16
+    per = ctx // tpb
+    total = per * (1 if shared else rows)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    kc, vc = (torch.randn(total * tpb * nkv * hd, generator=g, device="cuda").half() for _ in range(2))
+    bt = torch.arange(total, device="cuda", dtype=torch.int32).view(-1, per).expand(rows, per).contiguous()
+    pos = torch.arange(ctx - rows, ctx, device="cuda", dtype=torch.int32)
+    q = torch.randn(rows, nh * hd, generator=g, device="cuda")
+    out = torch.empty_like(q)
+    call = lambda: ops.encode_attention(q, kc, vc, bt, pos, out, nh, nkv, hd, total, 1, tpb, 0)
+    fine = _time(call)
+    vc[5] = float("nan")  # position 0 of the first row's session
+    bad = _time(call, 3)
+    assert bool(torch.isnan(out[0, 5])) and bad <= 40 * fine, (bad, fine)
