@@ -29,8 +29,8 @@
 // over two steps 9.7e-8 / 1.1e-7 / 1.2e-7, over four 1.3e-7 / 1.4e-7 / 1.4e-7, the
 // one-wave-per-row kernels 9.7e-8 / 1.3e-7 / 1.7e-7 / 2.1e-7); against chains over
 // four steps this costs 4-5 % of the wide shapes' time.
-// Results that are not finite (an infinity or NaN in x or w, or an overflow: the
-// split turns inf into inf * lo) are recomputed by a plain f32 sum.
+// Results that are not finite (an infinity or NaN in x or w, or an overflow) are
+// recomputed by plain f32 sums where these may differ (kPlain).
 //
 // Measured, int8 at 512 rows (us, one-wave-per-row kernel -> this one with its
 // split of x): 960 -> 960 1963 -> 20, 2560 -> 960 5098 -> 25, 4096 -> 4096
@@ -165,32 +165,59 @@ __device__ __forceinline__ float scale_at(const void* s, int sdt, size_t i)
     return sdt == DT_F32 ? load_f32<DT_F32>(s, i) : sdt == DT_F16 ? load_f32<DT_F16>(s, i) : load_f32<DT_BF16>(s, i);
 }
 
-// sum_k w[n,k] x[m,k] by a plain f32 loop: the results that MFMA left non-finite
+// Results that MFMA leaves non-finite may be finite or another infinity in a plain sum where the weights' side can
+// be infinite (f16 weights, group scales): inf * lo, or s inf - 8 s inf.  int8 and i4 under row scales are what a plain
+// sum gives: exact finite weights, lo = 0 beside an infinite hi, one product each.
+template <int FMT>
+constexpr bool kPlain = FMT == XG_F16 || FMT == XG_Q4;
+
+// sum_k w[n,k] x[m,k] by plain f32 sums, eight chains: the results that MFMA left non-finite.  Where every output of
+// 512 x 2048 x 2048 was one, a loop of single elements took 5.9 ms (f16 weights) and 19 (q4), this 0.72 and 1.3 (the
+// one-wave-per-row kernels 1.6 and 0.76 at any input); one infinite weight 0.076 and 0.19 ms for 0.23 and 0.66.
 template <int FMT, int P>
 __device__ __forceinline__ float plain_dot(const XgArgs& a, const XgSeg& g, int m, int n)
 {
 #pragma clang fp contract(off)
     const int K = a.K;
-    const void* x = a.x;
-    float acc = 0.0f;
-    for (int k = 0; k < K; ++k) {
-        float xv;
-        if constexpr (P == 2) xv = static_cast<const float*>(x)[(size_t)m * K + k];
-        else xv = (float)static_cast<const _Float16*>(x)[(size_t)m * K + k];
-        float w;
-        if constexpr (FMT == XG_I8) w = (float)static_cast<const int8_t*>(g.w)[(size_t)n * K + k];
-        else if constexpr (FMT == XG_F16) w = (float)static_cast<const _Float16*>(g.w)[(size_t)n * K + k];
-        else w = (float)((static_cast<const uint8_t*>(g.w)[((size_t)n * K + k) >> 1] >> (4 * (k & 1))) & 15);
+    float acc[8] = {};
+    for (int k0 = 0; k0 < K; k0 += kBK) {
+        float s = 1.0f, b = 0.0f;
         if constexpr (FMT == XG_Q4) {
-            const size_t i = (size_t)n * a.gpr + k / a.group;
-            const float s = scale_at(g.gs, a.sdt, i);
-            w = g.gb ? w * s + scale_at(g.gb, a.sdt, i) : (w - 8.0f) * s;
-        } else if constexpr (FMT == XG_I4) {
-            w -= 8.0f;
+            const size_t i = (size_t)n * a.gpr + k0 / a.group;
+            s = scale_at(g.gs, a.sdt, i);
+            if (g.gb) b = scale_at(g.gb, a.sdt, i);
         }
-        acc += w * xv;
+        const int end = min(k0 + kBK, K);  // K % 8 == 0
+#pragma unroll 4
+        for (int k = k0; k < end; k += 8) {
+            float x[8], w[8];
+            if constexpr (P == 2) {
+                const f4_t* p = reinterpret_cast<const f4_t*>(static_cast<const float*>(a.x) + (size_t)m * K + k);
+                const f4_t x0 = p[0], x1 = p[1];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = i < 4 ? x0[i & 3] : x1[i & 3];
+            } else {
+                const h8_t h = *reinterpret_cast<const h8_t*>(static_cast<const _Float16*>(a.x) + (size_t)m * K + k);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = (float)h[i];
+            }
+            if constexpr (FMT == XG_F16) {
+                const h8_t h = *reinterpret_cast<const h8_t*>(static_cast<const _Float16*>(g.w) + (size_t)n * K + k);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) w[i] = (float)h[i];
+            } else {
+                const uint32_t q = static_cast<const uint32_t*>(g.w)[((size_t)n * K + k) / 8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float v = (float)(q >> (4 * i) & 15u);
+                    w[i] = g.gb ? v * s + b : (v - 8.0f) * s;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[i] = acc[i] + w[i] * x[i];
+        }
     }
-    return acc;
+    return ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
 }
 
 __device__ __forceinline__ bool finite_f32(float v) { return (__builtin_bit_cast(uint32_t, v) & 0x7F800000u) != 0x7F800000u; }
@@ -512,7 +539,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
                         v = act_mul(decltype(act)::value, v, value(sum[i][TB - 1][r], ev, sc1, bi1));
                     if (m < a.M) {
                         g.y[(size_t)m * g.n + n] = v;
-                        bad |= !finite_f32(v);
+                        if constexpr (kPlain<FMT>) bad |= !finite_f32(v);
                     }
                 }
         }
@@ -521,13 +548,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
         store(std::integral_constant<int, ACT_GELU_TANH>{});
     else
         store(std::integral_constant<int, ACT_SILU>{});
-    if (!bad) return;
-    // rolled and rare: this lane's non-finite results again (a non-finite gate or up sum makes h non-finite)
-    for (int t = 0; t < TA * TO * 16; ++t) {
-        const int i = t / (16 * TO), j = (t / 16) % TO, r = t & 15;
-        const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3), n = out_col(j);
-        if (m >= a.M || n >= g.n || finite_f32(g.y[(size_t)m * g.n + n])) continue;
-        g.y[(size_t)m * g.n + n] = plain_output<FMT, P, ACT>(a, g, gu, m, n);
+    if constexpr (kPlain<FMT>) {
+        if (!bad) return;
+        // rolled and rare: this lane's non-finite results again (a non-finite gate or up sum makes h non-finite)
+        for (int t = 0; t < TA * TO * 16; ++t) {
+            const int i = t / (16 * TO), j = (t / 16) % TO, r = t & 15;
+            const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3), n = out_col(j);
+            if (m >= a.M || n >= g.n || finite_f32(g.y[(size_t)m * g.n + n])) continue;
+            g.y[(size_t)m * g.n + n] = plain_output<FMT, P, ACT>(a, g, gu, m, n);
+        }
     }
 }
 
@@ -559,7 +588,8 @@ __global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a,
                 o[c] = act_mul(a.act, o[c],
                                (P == 2 ? ldexpf(u[c], e) : u[c]) * column_scale(gu, a.sdt, nc) +
                                    (gu.bias ? gu.bias[nc] : 0.0f));
-            if (!finite_f32(o[c])) o[c] = plain_output<FMT, P, ACT>(a, g, gu, m, nc);
+            if constexpr (kPlain<FMT>)
+                if (!finite_f32(o[c])) o[c] = plain_output<FMT, P, ACT>(a, g, gu, m, nc);
         }
         if ((g.n & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
             *reinterpret_cast<f4_t*>(y) = o;

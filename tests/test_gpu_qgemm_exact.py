@@ -434,3 +434,85 @@ def test_q4_f16_rows_ragged_k_sum_as_well_as_single_rows(ops, m, n, k):
     torch.cuda.synchronize()
     assert _rel(y, ref) <= 1.05 * _rel(rows, ref)
     assert torch.equal(kv[0], y) and torch.equal(kv[1], y)
+
+
+@pytest.mark.parametrize("m,k", [(9, 832), (70, 2560)])
+def test_i4_and_grouped_i4_non_finite(ops, m, k):
+    """inf and NaN in x, and in a group's scale, reach exactly the outputs they reach in a plain f32 sum."""
+    n = 70
+    x = _x(m, k, 8)
+    x[1, 5], x[2, 7], x[3, 0], x[3, 1] = float("inf"), float("nan"), float("inf"), float("-inf")
+    for gs in (k, 64):
+        w, s, _ = _i4(n, k, gs, 9)
+        if gs != k:
+            s[4, 2], s[5, 3] = float("inf"), float("nan")
+        w[::3, 2] |= 0x80  # k = 5 of these rows: q - 8 = 0
+        w[::3, 2] &= 0x8F
+        q = torch.stack([w.cpu() & 15, w.cpu() >> 4], 2).reshape(n, k).float() - 8
+        dense = q * s.cpu().float().repeat_interleave(gs, 1)[:, :k]
+        y = torch.empty(m, n, device="cuda")
+        ops.encode_qgemv_i4_sym(w, s, gs, x.cuda(), y, k)
+        torch.cuda.synchronize()
+        got, ref = y.cpu(), (x[:, None] * dense[None]).sum(2)
+        for f in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(f(got), f(ref)), (gs, f)
+        fine = torch.isfinite(ref)
+        assert _rel(got[fine], ref[fine]) <= 1e-5  # against f32 sums
+
+
+@pytest.mark.parametrize("m,k", [(70, 832), (70, 840), (300, 2560)])  # in place and padded
+def test_i8_f16_rows_non_finite(ops, m, k):
+    n = 70
+    x = _x(m, k, 8).half()
+    x[1, 5], x[2, 7], x[3, 0], x[3, 1] = float("inf"), float("nan"), float("inf"), float("-inf")
+    w, s = _i8(n, k, 9)
+    w[::3, 5] = 0
+    y = torch.empty(m, n, device="cuda")
+    ops.encode_qgemv_i8(w.cuda(), s.cuda(), x.cuda(), y)
+    torch.cuda.synchronize()
+    got, ref = y.cpu(), (x.float()[:, None] * w.float()[None]).sum(2) * s
+    for f in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(f(got), f(ref)), f
+    fine = torch.isfinite(ref)
+    assert _rel(got[fine], ref[fine]) <= 1e-5
+
+
+# the time of a call in times of the finite call.  One infinite weight (a column of outputs again): 9 (f16) and 20 (q4)
+# where the sums took an element at a time; an infinity in every row of x (every output again): 230 and 580, int8, which
+# needs no second sum, 170
+@pytest.mark.parametrize("fmt,one,all_", [("f16", 6, 60), ("q4", 10, 100), ("i8", 2, 2)])
+def test_non_finite_inputs_in_bounded_time(ops, fmt, one, all_):
+    m, n, k = 512, 2048, 2048
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, y = torch.randn(m, k, generator=g, device="cuda"), torch.empty(m, n, device="cuda")
+    if fmt == "f16":
+        w = (torch.randn(n, k, generator=g, device="cuda") * 0.02).half()
+        call, poison = lambda v: ops.encode_qgemv_f16(w, v, y), lambda: w[3, 7].fill_(float("inf"))
+    elif fmt == "q4":
+        w, s, b, _ = _q4(n, k, 3)
+        call, poison = lambda v: ops.encode_qgemv_q4_affine(w, s, b, v, y), lambda: s[3, 0].fill_(float("inf"))
+    else:
+        w, s = (t.cuda() for t in _i8(n, k, 3))
+        call, poison = lambda v: ops.encode_qgemv_i8(w, s, v, y), lambda: s[3].fill_(float("inf"))
+
+    def time(v):
+        call(v)
+        best = float("inf")
+        for _ in range(3):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                call(v)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    fine = time(x)
+    bad = x.clone()
+    bad[:, 7] = float("inf")
+    every = time(bad)
+    assert not bool(torch.isfinite(y).any()) and every <= all_ * fine, (every, fine)
+    poison()
+    column = time(x)
+    assert not bool(torch.isfinite(y[:, 3]).any()) and column <= one * fine, (column, fine)
