@@ -741,7 +741,10 @@ XgPlan xg_plan(int fmt, int P, const XgSeg* segs, int nseg, bool act, int M, int
     };
     int64_t blocks = tiles(chained ? 256 : 128, 256);
     p.form = 2;
-    if (blocks < 192) {
+    // up to 64 rows keep tiles of their own height however many columns there are: 5 rows of 1152 -> 262144 took 165 /
+    // 166 / 152 / 185 us (int8 / f16 / i4 / q4) in tiles of 128 rows, 75 / 111 / 57 / 87 so, 64 rows 171 / 182 / 159 / 199
+    // and 111 / 156 / 95 / 120 (single rows' kernels at 5 rows 886 / 591 / 1047 / 308)
+    if (blocks < 192 || M <= 64) {
         p.form = M > 32 ? 1 : 0;
         blocks = p.form ? tiles(P == 2 ? 64 : 128, 128) : tiles(32, 128);
     }

@@ -516,3 +516,55 @@ def test_non_finite_inputs_in_bounded_time(ops, fmt, one, all_):
     poison()
     column = time(x)
     assert not bool(torch.isfinite(y[:, 3]).any()) and column <= one * fine, (column, fine)
+
+
+def _wide(fmt, n, k):
+    """One matrix: its call over x and y, and its dense 64-bit weights."""
+    if fmt in ("i8", "i8 f16 x"):
+        w, s = (t.cuda() for t in _i8(n, k, 3))
+        return (lambda ops, x, y: ops.encode_qgemv_i8(w, s, x, y)), lambda: w.double() * s.double()[:, None]
+    if fmt == "f16":
+        w = (torch.randn(n, k, generator=torch.Generator().manual_seed(3)) * 0.02).half().cuda()
+        return (lambda ops, x, y: ops.encode_qgemv_f16(w, x, y)), lambda: w.double()
+    if fmt == "i4":
+        w, s, dense = _i4(n, k, k, 3)
+        return (lambda ops, x, y: ops.encode_qgemv_i4_sym(w, s, k, x, y, k)), lambda: dense.cuda()
+    w, s, b, dense = _q4(n, k, 3)
+    return (lambda ops, x, y: ops.encode_qgemv_q4_affine(w, s, b, x, y)), lambda: dense.cuda()
+
+
+# the tile heights of few rows over outputs wide enough for the tallest (int8 over f16 x: k not a multiple of 64)
+@pytest.mark.parametrize("fmt,k", [("i8", 96), ("i8 f16 x", 112), ("f16", 96), ("i4", 96), ("q4", 160)])
+@pytest.mark.parametrize("m", [32, 33, 64, 65])
+def test_few_rows_of_wide_outputs(ops, fmt, k, m):
+    n = 50100
+    call, dense = _wide(fmt, n, k)
+    x = _x(m, k, m).cuda()
+    x = x.half() if fmt == "i8 f16 x" else x
+    y = torch.full((m, n), float("nan"), device="cuda")
+    call(ops, x, y)
+    torch.cuda.synchronize()
+    assert _rel(y, torch.matmul(x.double(), dense().t().contiguous())) <= TOL
+
+
+@pytest.mark.parametrize("fmt", ["i8", "f16", "i4", "q4"])
+def test_five_rows_of_a_wide_output_take_less_than_128(ops, fmt):
+    n, k = 131072, 1152
+    call, _ = _wide(fmt, n, k)
+    x, y = _x(128, k, 1).cuda(), torch.empty(128, n, device="cuda")
+
+    def time(rows):
+        call(ops, x[:rows], y[:rows])
+        best = float("inf")
+        for _ in range(3):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                call(ops, x[:rows], y[:rows])
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    few, many = time(5), time(128)
+    assert few <= 0.7 * many, (few, many)  # 0.3 to 0.6; 0.8 to 0.9 in tiles of 128 rows
