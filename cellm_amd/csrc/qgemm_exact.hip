@@ -174,7 +174,7 @@ constexpr bool kPlain = FMT == XG_F16 || FMT == XG_Q4;
 // sum_k w[n,k] x[m,k] by plain f32 sums, eight chains: the results that MFMA left non-finite.  Where every output of
 // 512 x 2048 x 2048 was one, a loop of single elements took 5.9 ms (f16 weights) and 19 (q4), this 0.72 and 1.3 (the
 // one-wave-per-row kernels 1.6 and 0.76 at any input); one infinite weight 0.076 and 0.19 ms for 0.23 and 0.66.
-template <int FMT, int P>
+template <int FMT, int P, int UNROLL>
 __device__ __forceinline__ float plain_dot(const XgArgs& a, const XgSeg& g, int m, int n)
 {
 #pragma clang fp contract(off)
@@ -188,7 +188,7 @@ __device__ __forceinline__ float plain_dot(const XgArgs& a, const XgSeg& g, int 
             if (g.gb) b = scale_at(g.gb, a.sdt, i);
         }
         const int end = min(k0 + kBK, K);  // K % 8 == 0
-#pragma unroll 4
+#pragma unroll UNROLL
         for (int k = k0; k < end; k += 8) {
             float x[8], w[8];
             if constexpr (P == 2) {
@@ -227,12 +227,12 @@ __device__ __forceinline__ float column_scale(const XgSeg& g, int sdt, int n)
     return g.s ? scale_at(g.s, sdt, (size_t)n * g.s_stride) : 1.0f;
 }
 
-template <int FMT, int P, bool ACT>
+template <int FMT, int P, bool ACT, int UNROLL>
 __device__ __forceinline__ float plain_output(const XgArgs& a, const XgSeg& g, const XgSeg& gu, int m, int n)
 {
-    const float v = plain_dot<FMT, P>(a, g, m, n) * column_scale(g, a.sdt, n) + (g.bias ? g.bias[n] : 0.0f);
+    const float v = plain_dot<FMT, P, UNROLL>(a, g, m, n) * column_scale(g, a.sdt, n) + (g.bias ? g.bias[n] : 0.0f);
     if constexpr (!ACT) return v;
-    return act_mul(a.act, v, plain_dot<FMT, P>(a, gu, m, n) * column_scale(gu, a.sdt, n) + (gu.bias ? gu.bias[n] : 0.0f));
+    return act_mul(a.act, v, plain_dot<FMT, P, UNROLL>(a, gu, m, n) * column_scale(gu, a.sdt, n) + (gu.bias ? gu.bias[n] : 0.0f));
 }
 
 // S16: XG_Q4's scales are 16 bits wide.  FOLD: the sums of two K steps (int8 over f16 rows: four) meet before they
@@ -555,7 +555,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void qgemm_exact_kernel(const XgAr
             const int i = t / (16 * TO), j = (t / 16) % TO, r = t & 15;
             const int m = m0 + (wm * TA + i) * 32 + (r >> 2) * 8 + h32 * 4 + (r & 3), n = out_col(j);
             if (m >= a.M || n >= g.n || finite_f32(g.y[(size_t)m * g.n + n])) continue;
-            g.y[(size_t)m * g.n + n] = plain_output<FMT, P, ACT>(a, g, gu, m, n);
+            g.y[(size_t)m * g.n + n] = plain_output<FMT, P, ACT, 4>(a, g, gu, m, n);
         }
     }
 }
@@ -588,8 +588,6 @@ __global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a,
                 o[c] = act_mul(a.act, o[c],
                                (P == 2 ? ldexpf(u[c], e) : u[c]) * column_scale(gu, a.sdt, nc) +
                                    (gu.bias ? gu.bias[nc] : 0.0f));
-            if constexpr (kPlain<FMT>)
-                if (!finite_f32(o[c])) o[c] = plain_output<FMT, P, ACT>(a, g, gu, m, nc);
         }
         if ((g.n & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
             *reinterpret_cast<f4_t*>(y) = o;
@@ -597,6 +595,12 @@ __global__ __launch_bounds__(256) void qgemm_exact_reduce_kernel(const XgArgs a,
 #pragma unroll
             for (int c = 0; c < 4; ++c)
                 if (n + c < g.n) y[c] = o[c];
+        }
+        if constexpr (kPlain<FMT>) {
+            if (finite_f32(o[0]) && finite_f32(o[1]) && finite_f32(o[2]) && finite_f32(o[3])) continue;
+#pragma unroll 1
+            for (int c = 0; c < min(4, g.n - n); ++c)
+                if (!finite_f32(y[c])) y[c] = plain_output<FMT, P, ACT, 1>(a, g, gu, m, n + c);  // 4: 110 registers for 72
         }
     }
 }
