@@ -568,3 +568,50 @@ def test_five_rows_of_a_wide_output_take_less_than_128(ops, fmt):
 
     few, many = time(5), time(128)
     assert few <= 0.7 * many, (few, many)  # 0.3 to 0.6; 0.8 to 0.9 in tiles of 128 rows
+
+
+# the tallest tiles (192 of them and more): several matrices, the activation in the epilogue, a padded last step
+@pytest.mark.parametrize("m,n,k,x_f16", [(1100, 2900, 320, False), (2049, 3300, 192, True), (1100, 2900, 336, True)])
+def test_gate_up_i8_tall_tiles(ops, m, n, k, x_f16):
+    x = _x(m, k, 8).cuda() * 0.3
+    x = x.half() if x_f16 else x
+    (wg, sg), (wu, su) = ((w.cuda(), s.cuda() * 0.02) for w, s in (_i8(n, k, 1), _i8(n, k, 2)))
+    h = torch.full((m, n), float("nan"), device="cuda")
+    ops.encode_gate_up_silu_i8(wg, sg, wu, su, x, h)
+    torch.cuda.synchronize()
+    g, u = (torch.matmul(x.double(), w.double().t().contiguous()) * s.double() for w, s in ((wg, sg), (wu, su)))
+    assert _rel(h, _act(g, u, "silu")) <= 2 * TOL
+
+
+@pytest.mark.parametrize("m,n,k", [(1100, 2900, 320), (1100, 2900, 352)])
+def test_q4_and_i4_tall_tiles(ops, m, n, k):
+    x = _x(m, k, 8).cuda() * 0.3
+    h = torch.full((m, n), float("nan"), device="cuda")
+    one = lambda w, x: torch.matmul(x.double(), w.cuda().t().contiguous())
+    for v in (x, x.half()):
+        if v.dtype == torch.float16 and k % 128 == 0:
+            continue
+        g, u = _q4(n, k, 5), _q4(n, k, 6)
+        h.fill_(float("nan"))
+        ops.encode_gate_up_silu_q4_affine(*g[:3], *u[:3], v, h)
+        torch.cuda.synchronize()
+        assert _rel(h, _act(one(g[3], v), one(u[3], v), "silu")) <= 2 * TOL, v.dtype
+    g, u = _i4(n, k, k, 8), _i4(n, k, k, 9)
+    h.fill_(float("nan"))
+    ops.encode_gate_up_gelu_i4_sym(*g[:2], *u[:2], k, x, h, k)
+    torch.cuda.synchronize()
+    assert _rel(h, _act(one(g[2], x), one(u[2], x), "gelu")) <= 2 * TOL
+
+
+@pytest.mark.parametrize("m,rq,rkv,k,x_f16", [(1030, 4000, 700, 320, False), (2049, 4000, 700, 128, True),
+                                              (1100, 4000, 700, 976, True)])
+def test_qkv_i8_tall_tiles(ops, m, rq, rkv, k, x_f16):
+    x = _x(m, k, k).cuda()
+    x = x.half() if x_f16 else x
+    rows = (rq, rkv, rkv)
+    w = [tuple(t.cuda() for t in _i8(r, k, 7 + i)) for i, r in enumerate(rows)]
+    y = [torch.full((m, r), float("nan"), device="cuda") for r in rows]
+    ops.encode_qkv_i8(*[t for ws in w for t in ws], x, *y)
+    torch.cuda.synchronize()
+    for i in range(3):
+        assert _rel(y[i], torch.matmul(x.double(), w[i][0].double().t().contiguous()) * w[i][1].double()) <= TOL, i
