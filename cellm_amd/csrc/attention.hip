@@ -24,9 +24,11 @@
 // V^T and P^T agree, so those eight weights are its B operand as they are.
 // Each wave keeps a running maximum, sum and O^T; the waves meet in LDS once.
 //
-// q and the softmax weights keep their 32 bits: each is two f16 parts, hi =
+// q and the softmax weights are two f16 parts each, 23 bits of their 24: hi =
 // RNE_f16(v') and lo = RNE_f16(v' - hi), of v scaled by a power of two (q: its
 // largest |q| to [2^13, 2^14); weights: by 2^13), multiplied one after the other.
+// Elements below 2^-15 of the head's largest |q| are held to 2^-38 of that, weights
+// below 2^-15 to 2^-38.
 // K and V are f16 and exact.  Scores, exponentials and sums are f32.  Sums of a
 // block that are not finite (an infinity or NaN in q, K or V: inf * lo may be NaN
 // where inf * v is not, and a masked position's 0 * inf is) are computed again by

@@ -14,21 +14,26 @@
 // the step's scales and biases with the weights through the DMA ring.  With q - 8
 // in place of q the step's two terms do not cancel (b is near -7.5 s).
 //
-// f32 activations keep their 24 bits: a first kernel scales each row by the
-// power of two that puts its largest |x| in [2^13, 2^14) and splits it into
-// hi = RNE_f16(x') and lo = RNE_f16(x' - hi); x' - hi - lo is below 2^-23 |x'|
-// (and 2^-25 absolute, 2^-38 of the row's largest).  Both parts are rows of the
-// GEMM's A operand over one weight tile, so every weight is fetched and unpacked
-// once for the two.  Products of f16 values are exact in f32.  The MFMA chain
-// rounds its f32 accumulator once per 8 or 16 products, so a chain over the whole
-// K carries more rounding error than the tree sums of the one-wave-per-row
-// kernels: accumulators run over one K step (64 k), low parts before high ones,
-// the sums of two steps are added and then join the total.  Error against 64 bits,
-// int8 at 512 rows, K = 960 / 2560 / 4096 / 8192: 8.4e-8 / 1.0e-7 / 1.1e-7 / 1.2e-7
-// (each step added to the total by itself 8.6e-8 / 1.0e-7 / 1.3e-7 / 1.3e-7, chains
-// over two steps 9.7e-8 / 1.1e-7 / 1.2e-7, over four 1.3e-7 / 1.4e-7 / 1.4e-7, the
-// one-wave-per-row kernels 9.7e-8 / 1.3e-7 / 1.7e-7 / 2.1e-7); against chains over
-// four steps this costs 4-5 % of the wide shapes' time.
+// f32 activations are two f16 parts, 23 bits of the 24: a first kernel scales each
+// row by the power of two that puts its largest |x| in [2^13, 2^14) and splits it
+// into hi = RNE_f16(x') and lo = RNE_f16(x' - hi); x' - hi - lo is at most 2^-23 |x'|,
+// and elements below 2^-15 of the row's largest are held to 2^-38 of that.  Both
+// parts are rows of the GEMM's A operand over one weight tile, so every weight is
+// fetched and unpacked once for the two.  Products of f16 values are exact in f32.
+// The MFMA chain rounds its f32 accumulator once per 8 or 16 products, so a chain
+// over the whole K carries more rounding error than the tree sums of the
+// one-wave-per-row kernels: accumulators run over one K step (64 k), low parts
+// before high ones, the sums of two steps are added and then join the total.  Error
+// against 64 bits, int8 at 512 rows, K = 960 / 2560 / 4096 / 8192: 8.4e-8 / 1.0e-7 /
+// 1.1e-7 / 1.2e-7 (each step added to the total by itself 8.6e-8 / 1.0e-7 / 1.3e-7 /
+// 1.3e-7, chains over two steps 9.7e-8 / 1.1e-7 / 1.2e-7, over four 1.3e-7 / 1.4e-7 /
+// 1.4e-7, the one-wave-per-row kernels 9.7e-8 / 1.3e-7 / 1.7e-7 / 2.1e-7); against
+// chains over four steps this costs 4-5 % of the wide shapes' time.  At few K the
+// split of x and the MFMA's own rounding show: 300 rows, K = 256 / 576 / 896 / 1024,
+// this and the row kernels, f16 weights 9.5e-8 and 6.8e-8 / 9.8e-8 and 8.6e-8 /
+// 9.7e-8 and 9.1e-8 / 9.9e-8 and 9.4e-8, int8 9.1e-8 and 8.2e-8 / 9.3e-8 and 9.0e-8 /
+// 9.1e-8 and 9.1e-8 / 9.3e-8 and 9.6e-8; i4 and q4 are below the row kernels there
+// already.  Shorter chains, added as a tree, change nothing.
 // Results that are not finite (an infinity or NaN in x or w, or an overflow) are
 // recomputed by plain f32 sums where these may differ (kPlain).
 //
@@ -36,8 +41,9 @@
 // split of x): 960 -> 960 1963 -> 20, 2560 -> 960 5098 -> 25, 4096 -> 4096
 // 8034 -> 60; 16 rows of 1152 -> 1536 35 -> 15; 2048 rows of 2048 -> 8192 164,
 // 839 TFLOP/s of MFMA work; 16 rows of 2560 -> 960, i4 109 -> 14, f16 63 -> 14; MLX
-// q4 with f32 scales, 512 rows of 4096 -> 4096, 1480 -> 67 (error 1.6e-7 -> 1.1e-7).  The small ones are bound by three dependent launches
-// and the latency of a few K steps, the wide ones by the MFMAs.
+// q4 with f32 scales, 512 rows of 4096 -> 4096, 1480 -> 67 (error 1.6e-7 -> 1.1e-7).  The
+// small ones are bound by three dependent launches and the latency of a few K steps,
+// the wide ones by the MFMAs.
 //
 // Tile: WM x WN waves of (32 TA) x (32 TB); X parts and raw weights go
 // global -> LDS by DMA through a ring of NST stages of 64 k, one barrier per
@@ -715,7 +721,7 @@ __global__ __launch_bounds__(256) void pair_x_kernel(const _Float16* __restrict_
 }
 
 // The tile forms, rows x columns: f32 x 32 x 128 (2 waves), 64 x 128 (4 waves), 128 x 256 (8 waves); f16 x
-// 32 x 128, 128 x 128, 256 x 256 (group-scaled nibbles, with their second accumulators, 128 x 256).
+// 32 x 128, 128 x 128, 256 x 256 (with second accumulators for the sums of steps, 128 x 256).
 struct XgPlan {
     int form, bm, bn, vtiles, steps_per_split, splits;
     size_t xp_off, sum_off, part_off, bytes;  // workspace: exponents, parts, sums of x', split sums

@@ -124,11 +124,11 @@ int32_t cellm_hip_weight_cache_stats(cellm_hip_ctx_t* ctx, size_t* out_entries, 
  * over k are exact and the row scale follows them, so x keeps 2^-20 of its
  * row's largest |x| (within 3e-5 normwise of the f32 reference order).  f32 x
  * at 5 rows and more (k % 16 == 0, 16-byte aligned w and x, m * k >= 7000 or
- * m * n * k >= 35e6) runs on f16 MFMA over two f16 parts of each x, 2^-23 of every
- * element, with the parts and split sums in the context's per-stream workspace;
- * without memory for it, or under graph capture on a stream whose workspace is
- * smaller (an eager call of the same shape reserves it), such calls take the
- * kernels that need none. */
+ * m * n * k >= 35e6) runs on f16 MFMA over two f16 parts of each x (2^-23 of an
+ * element, 2^-38 of its row's largest for elements below 2^-15 of that), with the
+ * parts and split sums in the context's per-stream workspace; without memory for
+ * it, or under graph capture on a stream whose workspace is smaller (an eager call
+ * of the same shape reserves it), such calls take the kernels that need none. */
 int32_t cellm_hip_qgemv_i8(cellm_hip_ctx_t* ctx, const int8_t* w, const void* scales, int32_t scale_dtype,
                            int64_t n_scales, const void* x, int32_t x_dtype, const float* bias, float* y, int64_t m,
                            int64_t n, int64_t k, void* stream);

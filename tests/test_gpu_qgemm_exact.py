@@ -1,10 +1,10 @@
 """The multi-row GEMM over f32 activations (qgemm_exact.hip) against 64-bit results.
 
-The bar: x is carried to 2^-23 of each element and every sum is f32 over chains
-of at most 16 MFMA roundings plus one add per 64 k, so the 2-norm error stays
-within a few 2^-24 (6e-8) times the square root of the number of roundings: 1e-6
-holds up to K = 8192 with a wide margin (the one-wave-per-row kernels show 1e-7
-to 2e-7 at these sizes)."""
+The bar: x is carried to 2^-23 of each element (the smallest to 2^-38 of their
+row's largest) and every sum is f32 over chains of at most 16 MFMA roundings plus
+one add per 64 k, so the 2-norm error stays within a few 2^-24 (6e-8) times the
+square root of the number of roundings: 1e-6 holds up to K = 8192 with a wide
+margin (the one-wave-per-row kernels show 1e-7 to 2e-7 at these sizes)."""
 from __future__ import annotations
 
 import numpy as np
