@@ -70,7 +70,7 @@ struct AttnArgs {
     int rows, n_heads, n_kv, group, layer, window, tiles;
     float scale, soft_cap;
     int nsplit, cap;        // splits of a row's positions at most; positions of a table
-    int tsplit, slots;      // splits of a shared tile's positions at most; slots for splits in `part`
+    int tsplit, tsplit_last, slots;  // splits of a full and of the last, ragged tile's set at most; slots in `part`
     int busy;               // rows of a shared tile whose blocks have a unit of it, at most
     float* part;            // [row][kv head][slot][group][HD + 2]
     uint32_t* counters;     // per (row, kv head): splits done, zero between calls
@@ -202,23 +202,27 @@ __device__ __forceinline__ float plain_range(const AttnArgs& a, int row, int hea
     return o;
 }
 
-// Row of the i-th block of a kv head.  The last tile first (in a prompt its rows see the most positions), and
-// the rows a shared tile needs blocks of (one per query head and split) before those whose blocks then leave at
-// once: blocks go to the XCDs in turn, and with the rows in order one XCD in four had half the others' work (a
-// 2048-token prompt of 14 / 2 heads 126 us in row order, 74 so).
+// Row of the i-th block of a kv head: of all tiles the rows whose blocks have the units of a set's first split (one
+// per query head), then those of its other splits, then those whose blocks then leave at once, and the last tile
+// first (in a prompt its rows see the most positions).  Blocks go to the XCDs in turn: with the rows in order one
+// XCD in four had half the others' work (a 2048-token prompt of 14 / 2 heads 126 us in row order, 74 so), and with
+// the rows of all splits together sets that have no splits fill half the XCDs (855 tokens of 4 / 1 heads of 128 at
+// 1100 positions, window 512, 26.7 us, 20.5 so).
 __device__ __forceinline__ int block_row(const AttnArgs& a, int i)
 {
-    const int full = a.rows / kCols, rem = a.rows - full * kCols, g = a.busy, first = min(rem, g);
-    const int active = full * g + first;
-    if (i < active) {
-        if (i < first) return full * kCols + i;
-        const int j = i - first;
-        return (full - 1 - j / g) * kCols + j % g;
+    const int full = a.rows / kCols, rem = a.rows - full * kCols;
+    int lo = 0, hi = a.group, first = min(rem, hi);
+    for (int next = a.busy;; next = kCols) {
+        const int n = full * (hi - lo) + first;
+        if (i < n) break;
+        i -= n;
+        lo = hi;
+        hi = next;
+        first = max(0, min(rem, hi) - lo);
     }
-    const int k = i - active, rest = rem - first;
-    if (k < rest) return full * kCols + first + k;
-    const int j = k - rest;
-    return (full - 1 - j / (kCols - g)) * kCols + g + j % (kCols - g);
+    if (i < first) return full * kCols + lo + i;
+    const int j = i - first, w = hi - lo;
+    return (full - 1 - j / w) * kCols + lo + j % w;
 }
 
 // Registers: four waves per SIMD at HD 64 (a 2048-token prompt of 14 / 2 heads 74 us at three, 67 at four); HD 128
@@ -262,6 +266,7 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
     const int seq_own = __builtin_amdgcn_readlane(pj, a.tiles ? sub : 0);
 
     // ---- which rows of the tile share their pages
+    const int most_splits = nr == kCols ? a.tsplit : a.tsplit_last;
     uint32_t members = 0;  // of the shared set, by row of the tile
     int leader = sub, seq_lead = 0;
     if (a.tiles) {
@@ -290,7 +295,7 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
             // every candidate where this block needs the set, of its own row where that is all
             if (t == 0) flags = 0;
             __syncthreads();
-            const bool mine = (members >> c & 1) && c != leader && (c == sub || sub < a.group || sub == leader || a.tsplit > 1);
+            const bool mine = (members >> c & 1) && c != leader && (c == sub || sub < a.group || sub == leader || most_splits > 1);
             const int nb = mine ? (pj + a.tpb - 1) / a.tpb : 0;
             const uint32_t* own = a.bt + (size_t)jr * a.max_blocks;
             bool differ = false;
@@ -330,7 +335,7 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(co
             lo_set = __builtin_amdgcn_readfirstlane(lo_set) & ~(kChunk - 1);
         }
         const int len = seq_lead - lo_set;
-        const int n = len < 4 * kMinTileSplit ? 1 : max(1, min(min(a.tsplit, nr * a.nsplit / a.group), len / kMinTileSplit));
+        const int n = len < 4 * kMinTileSplit ? 1 : max(1, min(most_splits, len / kMinTileSplit));
         tper = __builtin_amdgcn_readfirstlane(((len + n - 1) / n + kChunk - 1) & ~(kChunk - 1));
         tsplits = __builtin_amdgcn_readfirstlane((len + tper - 1) / tper);
     }
@@ -718,10 +723,31 @@ hipError_t launch_attention_mma(const float* q, const uint16_t* kcache, const ui
     const int want = std::min(max_splits, std::max(1, 512 / (rows * n_kv_heads)));
     a.nsplit = std::min(want, (cap + 511) / 512);
     a.slots = (cap + 63) / 64;  // as attention_workspace_bytes counts them
-    // sets of all tiles' heads: 512 blocks
-    const int tiles = (rows + kCols - 1) / kCols;
-    a.tsplit = max_splits == 1 ? 1 : std::min({kMaxTileSplits, a.slots, std::max(1, 512 / (tiles * n_heads))});
-    a.busy = std::min(kCols, a.group * a.tsplit);
+    // Sets of all tiles' heads: 512 blocks, where the table or the window is long enough for splits.  A full tile's
+    // set has a block for each of its units; a ragged last one has fewer blocks, which take several units each
+    // where that is the shorter walk.  Where it is not the launch ends with that tile, and the others' splits only
+    // cost: us, without / with them, 8/1 heads of 128, 300 rows at 2048 positions 44 / 48, 16/2, 200 rows at 3008
+    // 60 / 67; without a ragged tile, 8/1, 400 rows at 4096, 78 / 66; 300 there 78, 89 with the last tile unsplit, 76 so.
+    const int tiles = (rows + kCols - 1) / kCols, ragged = rows % kCols;
+    const int span = window > 0 ? std::min(window + kCols, cap) : cap;
+    a.tsplit = a.tsplit_last = 1;
+    if (max_splits > 1 && span >= 4 * kMinTileSplit) {
+        const int most = std::min({kMaxTileSplits, a.slots, std::max(1, 512 / (tiles * n_heads))});
+        const int blocks = ragged * a.nsplit;
+        // a block's walk, in positions: its units' own and what a unit takes besides (8 us of 4096 positions' 79 at
+        // heads of 128, 12 with the adding of splits)
+        const auto walk = [&](int n) { return (a.group * n + blocks - 1) / blocks * (span / n + (n > 1 ? 700 : 450)); };
+        a.tsplit = std::min(most, std::max(1, kCols * a.nsplit / a.group));
+        if (ragged >= std::max(a.group, 2)) {
+            a.tsplit_last = std::min(most, blocks / a.group);
+            for (int n = 2; n <= most && blocks < 2 * a.group; ++n)
+                if (walk(n) < walk(a.tsplit_last)) a.tsplit_last = n;
+            if (a.tsplit_last == 1) a.tsplit = 1;
+        } else if (ragged > 0 && a.nsplit == 1) {
+            a.tsplit = 1;  // its rows stay by themselves, unsplit
+        }
+    }
+    a.busy = std::min(kCols, a.group * std::max(a.tsplit, a.tsplit_last));
     a.cap = cap;
     a.part = part;
     a.counters = counters;

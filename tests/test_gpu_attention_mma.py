@@ -192,7 +192,11 @@ def _one_session(q, kc, vc, table, pos, nkv, window=0):
 @pytest.mark.parametrize("rows,nh,nkv,hd,ctx,window", [(64, 14, 2, 64, 4200, 0), (16, 32, 8, 128, 4100, 0),
                                                        (36, 8, 8, 64, 2100, 0), (130, 12, 2, 64, 2300, 2100),
                                                        (20, 40, 8, 128, 3100, 0), (33, 8, 1, 128, 6200, 0),
-                                                       (2, 14, 2, 64, 8200, 0), (15, 8, 2, 128, 8192, 5000)])
+                                                       (2, 14, 2, 64, 8200, 0), (15, 8, 2, 128, 8192, 5000),
+                                                       # ragged last tiles: blocks with two units, none split, by themselves
+                                                       (76, 8, 1, 128, 2700, 0), (300, 8, 1, 64, 4100, 0),
+                                                       (277, 9, 3, 128, 2048, 0), (133, 5, 1, 64, 1100, 0),
+                                                       (269, 9, 3, 64, 2300, 2100)])
 def test_rows_of_one_session_in_splits(ops, rows, nh, nkv, hd, ctx, window):
     tpb = 16
     per = -(-ctx // tpb)
