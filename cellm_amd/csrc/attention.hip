@@ -228,10 +228,11 @@ __device__ __forceinline__ int block_row(const AttnArgs& a, int i)
 // Registers: four waves per SIMD at HD 64 (a 2048-token prompt of 14 / 2 heads 74 us at three, 67 at four); HD 128
 // needs the registers of three.  Measured, us, vector kernels -> this: prompts of 512 and 2048 tokens, 14 / 2 heads
 // of 64, 90 -> 13 and 589 -> 61; 1024 tokens at 2048 positions, 32 / 8 heads of 128, 1586 -> 182; 8 sessions at
-// 4096..8192 positions, 32 / 8 heads of 128, 86 -> 56 (3.6 TB/s), 16 sessions at 8192..16384, 8 / 8 heads of 128,
+// 4096..8192 positions, 32 / 8 heads of 128, 82 -> 54 (3.7 TB/s), 16 sessions at 8192..16384, 8 / 8 heads of 128,
 // 190 -> 176 (4.6 TB/s).  Prompts are bound by the latency of a chunk (page, K, scores, maximum, weights, V in LDS)
-// at about two waves per SIMD, long contexts by memory.  The error against 64 bits is no larger than the vector
-// kernels' (3.7e-7 / 3.8e-7, 1.8e-7 / 1.9e-7 on these).
+// at about two waves per SIMD, long contexts by memory.  The error against 64 bits is 0.92 of the vector
+// kernels' over 70 calls of both directions and none larger by more than 5 % (8 sessions at 4096..8192, by the seed,
+// 3.7e-7 / 3.8e-7 and 4.5e-7 / 4.3e-7).
 template <int HD, bool CAP>
 __global__ __launch_bounds__(kThreads, HD == 64 ? 4 : 3) void attn_mma_kernel(const AttnArgs a)
 {
